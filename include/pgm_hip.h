@@ -191,8 +191,8 @@ int pgm_set_graphs(pgm_ctx *ctx, int on);
 
 /* Layout of the CG row field (the data of PGMForceField._row_field, forcefield.py:1395-1402): 0 atom
  * rows (partner index, G1, G2 per pair in sliced ELL), 1 molecule blocks (contexts of consecutive
- * 3-atom molecules: per molecule pair the 9 atom pairs' G1, G2, `lanes` = 4, 8 or 16 lanes per
- * molecule; the default where it applies).  Same sums in another order; rows are rebuilt at the
+ * 3-atom molecules: per molecule pair the 9 atom pairs' G1, G2, `lanes` = 4, 8 or 16: at least so many
+ * lanes per molecule (the launch takes 16 to 64 by the size of the system); the default where it applies).  Same sums in another order; rows are rebuilt at the
  * next evaluation.  pgm_row_layout reports the layout and its lanes. */
 int pgm_set_row_layout(pgm_ctx *ctx, int layout, int lanes);
 int pgm_row_layout(const pgm_ctx *ctx, int *layout, int *lanes);

@@ -102,6 +102,8 @@ struct DevBuf {
     template <typename T> T *as() const { return (T *)p; }
 };
 
+constexpr int ROW_FIELD_WAVES = 2048;  // two waves per SIMD (row_field_lanes)
+
 struct pgm_ctx {
     int n = 0;
     // beads: nbead copies of one system of nper atoms stacked along the atom axis (n = nbead nper);
@@ -178,8 +180,9 @@ struct pgm_ctx {
     bool fused_ok = false, pme_fused = false;
     // where a CG field evaluation forks the row field onto the side stream: 0 before the spread,
     // 1 after the spread, 2 after the forward planes, 3 before the spread with the forward planes
-    // waiting for it (2 and 3: fused transform only); chosen by pgm_autotune
-    int fork_stage = 0;
+    // waiting for it (2 and 3: fused transform only), 4 no side stream; set from the size at creation
+    // (default_fork) and by pgm_autotune
+    int fork_stage = 4;
     PFFTGeom pfg{};
     DevBuf pfft_tw;
     // tiled spread (atoms sorted by grid tile)
@@ -259,6 +262,15 @@ struct pgm_ctx {
 static double *aux_slots(const pgm_ctx *c) { return c->energy.as<double>() + 4 * c->nbead; }
 // The largest displacement since the row build, written by the MD step's reduction into pinned host memory.
 static double *h_disp(const pgm_ctx *c) { return reinterpret_cast<double *>(c->h_mirror + 4 * (size_t)c->nbead); }
+
+// Fork point of a new context: a fork and its join cost a field evaluation 10-20 us of cross-stream
+// latency, which pays only where the row field is long enough to hide the PME chain behind it.  Whole
+// field evaluations, FP32, fork after the spread / no side stream [us]: 64 waters 57.5 / 46.7, 1,331:
+// 92.7 / 84.4, 4,096: 92.9 / 91.5, 12,167: 139 / 135, 32,768: 176 / 207.  With the library transform the
+// row field starts first: its many small kernels leave room beside it (32 beads of 1,024 waters: 4.52 ms
+// per evaluation of all beads against 4.69 with the fork after the spread).
+constexpr int FORK_ATOMS = 49152;
+static int default_fork(const pgm_ctx *c) { return c->n < FORK_ATOMS ? 4 : (c->fused_ok && c->tiled ? 1 : 0); }
 
 static void drop_graphs(pgm_ctx *c) {
     for (hipGraphExec_t &g : c->it_graphs)
@@ -673,12 +685,12 @@ static int alloc_rows(pgm_ctx *c, int cap) {
     return PGM_OK;
 }
 
-// Molecule-block buffers for candidate capacity mcap_full (records rounded up to rlm lanes).
+// Molecule-block buffers for candidate capacity mcap_full (records rounded up to whole chunks).
 static int alloc_mol(pgm_ctx *c, int mcap_full) {
     drop_graphs(c);
     const int nmol = c->n / 3;
     c->mcap_full = mcap_full;
-    c->mcap = (mcap_full + c->rlm - 1) / c->rlm * c->rlm;
+    c->mcap = (mcap_full + MCH - 1) / MCH * MCH;
     PGM_TRY(c->mrows.ensure(sizeof(int) * (size_t)nmol * mcap_full));
     PGM_TRY(c->mcount_full.ensure(sizeof(int) * nmol));
     PGM_TRY(c->mcount.ensure(sizeof(int) * nmol));
@@ -816,18 +828,18 @@ static int prepare(pgm_ctx *c, const double *pos, bool defer_records = false) {
         const bool rows_too = c->mixed && c->rc_v > c->rc_e;
         if (rows_too)
             k_mol_tensors<float, true><<<nblk(nmol, 4), 256, 0, rs>>>(nmol, c->mrows.as<int>(), c->mcount_full.as<int>(), c->mcap_full,
-                                                               c->mcap, c->rlm, c->xr.as<double4>(), c->box, rc2, rce2,
+                                                               c->mcap, c->xr.as<double4>(), c->box, rc2, rce2,
                                                                (float)c->s.ewald_beta, c->mj.as<int>(), c->mg.as<float>(),
                                                                c->mcount.as<int>(), c->rows.as<int>(), c->cap,
                                                                c->count.as<int>(), c->count_near.as<int>(), beta2);
         else if (c->mixed)
             k_mol_tensors<float, false><<<nblk(nmol, 4), 256, 0, rs>>>(
-                nmol, c->mrows.as<int>(), c->mcount_full.as<int>(), c->mcap_full, c->mcap, c->rlm, c->xr.as<double4>(), c->box,
+                nmol, c->mrows.as<int>(), c->mcount_full.as<int>(), c->mcap_full, c->mcap, c->xr.as<double4>(), c->box,
                 rc2, rce2, (float)c->s.ewald_beta, c->mj.as<int>(), c->mg.as<float>(), c->mcount.as<int>(), nullptr, 0, nullptr,
                 nullptr, beta2);
         else
             k_mol_tensors<double, false><<<nblk(nmol, 4), 256, 0, rs>>>(
-                nmol, c->mrows.as<int>(), c->mcount_full.as<int>(), c->mcap_full, c->mcap, c->rlm, c->xr.as<double4>(), c->box,
+                nmol, c->mrows.as<int>(), c->mcount_full.as<int>(), c->mcap_full, c->mcap, c->xr.as<double4>(), c->box,
                 rc2, rce2, c->s.ewald_beta, c->mj.as<int>(), c->mg.as<double>(), c->mcount.as<int>(), nullptr, 0, nullptr, nullptr,
                 beta2);
         c->atom_rows_fresh = rows_too;
@@ -1063,6 +1075,17 @@ static int gather_combine(pgm_ctx *c, const real4<real> *dq, int mode, const rea
     return PGM_OK;
 }
 
+// Lanes that share a molecule's records in the row field: 16 (a chunk of records is read in whole
+// 256-byte segments), more while the launch has fewer than ROW_FIELD_WAVES waves and would leave SIMDs
+// idle behind a few long chains of dependent gathers.  Measured alone (FP32, us per launch, with 4 / 16
+// / 32 / 64 lanes): 512 waters 31.6 / 10.3 / 7.4 / 5.9, 4,096: 39.4 / 14.8 / 12.2 / 13.6, 12,167: 43.7 /
+// 27.2 / 28.0 / 32.3, 32,768: 111.6 / 84.9 / 86.9 / 100.6.
+static int row_field_lanes(const pgm_ctx *c) {
+    int lanes = std::max(c->rlm, 16);
+    while (lanes < 64 && (long long)(c->n / 3) * lanes < 64LL * ROW_FIELD_WAVES) lanes *= 2;
+    return lanes;
+}
+
 // The CG row field of dq into vrow on stream st, in the context's layout.
 template <typename real, bool WITHQ>
 static int row_field_launch(pgm_ctx *c, const real4<real> *dq, const int *conv, int iter, hipStream_t st, TimedPair tp = {},
@@ -1074,11 +1097,14 @@ static int row_field_launch(pgm_ctx *c, const real4<real> *dq, const int *conv, 
         const real *mg = c->mg.as<real>();
         const double4 *xr = c->xr.as<double4>();
         R4 *out = c->vrow.as<R4>();
-        const dim3 b(256);
-        switch (c->rlm) {
-            case 4: launch_timed(tp, k_row_field_mol<real, WITHQ, 4>, dim3(nblk((long long)nmol * 4, 256)), b, 0, st, nmol, nb, mj, mg, mc, xr, dq, c->box, out, conv, iter, ext); break;
-            case 8: launch_timed(tp, k_row_field_mol<real, WITHQ, 8>, dim3(nblk((long long)nmol * 8, 256)), b, 0, st, nmol, nb, mj, mg, mc, xr, dq, c->box, out, conv, iter, ext); break;
-            default: launch_timed(tp, k_row_field_mol<real, WITHQ, 16>, dim3(nblk((long long)nmol * 16, 256)), b, 0, st, nmol, nb, mj, mg, mc, xr, dq, c->box, out, conv, iter, ext); break;
+        const auto go = [&](auto k, int lanes) {
+            launch_timed(tp, k, dim3(nblk((long long)nmol * lanes, 256)), dim3(256), 0, st, nmol, nb, c->mcap, mj, mg, mc, xr, dq, c->box, out,
+                         conv, iter, ext);
+        };
+        switch (row_field_lanes(c)) {
+            case 16: go(k_row_field_mol<real, WITHQ, 16>, 16); break;
+            case 32: go(k_row_field_mol<real, WITHQ, 32>, 32); break;
+            default: go(k_row_field_mol<real, WITHQ, 64>, 64); break;
         }
     } else {
         launch_timed(tp, k_row_field<real, WITHQ>, dim3(nblk((long long)c->n * RL, 256)), dim3(256), 0, st, c->n, c->nper,
@@ -1748,7 +1774,7 @@ static int energy_forces_impl(pgm_ctx *c, const double *mu, pgm_energy *energy, 
         }
         if (mol_forces)
             k_pair_forces_mol<real, MOL_FORCE_LANES><<<gpair, 256, 0, ps>>>(
-                nper, n / 3, c->rlm, c->mj.as<int>(), c->mg.as<real>(), c->mcount.as<int>(), c->xr.as<double4>(), dq, c->box,
+                nper, c->mcap, c->mj.as<int>(), c->mg.as<real>(), c->mcount.as<int>(), c->xr.as<double4>(), dq, c->box,
                 (real)c->s.ewald_beta, c->rc_e * c->rc_e, c->rc_v * c->rc_v, c->rh.as<double>(), c->se.as<double>(),
                 c->g_el.as<double>(), c->g_lj.as<double>(), c->rowf.as<double>(), c->pair_part.as<double>(), ext);
         else
@@ -2097,6 +2123,7 @@ extern "C" int pgm_ctx_create(pgm_ctx **out, const pgm_topology *top, const pgm_
     if ((r = alloc_rows(c, std::min(cap0, c->nper))) < 0) return fail(r);
     if ((r = make_plans(c)) < 0) return fail(r);
     if ((r = setup_fused(c)) < 0) return fail(r);
+    c->fork_stage = default_fork(c);
     *out = c;
     return PGM_OK;
 }

@@ -552,14 +552,66 @@ __global__ __launch_bounds__(256) void k_pair_forces(int nper, const int *__rest
 // For systems of 3-site molecules (atoms 3I, 3I+1, 3I+2) the CG row field runs on molecule pairs:
 // record (I, J) holds the 9 atom pairs (p of I, k of J) as G1[3p+k], G2[3p+k] (zero beyond the
 // cutoff and for p == k when J == I), so one lane fetches J's three positions and dipoles once for
-// nine pair terms instead of one gather per pair.  Records of molecule I sit at
-// mell(e, I) = (e / RLM) nmol RLM + I RLM + e % RLM for its RLM lanes.  The record's word is
+// nine pair terms instead of one gather per pair.  The record's word (mj[I mcap + e]) is
 // J | code << 26: code = the lattice shifts (n_a + 1 in two bits per axis) shared by every pair
 // within the cutoff, or MOL_OWN_IMAGES when they differ (the pairs then take min_image each).
+//
+// The 18 reals of the records are stored in chunks of MCH = 16 records of one molecule, in planes of
+// 16 bytes per record (FP32: four planes of four reals and one of two; FP64: nine planes of two),
+// so the lanes that take consecutive records read (and the record pass writes) whole 256-byte
+// segments.  One 72-byte record per lane in a row made every load instruction of a wave touch 36
+// cache lines instead of 8.  The layout does not depend on how many lanes share a molecule.
 constexpr int MOL_OWN_IMAGES = 63;
 constexpr int MOL_REC = 18;  // reals per record: G1 of the 9 pairs, then G2
-PGM_DEV size_t mell(int e, int I, int nmol, int rlm) {
-    return (size_t)(e / rlm) * ((size_t)nmol * rlm) + (size_t)I * rlm + (e % rlm);
+constexpr int MCH = 16;      // records per chunk
+// First real of the chunk of record e of molecule I (mcap a multiple of MCH).
+PGM_DEV size_t mchunk(int e, int I, int mcap) { return ((size_t)I * (mcap / MCH) + e / MCH) * (size_t)(MCH * MOL_REC); }
+// Offset of real t (0..17) of record e within its chunk.
+template <typename real> PGM_DEV int mslot(int e, int t) {
+    constexpr int V = 16 / (int)sizeof(real);  // reals per plane entry
+    constexpr int FULL = MOL_REC / V * V;      // reals in whole planes
+    const int s = e % MCH;
+    return t < FULL ? (t / V) * (V * MCH) + s * V + t % V : FULL * MCH + s * (MOL_REC - FULL) + (t - FULL);
+}
+// The 18 reals of record e of the chunk at g, to or from registers.
+PGM_DEV void mload(const float *__restrict__ g, int e, float (&G)[MOL_REC]) {
+    const int s = e % MCH;
+    const float4 *q = reinterpret_cast<const float4 *>(g) + s;
+    const float4 a = q[0], b = q[MCH], c = q[2 * MCH], d = q[3 * MCH];
+    const float2 t = reinterpret_cast<const float2 *>(g + 16 * MCH)[s];
+    const float v[MOL_REC] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, c.x, c.y, c.z, c.w, d.x, d.y, d.z, d.w, t.x, t.y};
+#pragma unroll
+    for (int k = 0; k < MOL_REC; ++k) G[k] = v[k];
+}
+PGM_DEV void mload(const double *__restrict__ g, int e, double (&G)[MOL_REC]) {
+    const double2 *q = reinterpret_cast<const double2 *>(g) + e % MCH;
+#pragma unroll
+    for (int k = 0; k < MOL_REC / 2; ++k) {
+        const double2 v = q[k * MCH];
+        G[2 * k] = v.x;
+        G[2 * k + 1] = v.y;
+    }
+}
+PGM_DEV void mstore(float *__restrict__ g, int e, const float (&A)[9], const float (&B)[9]) {
+    const int s = e % MCH;
+    float4 *q = reinterpret_cast<float4 *>(g) + s;
+    q[0] = make_float4(A[0], A[1], A[2], A[3]);
+    q[MCH] = make_float4(A[4], A[5], A[6], A[7]);
+    q[2 * MCH] = make_float4(A[8], B[0], B[1], B[2]);
+    q[3 * MCH] = make_float4(B[3], B[4], B[5], B[6]);
+    reinterpret_cast<float2 *>(g + 16 * MCH)[s] = make_float2(B[7], B[8]);
+}
+PGM_DEV void mstore(double *__restrict__ g, int e, const double (&A)[9], const double (&B)[9]) {
+    double2 *q = reinterpret_cast<double2 *>(g) + e % MCH;
+    q[0] = make_double2(A[0], A[1]);
+    q[MCH] = make_double2(A[2], A[3]);
+    q[2 * MCH] = make_double2(A[4], A[5]);
+    q[3 * MCH] = make_double2(A[6], A[7]);
+    q[4 * MCH] = make_double2(A[8], B[0]);
+    q[5 * MCH] = make_double2(B[1], B[2]);
+    q[6 * MCH] = make_double2(B[3], B[4]);
+    q[7 * MCH] = make_double2(B[5], B[6]);
+    q[8 * MCH] = make_double2(B[7], B[8]);
 }
 
 // Candidate partner molecules of molecule I: the molecules of the atoms in the full (cutoff + skin)
@@ -656,7 +708,7 @@ __global__ __launch_bounds__(256) void k_mol_rows(int nmol, int nmol_bead, const
 // the FP64 variant at four.
 template <typename real, bool ROWS>
 __global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_mol_tensors(int nmol, const int *__restrict__ mrows, const int *__restrict__ mcount_full,
-                                                     int mcap_full, int mcap, int rlm, const double4 *__restrict__ xr, Box box,
+                                                     int mcap_full, int mcap, const double4 *__restrict__ xr, Box box,
                                                      double rc2, double rce2, real beta, int *__restrict__ mj, real *__restrict__ mg,
                                                      int *__restrict__ mcount, int *__restrict__ rows, int acap,
                                                      int *__restrict__ acount, int *__restrict__ acount_near, double beta2) {
@@ -766,19 +818,14 @@ __global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_mol_tensors(
         const unsigned long long m = __ballot(keep);
         const int slot_e = kept + __popcll(m & below);
         if (keep && slot_e < mcap) {
-            const size_t q = mell(slot_e, I, nmol, rlm);
-            mj[q] = (int)((unsigned)J | ((unsigned)code << 26));
-            real *g = mg + q * MOL_REC;
+            mj[(size_t)I * mcap + slot_e] = (int)((unsigned)J | ((unsigned)code << 26));
+            real *g = mg + mchunk(slot_e, I, mcap);
             if (own) {  // the diagonal (p == k) only; the six pairs follow
-                g[0] = g[4] = g[8] = real(0);
-                g[9] = g[13] = g[17] = real(0);
+#pragma unroll
+                for (int p = 0; p < 3; ++p) g[mslot<real>(slot_e, 4 * p)] = g[mslot<real>(slot_e, 9 + 4 * p)] = real(0);
                 self_slot = slot_e;
             } else {
-#pragma unroll
-                for (int t = 0; t < 9; ++t) {
-                    g[t] = G1[t];
-                    g[9 + t] = G2[t];
-                }
+                mstore(g, slot_e, G1, G2);
             }
         }
         kept += __popcll(m);
@@ -798,9 +845,9 @@ __global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_mol_tensors(
                 const real aij = rsqrt_(real(2) * (real)(ap.w + ak.w));
                 pair_G<real, 3>(aij, beta, x * x + y * y + z * z, G);
             }
-            real *g = mg + mell(sslot, I, nmol, rlm) * MOL_REC;
-            g[3 * p + k] = G[1];
-            g[9 + 3 * p + k] = G[2];
+            real *g = mg + mchunk(sslot, I, mcap);
+            g[mslot<real>(sslot, 3 * p + k)] = G[1];
+            g[mslot<real>(sslot, 9 + 3 * p + k)] = G[2];
         }
     }
     if (lane == 0) mcount[I] = kept < mcap ? kept : mcap;
@@ -813,9 +860,9 @@ __global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_mol_tensors(
 }
 
 // Row field of the molecule blocks: out_i for the three atoms of I (the same sum as k_row_field over
-// the pairs within rc, in molecule-pair order).  RLM lanes per molecule.
+// the pairs within rc, in molecule-pair order).  RLM lanes per molecule take its records in turn.
 template <typename real, bool WITHQ, int RLM>
-__global__ __launch_bounds__(256) void k_row_field_mol(int nmol, int nmol_bead, const int *__restrict__ mj,
+__global__ __launch_bounds__(256) void k_row_field_mol(int nmol, int nmol_bead, int mcap, const int *__restrict__ mj,
                                                        const real *__restrict__ mg, const int *__restrict__ mcount,
                                                        const double4 *__restrict__ xr, const real4<real> *__restrict__ dq,
                                                        Box box, real4<real> *__restrict__ out, const int *__restrict__ conv_it,
@@ -828,28 +875,12 @@ __global__ __launch_bounds__(256) void k_row_field_mol(int nmol, int nmol_bead, 
 #pragma unroll
     for (int t = 0; t < 9; ++t) acc[t] = real(0);
     const int c = mcount[I];
+    const int *words = mj + (size_t)I * mcap;
     for (int e = lane; e < c; e += RLM) {
-        const size_t q = mell(e, I, nmol, RLM);
-        const unsigned word = (unsigned)mj[q];
+        const unsigned word = (unsigned)words[e];
         const int J = (int)(word & ((1u << 26) - 1u)), code = (int)(word >> 26);
         real G[MOL_REC];
-        if (sizeof(real) == 4) {
-            const float2 *g2 = reinterpret_cast<const float2 *>(mg + q * MOL_REC);
-#pragma unroll
-            for (int t = 0; t < MOL_REC / 2; ++t) {
-                const float2 v = g2[t];
-                G[2 * t] = (real)v.x;
-                G[2 * t + 1] = (real)v.y;
-            }
-        } else {
-            const double2 *g2 = reinterpret_cast<const double2 *>(mg + q * MOL_REC);
-#pragma unroll
-            for (int t = 0; t < MOL_REC / 2; ++t) {
-                const double2 v = g2[t];
-                G[2 * t] = (real)v.x;
-                G[2 * t + 1] = (real)v.y;
-            }
-        }
+        mload(mg + mchunk(e, I, mcap), e, G);
         double4 b[3];
         real4<real> d[3];
 #pragma unroll
@@ -857,16 +888,23 @@ __global__ __launch_bounds__(256) void k_row_field_mol(int nmol, int nmol_bead, 
             b[k] = xr[3 * J + k];
             d[k] = dq[3 * J + k];
         }
-        const int n[3] = {(code & 3) - 1, ((code >> 2) & 3) - 1, ((code >> 4) & 3) - 1};
+        const bool own = code == MOL_OWN_IMAGES;
+        if (!own) {  // the lattice shift shared by the record's pairs moves J once, not every difference
+            const double n0 = (double)((code & 3) - 1), n1 = (double)(((code >> 2) & 3) - 1), n2 = (double)(((code >> 4) & 3) - 1);
+            const double sx = n0 * box.h[0] + n1 * box.h[3] + n2 * box.h[6], sy = n1 * box.h[4] + n2 * box.h[7], sz = n2 * box.h[8];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                b[k].x += sx;
+                b[k].y += sy;
+                b[k].z += sz;
+            }
+        }
 #pragma unroll
         for (int p = 0; p < 3; ++p)
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
                 double dx = a[p].x - b[k].x, dy = a[p].y - b[k].y, dz = a[p].z - b[k].z;
-                if (code == MOL_OWN_IMAGES)
-                    min_image(dx, dy, dz, box);
-                else
-                    apply_shift(dx, dy, dz, box, n);
+                if (own) min_image(dx, dy, dz, box);
                 const real x = (real)dx, y = (real)dy, z = (real)dz;
                 const real g1 = G[3 * p + k], g2 = G[9 + 3 * p + k];
                 const real dkx = d[k].x * x + d[k].y * y + d[k].z * z;
@@ -935,7 +973,7 @@ constexpr int MOL_NEAR_QUEUE = 8;  // queued series pairs per lane (more are eva
 // Launched with 256 threads per block (the LDS queue has 256 columns).  FP32: at most 128 VGPRs
 // (four waves per SIMD); FP64 unbounded.
 template <typename real, int FL>
-__global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_pair_forces_mol(int nper, int nmol, int rlm, const int *__restrict__ mj,
+__global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_pair_forces_mol(int nper, int mcap, const int *__restrict__ mj,
                                                          const real *__restrict__ mg, const int *__restrict__ mcount,
                                                          const double4 *__restrict__ xr, const real4<real> *__restrict__ dq,
                                                          Box box, real beta, double rce2, double rcv2,
@@ -962,7 +1000,7 @@ __global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_pair_forces_
         int qlen = 0;
         // the pair (p, k) of record e on the series branch
         auto near_pair = [&](int e, int k, real &pe, real &pg0, real &pg1, real &pg2, real &pf0, real &pf1, real &pf2) {
-            const unsigned word = (unsigned)mj[mell(e, I, nmol, rlm)];
+            const unsigned word = (unsigned)mj[(size_t)I * mcap + e];
             const int J = (int)(word & ((1u << 26) - 1u)), code = (int)(word >> 26);
             const int n[3] = {(code & 3) - 1, ((code >> 2) & 3) - 1, ((code >> 4) & 3) - 1};
             const double4 b = xr[3 * J + k];
@@ -979,12 +1017,16 @@ __global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_pair_forces_
             MOL_FORCE_TERMS(G[0], G[1], G[2], G[3])
         };
         for (int e = lane; e < c; e += FL) {
-            const size_t q = mell(e, I, nmol, rlm);
-            const unsigned word = (unsigned)mj[q];
+            const unsigned word = (unsigned)mj[(size_t)I * mcap + e];
             const int J = (int)(word & ((1u << 26) - 1u)), code = (int)(word >> 26);
             const bool own = J == I;
-            const real *gr = mg + q * MOL_REC + 3 * p;
-            const real G1[3] = {gr[0], gr[1], gr[2]}, G2[3] = {gr[9], gr[10], gr[11]};
+            const real *gr = mg + mchunk(e, I, mcap);
+            real G1[3], G2[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                G1[k] = gr[mslot<real>(e, 3 * p + k)];
+                G2[k] = gr[mslot<real>(e, 9 + 3 * p + k)];
+            }
             const int n[3] = {(code & 3) - 1, ((code >> 2) & 3) - 1, ((code >> 4) & 3) - 1};
             real pg0 = 0, pg1 = 0, pg2 = 0, pf0 = 0, pf1 = 0, pf2 = 0, pe = 0;
             unsigned nearm = 0u;
