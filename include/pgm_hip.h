@@ -217,7 +217,7 @@ int pgm_set_row_fork(pgm_ctx *ctx, int stage);
 
 /* Autotuner (no counterpart in the reference): times, on this context's system at positions pos
  * (device), every applicable row-field layout (molecule blocks with 4, 8, 16 lanes; atom rows),
- * every valid PME spread-tile width (8 down to order - 1 points per axis; gather tiles twice that),
+ * every valid PME tile width (8 down to order - 1 points per axis),
  * both reciprocal transforms and the point where a CG field evaluation starts the row field on its
  * side stream (before the spread, after it, after the forward planes of the fused transform) or
  * runs it on the context's stream (jointly with the row layouts within 10 % of the fastest row

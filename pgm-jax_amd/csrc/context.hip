@@ -186,12 +186,12 @@ struct pgm_ctx {
     PFFTGeom pfg{};
     DevBuf pfft_tw;
     // tiled spread (atoms sorted by grid tile)
-    // spread tiles of T8 points per axis (tiles8, one fine key each) inside gather tiles of 2 T8
-    // (tiles); tstart/tend by fine key, tstart16/tend16 by gather tile
+    // tiles of T points per axis (one fine key each) in cubes of 2 x 2 x 2; trange (start, end) by fine key
     bool tiled = false;
     int tile_cap = 8;  // largest spread-tile width tried per axis (pgm_autotune lowers it)
-    PMETiles tiles{}, tiles8{};
-    DevBuf pkey, pidx, pskey, psidx, tstart, tend, tstart16, tend16, spl, loc, loc16, blocks, pme_sort_tmp, merge_tab;
+    PMETiles tiles{};
+    DevBuf corg;  // packed cube coordinates (octant_tile)
+    DevBuf pkey, pidx, pskey, psidx, trange, sten, blocks, pme_sort_tmp, merge_tab;
     // vectors (real4 N) and FP64 (N, 3) work arrays
     DevBuf vx, vr, vz, vp, vAp, vb, vx0, vrow, vdq, vtmp;
     DevBuf pperm, dd, g_el, g_lj, rowf, rec_dr, gp;
@@ -448,39 +448,13 @@ static int set_box(pgm_ctx *c, const double *H) {
 
 // Tile widths of the spread: per axis the smallest T in 8..16 (else 7..P-1) with at least two tiles
 // and a last tile at least P-1 wide; no such T: the atomic spread is used.
-static size_t spread_lds_bytes(const pgm_ctx *c) {
-    const int P = c->s.order;
-    return (size_t)SPREAD_CHUNK * (6 * P + 4) * c->rsize + SPREAD_CHUNK * sizeof(int) + c->rsize * (size_t)c->tiles8.bsize;
-}
-
-// Raise the dynamic-LDS limit of the tiled spread / gather instantiations of this context.
-template <typename real, int P> static int allow_lds_p(size_t spread, size_t gather) {
-    HIP_TRY(hipFuncSetAttribute((const void *)k_spread_tiles<real, P, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)spread));
-    HIP_TRY(hipFuncSetAttribute((const void *)k_spread_tiles<real, P, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)spread));
-    HIP_TRY(hipFuncSetAttribute((const void *)k_gather_tiles<real, P>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gather));
-    return PGM_OK;
-}
-static int allow_lds(pgm_ctx *c, size_t spread, size_t gather) {
-    if (spread > 160 * 1024 || gather > 160 * 1024) {
-        g_err = "PME tile block exceeds the LDS";
-        return PGM_ERR_ARG;
-    }
-    int r = PGM_OK;
-    if (c->mixed) {
-        ORDER_SWITCH(c->s.order, r = (allow_lds_p<float, PO>(spread, gather)));
-    } else {
-        ORDER_SWITCH(c->s.order, r = (allow_lds_p<double, PO>(spread, gather)));
-    }
-    return r;
-}
-
-// Spread tiles: per axis the largest T8 in tile_cap (8 unless tuned)..P-1 with at least three tiles
-// and a last tile at least P-1 wide; gather tiles of T16 = 2 T8 (the union of two spread tiles per axis).  No such T8: the
-// atomic spread and the per-atom gather are used.
+// Tiles: per axis the largest T in tile_cap (8 unless tuned)..P-1 with at least three tiles and a last
+// tile at least P-1 wide, numbered in cubes of 2 x 2 x 2 tiles.  No such T: the atomic spread and the
+// per-atom gather are used.
 static int setup_tiles(pgm_ctx *c) {
     drop_graphs(c);
     const int P = c->s.order;
-    PMETiles t8{}, t16{};
+    PMETiles t{};
     bool ok = true;
     for (int a = 0; a < 3; ++a) {
         const int K = c->s.grid[a];
@@ -494,91 +468,76 @@ static int setup_tiles(pgm_ctx *c) {
             ok = false;
             break;
         }
-        t8.T[a] = best;
-        t8.nt[a] = (K + best - 1) / best;
-        t8.B[a] = best + P - 1;
-        t16.T[a] = 2 * best;
-        t16.nt[a] = (t8.nt[a] + 1) / 2;
-        t16.B[a] = 2 * best + P - 1;
+        t.T[a] = best;
+        t.nt[a] = (K + best - 1) / best;
+        t.nc[a] = (t.nt[a] + 1) / 2;
+        t.B[a] = best + P - 1;
     }
     c->tiled = ok;
     if (!ok) return PGM_OK;
-    t16.ntiles = t16.nt[0] * t16.nt[1] * t16.nt[2];
-    t16.bsize = t16.B[0] * t16.B[1] * t16.B[2];
-    t8.ntiles = 8 * t16.ntiles;  // by fine key (octants past the grid stay empty)
-    t8.bsize = t8.B[0] * t8.B[1] * t8.B[2];
-    c->tiles = t16;
-    c->tiles8 = t8;
+    t.ncubes = t.nc[0] * t.nc[1] * t.nc[2];
+    t.ntiles = 8 * t.ncubes;
+    t.bsize = t.B[0] * t.B[1] * PME_ZROW;
+    c->tiles = t;
     const int n = c->n;
     const size_t B = (size_t)c->nbead;
     PGM_TRY(c->pkey.ensure(sizeof(int) * n));
     PGM_TRY(c->pidx.ensure(sizeof(int) * n));
     PGM_TRY(c->pskey.ensure(sizeof(int) * n));
     PGM_TRY(c->psidx.ensure(sizeof(int) * n));
-    PGM_TRY(c->loc.ensure(sizeof(int) * n));
-    PGM_TRY(c->loc16.ensure(sizeof(int) * n));
-    PGM_TRY(c->tstart.ensure(sizeof(int) * B * t8.ntiles));
-    PGM_TRY(c->tend.ensure(sizeof(int) * B * t8.ntiles));
-    PGM_TRY(c->tstart16.ensure(sizeof(int) * B * t16.ntiles));
-    PGM_TRY(c->tend16.ensure(sizeof(int) * B * t16.ntiles));
-    PGM_TRY(c->spl.ensure(c->rsize * 6 * P * (size_t)n));
-    PGM_TRY(c->blocks.ensure(c->rsize * B * t8.ntiles * t8.bsize));
+    PGM_TRY(c->trange.ensure(sizeof(int2) * B * t.ntiles));
+    PGM_TRY(c->sten.ensure(c->rsize * 4 * (size_t)n));
+    PGM_TRY(c->blocks.ensure(c->rsize * B * t.ntiles * t.bsize));
     {  // per-axis offsets of the block merge (k_merge_table, k_pme_fwd_plane)
-        std::vector<int> tab;
+        std::vector<int> tab, org;
         for (int a = 0; a < 3; ++a) {
-            const int K = c->s.grid[a], T = t8.T[a], nt = t8.nt[a];
-            const int stride = a == 0 ? t8.B[1] * t8.B[2] : (a == 1 ? t8.B[2] : 1);
-            auto A = [&](int u) {
-                const int hi = u >> 1, lo = u & 1;
-                if (a == 0) return hi * t16.nt[1] * t16.nt[2] * 8 + lo * 4;
-                if (a == 1) return hi * t16.nt[2] * 8 + lo * 2;
-                return hi * 8 + lo;
-            };
+            const int K = c->s.grid[a], T = t.T[a], nt = t.nt[a];
+            const int stride = a == 0 ? t.B[1] * PME_ZROW : (a == 1 ? PME_ZROW : 1);
+            const int cube = 8 * (a == 0 ? t.nc[1] * t.nc[2] : (a == 1 ? t.nc[2] : 1)), oct = 4 >> a;
+            auto A = [&](int u) { return ((u >> 1) * cube + (u & 1) * oct) * t.bsize; };
             for (int g = 0; g < K; ++g) {
                 const int u = std::min(g / T, nt - 1), l = g - u * T;
-                tab.push_back(A(u) * t8.bsize + l * stride);
+                tab.push_back(A(u) + l * stride);
                 if (l <= P - 2) {
                     const int up = u > 0 ? u - 1 : nt - 1;
                     const int width = up < nt - 1 ? T : K - (nt - 1) * T;
-                    tab.push_back(A(up) * t8.bsize + (l + width) * stride);
+                    tab.push_back(A(up) + (l + width) * stride);
                 } else {
                     tab.push_back(-1);
                 }
             }
         }
         PGM_TRY(upload(c->merge_tab, tab.data(), tab.size(), c->stream));
+        for (int u0 = 0; u0 < t.nc[0]; ++u0)
+            for (int u1 = 0; u1 < t.nc[1]; ++u1)
+                for (int u2 = 0; u2 < t.nc[2]; ++u2) org.push_back(u0 | (u1 << 10) | (u2 << 20));
+        PGM_TRY(upload(c->corg, org.data(), org.size(), c->stream));
     }
-    // gather partials come per gather tile: the partial buffers must hold B ntiles entries
-    for (DevBuf *b : {&c->partA, &c->partB}) PGM_TRY(b->ensure(std::max(b->bytes, sizeof(double) * 4 * B * t16.ntiles)));
-    // dynamic LDS of the tiled spread and gather beyond the default limit
-    const size_t lds_spread = spread_lds_bytes(c), lds_gather = c->rsize * (size_t)t16.bsize;
-    PGM_TRY(allow_lds(c, lds_spread, lds_gather));
+    // gather partials come per workgroup of the tiled gather (at least two tiles)
+    for (DevBuf *b : {&c->partA, &c->partB}) PGM_TRY(b->ensure(std::max(b->bytes, sizeof(double) * B * t.ntiles)));
     return PGM_OK;
 }
 
-// Sort the atoms by fine key and store their spline weights (once per geometry).
+// Sort the atoms by fine key and store their stencils in that order (once per geometry).
 template <typename real> static int pme_bin(pgm_ctx *c, const double *pos) {
     if (!c->tiled) return PGM_OK;
     const int n = c->n;
     hipStream_t st = c->stream;
-    const PMETiles &t8 = c->tiles8, &t16 = c->tiles;
-    const int nk8 = c->nbead * t8.ntiles, nk16 = c->nbead * t16.ntiles;
-    k_pme_bin<<<nblk(n, 256), 256, 0, st>>>(n, c->nper, pos, c->pg, t8, t16, c->pkey.as<int>(), c->pidx.as<int>());
+    const PMETiles &t = c->tiles;
+    const int nk = c->nbead * t.ntiles;
+    k_pme_bin<<<nblk(n, 256), 256, 0, st>>>(n, c->nper, pos, c->pg, t, c->pkey.as<int>(), c->pidx.as<int>());
     LAUNCH_CHECK();
     int bits = 1;
-    while ((1 << bits) < nk8) ++bits;
+    while ((1 << bits) < nk) ++bits;
     size_t tmp = 0;
     HIP_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, c->pkey.as<int>(), c->pskey.as<int>(), c->pidx.as<int>(),
                                                c->psidx.as<int>(), n, 0, bits, st));
     PGM_TRY(c->pme_sort_tmp.ensure(tmp));
     HIP_TRY(hipcub::DeviceRadixSort::SortPairs(c->pme_sort_tmp.p, tmp, c->pkey.as<int>(), c->pskey.as<int>(), c->pidx.as<int>(),
                                                c->psidx.as<int>(), n, 0, bits, st));
-    k_tile_bounds<<<nblk(n + 1, 256), 256, 0, st>>>(n, c->pskey.as<int>(), nk8, c->tstart.as<int>(), c->tend.as<int>(), nk16,
-                                                         3, c->tstart16.as<int>(), c->tend16.as<int>());
+    k_tile_bounds<<<nblk(n + 1, 256), 256, 0, st>>>(n, c->pskey.as<int>(), nk, c->trange.as<int2>());
     LAUNCH_CHECK();
-    ORDER_SWITCH(c->s.order, (k_pme_splines<real, PO><<<nblk(n, 256), 256, 0, st>>>(n, pos, c->pg, t8, c->psidx.as<int>(),
-                                                                                    c->spl.as<real>(), c->loc.as<int>(),
-                                                                                    c->loc16.as<int>())));
+    k_pme_stencils<real><<<nblk(n, 256), 256, 0, st>>>(n, pos, c->pg, t, c->psidx.as<int>(), c->sten.as<real4<real>>());
     LAUNCH_CHECK();
     return PGM_OK;
 }
@@ -938,7 +897,7 @@ static int fused_transform(pgm_ctx *c, const int *conv, int iter, hipStream_t st
     const int nth = f.K2 * f.K3 >= 8192 ? pfft_plane_threads<real>() : 256;
     const C *tw = c->pfft_tw.as<C>();
     if (fork && c->fork_stage == 3) HIP_TRY(hipStreamWaitEvent(st, c->ev_join, 0));  // planes after the row field
-    k_pme_fwd_plane<real><<<f.K1 * B, nth, plane, st>>>(f, (size_t)c->tiles8.ntiles * c->tiles8.bsize, c->merge_tab.as<int>(),
+    k_pme_fwd_plane<real><<<f.K1 * B, nth, plane, st>>>(f, (size_t)c->tiles.ntiles * c->tiles.bsize, c->merge_tab.as<int>(),
                                                          c->blocks.as<real>(), c->cgrid.as<C>(), tw, conv, iter);
     if (fork && c->fork_stage == 2) PGM_TRY((*fork)());
     const dim3 gx(nblk((long long)f.K2 * f.K3h, PFFT_COLS), B);
@@ -963,6 +922,23 @@ static int conv_partials(const pgm_ctx *c, bool vir) {
     return use_fused(c, vir) ? nblk((long long)c->pfg.K2 * c->pfg.K3h, PFFT_COLS) : nblk((long long)c->ncplx, 256);
 }
 
+// The tiled spread of dq into the blocks.
+template <typename real>
+static int spread_tiles(pgm_ctx *c, const real4<real> *dq, bool withq, const int *conv, int iter, hipStream_t st, TimedPair tp = {}) {
+    const PMETiles &t = c->tiles;
+    const auto go = [&](auto k) {
+        launch_timed(tp, k, dim3(c->nbead * t.ntiles), dim3(WAVE), 0, st, t, c->corg.as<int>(), c->pg,
+                     c->trange.as<int2>(), c->psidx.as<int>(), c->sten.as<real4<real>>(), dq, c->blocks.as<real>(), conv, iter);
+    };
+    if (withq) {
+        ORDER_SWITCH(c->s.order, go(k_spread_tiles<real, PO, true>));
+    } else {
+        ORDER_SWITCH(c->s.order, go(k_spread_tiles<real, PO, false>));
+    }
+    LAUNCH_CHECK();
+    return PGM_OK;
+}
+
 // fork: called once the spread (fork_stage 1 and 4) or the forward planes (fork_stage 2) are enqueued.
 template <typename real>
 static int spread_fft(pgm_ctx *c, const real4<real> *dq, bool withq, bool energy, const int *conv, int iter,
@@ -973,18 +949,8 @@ static int spread_fft(pgm_ctx *c, const real4<real> *dq, bool withq, bool energy
     const TimedPair tp = energy ? TimedPair{} : timing_pair(c, 1);  // the spread kernel
     const int B = c->nbead;
     if (c->tiled) {
-        const PMETiles &t = c->tiles8;
-        const size_t lds = spread_lds_bytes(c);
-        if (withq) {
-            ORDER_SWITCH(P, launch_timed(tp, k_spread_tiles<real, PO, true>, dim3(B * t.ntiles), dim3(WAVE), lds, st, t, c->pg,
-                                         c->tstart.as<int>(), c->tend.as<int>(), c->psidx.as<int>(), c->spl.as<real>(),
-                                         c->loc.as<int>(), dq, c->blocks.as<real>(), conv, iter));
-        } else {
-            ORDER_SWITCH(P, launch_timed(tp, k_spread_tiles<real, PO, false>, dim3(B * t.ntiles), dim3(WAVE), lds, st, t, c->pg,
-                                         c->tstart.as<int>(), c->tend.as<int>(), c->psidx.as<int>(), c->spl.as<real>(),
-                                         c->loc.as<int>(), dq, c->blocks.as<real>(), conv, iter));
-        }
-        LAUNCH_CHECK();
+        const PMETiles &t = c->tiles;
+        PGM_TRY(spread_tiles<real>(c, dq, withq, conv, iter, st, tp));
         if (use_fused(c, vir_part != nullptr)) {  // merge + transforms + Gc fused (fft.h)
             if (fork && (c->fork_stage == 1 || c->fork_stage == 4)) PGM_TRY((*fork)());
             return fused_transform<real>(c, conv, iter, st, fork, energy ? c->conv_part.as<double>() : nullptr);
@@ -1046,7 +1012,7 @@ static double c_self(const pgm_ctx *c) { return 4.0 * std::pow(c->s.ewald_beta, 
 // Number of per-block partials per bead a field evaluation writes (MODE_FIELD / MODE_AV).
 static int gather_parts(const pgm_ctx *c) {
     if (c->ewald) return nblk(c->n, EW_TILE);
-    return c->tiled ? c->tiles.ntiles : nblk(c->n, 256);
+    return c->tiled ? c->tiles.ntiles / (c->mixed ? gather_waves<float>() : gather_waves<double>()) : nblk(c->n, 256);
 }
 
 // Grid of a per-atom kernel with per-block partials: (blocks per bead, beads).
@@ -1061,11 +1027,17 @@ static int gather_combine(pgm_ctx *c, const real4<real> *dq, int mode, const rea
     const real cself = (real)c_self(c);
     if (c->tiled) {
         const PMETiles &t = c->tiles;
-        ORDER_SWITCH(c->s.order, launch_timed(tp, k_gather_tiles<real, PO>, dim3(c->nbead * t.ntiles), dim3(GATHER_THREADS),
-                                              c->rsize * t.bsize, st, t, c->pg, c->tstart16.as<int>(), c->tend16.as<int>(),
-                                              c->psidx.as<int>(), c->spl.as<real>(), c->loc16.as<int>(), c->grid.as<real>(), dq,
-                                              c->vrow.as<real4<real>>(), c->alpha_r.as<real>(), extra, cself, mode, out, part,
-                                              conv, iter));
+        constexpr int GW = gather_waves<real>(), V = 16 / (int)sizeof(real);
+        const auto go = [&](auto k) {
+            launch_timed(tp, k, dim3(c->nbead * t.ntiles / GW), dim3(WAVE * GW), 0, st, t, c->corg.as<int>(), c->pg,
+                         c->trange.as<int2>(), c->psidx.as<int>(), c->sten.as<real4<real>>(), c->grid.as<real>(), dq,
+                         c->vrow.as<real4<real>>(), c->alpha_r.as<real>(), extra, cself, mode, out, part, conv, iter);
+        };
+        if (c->s.grid[2] % V == 0 && t.T[2] % V == 0) {
+            ORDER_SWITCH(c->s.order, go(k_gather_tiles<real, PO, true>));
+        } else {
+            ORDER_SWITCH(c->s.order, go(k_gather_tiles<real, PO, false>));
+        }
     } else {
         ORDER_SWITCH(c->s.order, launch_timed(tp, k_gather_combine<real, PO>, dim3(nblk(n, 256)), dim3(256), 0, st, n, c->pos,
                                               c->pg, c->grid.as<real>(), dq, c->vrow.as<real4<real>>(), c->alpha_r.as<real>(),
@@ -2160,8 +2132,8 @@ extern "C" int pgm_ctx_destroy(pgm_ctx *c) {
                      &c->pair_part, &c->pack_part, &c->conv_part, &c->st, &c->rz, &c->err, &c->energy, &c->bead_it, &c->bead_res,
                      &c->mrows, &c->mcount_full, &c->mcount, &c->mj, &c->mg, &c->pinv,
                      &c->pos_build, &c->minv, &c->mass, &c->d2, &c->md_part, &c->md_fail, &c->heat,
-                     &c->pkey, &c->pidx, &c->pskey, &c->psidx, &c->tstart, &c->tend, &c->tstart16, &c->tend16, &c->spl, &c->loc,
-                     &c->loc16, &c->blocks, &c->merge_tab, &c->pfft_tw,
+                     &c->pkey, &c->pidx, &c->pskey, &c->psidx, &c->trange, &c->corg, &c->sten,
+                     &c->blocks, &c->merge_tab, &c->pfft_tw,
                      &c->pme_sort_tmp, &c->stats, &c->mol_ptr, &c->mol_atoms, &c->com, &c->off, &c->rec_dd,
                      &c->vir_pair, &c->vir_conv, &c->vir_atoms, &c->vir_cov, &c->vir_out, &c->kvec, &c->sk,
                      &c->guess.params, &c->guess.grads, &c->guess.m, &c->guess.v, &c->guess.packed, &c->guess.bias,
@@ -2255,9 +2227,7 @@ static int pme_api(pgm_ctx *c, const double *pos, int withq, const double *d, do
     LAUNCH_CHECK();
     PGM_TRY(spread_fft<real>(c, c->vdq.as<R4>(), withq != 0, true, nullptr, -1));
     if (grad_d) {
-        ORDER_SWITCH(c->s.order, (k_gather_combine<real, PO><<<nb, 256, 0, c->stream>>>(
-                                     c->n, pos, c->pg, c->grid.as<real>(), c->vdq.as<R4>(), c->vrow.as<R4>(),
-                                     c->alpha_r.as<real>(), nullptr, real(0), MODE_REC, c->vtmp.as<R4>(), nullptr, nullptr, -1)));
+        PGM_TRY(gather_combine<real>(c, c->vdq.as<R4>(), MODE_REC, nullptr, c->vtmp.as<R4>(), nullptr, nullptr, -1));
         k_to_double3<real><<<nb, 256, 0, c->stream>>>(c->n, c->vtmp.as<R4>(), grad_d);
         LAUNCH_CHECK();
     }
@@ -2298,18 +2268,8 @@ template <typename real> static int spread_api(pgm_ctx *c, const double *pos, in
     const int *conv = nullptr;
     const int iter = -1;
     if (c->tiled) {
-        const PMETiles &t = c->tiles8;
-        const size_t lds = spread_lds_bytes(c);
-        if (withq) {
-            ORDER_SWITCH(P, (k_spread_tiles<real, PO, true><<<t.ntiles, WAVE, lds, st>>>(
-                                t, c->pg, c->tstart.as<int>(), c->tend.as<int>(), c->psidx.as<int>(), c->spl.as<real>(),
-                                c->loc.as<int>(), dq, c->blocks.as<real>(), conv, iter)));
-        } else {
-            ORDER_SWITCH(P, (k_spread_tiles<real, PO, false><<<t.ntiles, WAVE, lds, st>>>(
-                                t, c->pg, c->tstart.as<int>(), c->tend.as<int>(), c->psidx.as<int>(), c->spl.as<real>(),
-                                c->loc.as<int>(), dq, c->blocks.as<real>(), conv, iter)));
-        }
-        LAUNCH_CHECK();
+        const PMETiles &t = c->tiles;
+        PGM_TRY(spread_tiles<real>(c, dq, withq != 0, conv, iter, st));
         const int *K = c->s.grid;
         k_merge_table<real><<<dim3(nblk(K[2], 128), K[1], K[0]), 128, 0, st>>>(
             K[0], K[1], K[2], (size_t)t.ntiles * t.bsize, c->merge_tab.as<int>(), c->blocks.as<real>(), c->grid.as<real>(), conv,
@@ -3473,13 +3433,8 @@ template <typename real> static int time_impl(pgm_ctx *c, const double *pos, int
     };
     int rc = PGM_OK;
     if (c->tiled) {
-        const PMETiles &t = c->tiles8;
-        const size_t lds = spread_lds_bytes(c);
-        ORDER_SWITCH(c->s.order, rc = timed(1, [&] {
-                                     k_spread_tiles<real, PO, false><<<c->nbead * t.ntiles, WAVE, lds, st>>>(
-                                         t, c->pg, c->tstart.as<int>(), c->tend.as<int>(), c->psidx.as<int>(), c->spl.as<real>(),
-                                         c->loc.as<int>(), dq, c->blocks.as<real>(), nullptr, -1);
-                                 }));
+        const PMETiles &t = c->tiles;
+        rc = timed(1, [&] { (void)spread_tiles<real>(c, dq, false, nullptr, -1, st); });
         if (rc < 0) return rc;
         const int *K = c->s.grid;
         rc = timed(0, [&] {
@@ -3505,7 +3460,7 @@ template <typename real> static int time_impl(pgm_ctx *c, const double *pos, int
         const C *tw = c->pfft_tw.as<C>();
         ms[0] = 0.0;
         rc = timed(2, [&] {
-            k_pme_fwd_plane<real><<<f.K1 * c->nbead, nth, plane, st>>>(f, (size_t)c->tiles8.ntiles * c->tiles8.bsize,
+            k_pme_fwd_plane<real><<<f.K1 * c->nbead, nth, plane, st>>>(f, (size_t)c->tiles.ntiles * c->tiles.bsize,
                                                                         c->merge_tab.as<int>(), c->blocks.as<real>(),
                                                                         c->cgrid.as<C>(), tw, nullptr, -1);
         });
@@ -3612,7 +3567,7 @@ template <typename real> static int autotune_impl(pgm_ctx *c, const double *pos,
             c->tile_cap = cap;
             PGM_TRY(setup_tiles(c));
             if (!c->tiled) continue;
-            const int key = (c->tiles8.T[0] * 16 + c->tiles8.T[1]) * 16 + c->tiles8.T[2];
+            const int key = (c->tiles.T[0] * 16 + c->tiles.T[1]) * 16 + c->tiles.T[2];
             if (std::find(tried.begin(), tried.end(), key) != tried.end()) continue;
             tried.push_back(key);
             PGM_TRY(prepare(c, pos));
@@ -3681,7 +3636,7 @@ template <typename real> static int autotune_impl(pgm_ctx *c, const double *pos,
     HIP_TRY(hipEventDestroy(e1));
     out[0] = c->layout;
     out[1] = c->layout == 1 ? c->rlm : RL;
-    for (int a = 0; a < 3; ++a) out[2 + a] = c->tiled ? c->tiles8.T[a] : 0;
+    for (int a = 0; a < 3; ++a) out[2 + a] = c->tiled ? c->tiles.T[a] : 0;
     out[5] = best_row;
     out[6] = best_pme < 1e300 ? best_pme : 0.0;
     out[7] = (double)lays.size();

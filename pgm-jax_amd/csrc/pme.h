@@ -32,6 +32,21 @@ PGM_DEV void stencil(const double *__restrict__ pos, int i, const PMEGeom &g, in
     }
 }
 
+// bspline of order P at f, evaluated in FP64 and rounded to real.  FP32 recursions lose a few units in the
+// last place of every weight, with the same sign for the whole grid: at 32,768 waters the field's error
+// against float64 was 3.4e-7 with them and is 2.6e-7 with the weights rounded once; the spread's time did
+// not change.
+template <typename real, int P, bool D2> PGM_DEV void bspline_rounded(real f, real *th, real *dth, real *d2th) {
+    double t[P], d[P], d2[P];
+    bspline<double, P, D2>((double)f, t, d, d2);
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+        th[k] = (real)t[k];
+        dth[k] = (real)d[k];
+        if (D2) d2th[k] = (real)d2[k];
+    }
+}
+
 template <typename real>
 PGM_DEV void scaled_dipole(const real4<real> &d, const PMEGeom &g, real *e) {
 #pragma unroll
@@ -87,32 +102,34 @@ __global__ __launch_bounds__(256) void k_spread(int n, const double *__restrict_
 
 // ---------------------------------------------------------------------------- tiled spread
 // Atomic-free, deterministic spread.  The grid is cut into tiles (T_a points per axis, every tile at
-// least P-1 wide, at least two tiles per axis); every atom belongs to the tile holding its stencil
-// base.  Atoms are sorted by tile once per geometry (k_pme_bin + radix sort + k_pme_splines, which
-// also stores the spline weights in sorted order).  One wave per tile accumulates its atoms' full
-// P^3 stencils into an LDS block of (T+P-1)^3 points: one atom at a time, the 64 lanes take 64
-// distinct stencil points, so plain LDS read-add-write is race free and the order is fixed.  The
-// blocks are written out and k_merge_table sums, for every grid point, the (up to 8) blocks that
-// cover it in a fixed order.
+// least P-1 wide, at least three tiles per axis); every atom belongs to the tile holding its stencil
+// base.  Atoms are sorted by tile once per geometry (k_pme_bin + radix sort + k_pme_stencils).  One
+// wave per tile sums its atoms' stencils on the tile's block of (T+P-1)^3 points on the matrix cores
+// (k_spread_tiles), and k_merge_table (or the forward planes of the fused transform) sums, for
+// every grid point, the (up to 8) blocks that cover it in a fixed order.
 struct PMETiles {
     int T[3];    // tile width per axis (the last tile may be narrower, >= P-1)
     int nt[3];   // tiles per axis
-    int B[3];    // LDS block extent per axis: T + P - 1
-    int ntiles;  // nt0 nt1 nt2
-    int bsize;   // B0 B1 B2
+    int nc[3];   // cubes of 2 x 2 x 2 tiles per axis: (nt + 1) / 2
+    int ncubes;  // nc0 nc1 nc2
+    int ntiles;  // 8 ncubes: tiles by fine key (octants past the grid stay empty)
+    int B[3];    // extent of a tile's block per axis: T + P - 1
+    int bsize;   // values stored per block: B0 B1 PME_ZROW
 };
 
-// The spread works on tiles of T8 points per axis, the gather on tiles of T16 = 2 T8 (each the
-// union of 2 x 2 x 2 spread tiles).  Atoms are sorted once per geometry by the fine key
-// key = t16 index * 8 + octant, so both the spread tiles (one key each) and the gather tiles (eight
-// consecutive keys) are contiguous ranges of the sorted order.
-PGM_DEV int fine_key(const int (&u8)[3], const PMETiles &t16) {
+// z rows of the stored spread blocks: padded to 16 values, so that a row is one aligned segment and one
+// column block of the matrix instructions.
+constexpr int PME_ZROW = 16;
+
+// Tiles are numbered by the fine key = cube index * 8 + octant, so that consecutive keys are near each
+// other in space.
+PGM_DEV int fine_key(const int (&u8)[3], const PMETiles &t) {
     const int oct = ((u8[0] & 1) << 2) | ((u8[1] & 1) << 1) | (u8[2] & 1);
-    return (((u8[0] >> 1) * t16.nt[1] + (u8[1] >> 1)) * t16.nt[2] + (u8[2] >> 1)) * 8 + oct;
+    return (((u8[0] >> 1) * t.nc[1] + (u8[1] >> 1)) * t.nc[2] + (u8[2] >> 1)) * 8 + oct;
 }
 
 // key = bead * t8.ntiles + fine key of each atom's stencil base (nper atoms per bead); idx = atom index.
-__global__ void k_pme_bin(int n, int nper, const double *__restrict__ pos, PMEGeom g, PMETiles t8, PMETiles t16,
+__global__ void k_pme_bin(int n, int nper, const double *__restrict__ pos, PMEGeom g, PMETiles t8,
                           int *__restrict__ key, int *__restrict__ idx) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -126,164 +143,205 @@ __global__ void k_pme_bin(int n, int nper, const double *__restrict__ pos, PMEGe
         const int u = bb / t8.T[a];
         u8[a] = u < t8.nt[a] ? u : t8.nt[a] - 1;
     }
-    key[i] = (i / nper) * t8.ntiles + fine_key(u8, t16);
+    key[i] = (i / nper) * t8.ntiles + fine_key(u8, t8);
     idx[i] = i;
 }
 
-// Spline weights in sorted order: spl[s] = (t0[P], d0[P], t1[P], d1[P], t2[P], d2[P]) of atom
-// sidx[s]; loc8[s] / loc16[s] = the stencil base relative to its spread / gather tile start,
-// packed (lx | ly << 10 | lz << 20).
-template <typename real, int P>
-__global__ void k_pme_splines(int n, const double *__restrict__ pos, PMEGeom g, PMETiles t8, const int *__restrict__ sidx,
-                              real *__restrict__ spl, int *__restrict__ loc8, int *__restrict__ loc16) {
+// Tile coordinates of octant oct of a cube whose packed coordinates (u0 | u1 << 10 | u2 << 20) are org; false
+// for an octant past the grid.
+PGM_DEV bool octant_tile(int org, int oct, const PMETiles &t, int (&u8)[3]) {
+    u8[0] = 2 * (org & 1023) + (oct >> 2);
+    u8[1] = 2 * ((org >> 10) & 1023) + ((oct >> 1) & 1);
+    u8[2] = 2 * (org >> 20) + (oct & 1);
+    return u8[0] < t.nt[0] && u8[1] < t.nt[1] && u8[2] < t.nt[2];
+}
+
+// The stencil of a sorted atom: the offsets f in [0, 1) along the axes (rounded to real, the arguments of
+// bspline) and the base point relative to its tile, packed (lx | ly << 5 | lz << 10) in the bits of w.
+// 16 bytes per atom (FP32): the spread and the gather evaluate the splines from it (about 60
+// instructions per axis) rather than read 6 P stored weights per atom, whose rows of 144 bytes made each
+// of the gather's 36 loads touch one cache line per lane.
+PGM_DEV float pack_loc(int v, float) { return __int_as_float(v); }
+PGM_DEV double pack_loc(int v, double) { return __longlong_as_double((long long)v); }
+PGM_DEV int unpack_loc(float v) { return __float_as_int(v); }
+PGM_DEV int unpack_loc(double v) { return (int)__double_as_longlong(v); }
+
+template <typename real>
+__global__ void k_pme_stencils(int n, const double *__restrict__ pos, PMEGeom g, PMETiles t8, const int *__restrict__ sidx,
+                               real4<real> *__restrict__ sten) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n) return;
-    const int i = sidx[s];
     int base[3];
     real f[3];
-    stencil<real, P>(pos, i, g, base, f);
-    int l8[3], l16[3];
+    stencil<real, 4>(pos, sidx[s], g, base, f);
+    int loc = 0;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         const int bb = base[a] >= g.K[a] ? base[a] - g.K[a] : base[a];
         int u = bb / t8.T[a];
         u = u < t8.nt[a] ? u : t8.nt[a] - 1;
-        l8[a] = bb - u * t8.T[a];
-        l16[a] = l8[a] + (u & 1) * t8.T[a];
-        real th[P], dth[P];
-        bspline<real, P, false>(f[a], th, dth, nullptr);
-#pragma unroll
-        for (int k = 0; k < P; ++k) {
-            spl[(size_t)s * 6 * P + (2 * a) * P + k] = th[k];
-            spl[(size_t)s * 6 * P + (2 * a + 1) * P + k] = dth[k];
-        }
+        loc |= (bb - u * t8.T[a]) << (5 * a);
     }
-    loc8[s] = l8[0] | (l8[1] << 10) | (l8[2] << 20);
-    loc16[s] = l16[0] | (l16[1] << 10) | (l16[2] << 20);
+    real4<real> v;
+    v.x = f[0];
+    v.y = f[1];
+    v.z = f[2];
+    v.w = pack_loc(loc, real(0));
+    sten[s] = v;
 }
 
-// The atom ranges of every spread tile and every gather tile from the sorted keys, in one launch and
-// without clearing first.  Thread s in [0, n] looks at the keys either side of position s (key -1
-// before the first, the tile count after the last): position s is the start of every tile k with
-// key[s-1] < k <= key[s] and the end of tile k - 1, so every tile's start and end is written once
-// and an empty tile gets an empty range.  Spread tiles are the keys, gather tiles key >> shift.
-__global__ void k_tile_bounds(int n, const int *__restrict__ skey, int n8, int *__restrict__ start8, int *__restrict__ end8,
-                              int n16, int shift, int *__restrict__ start16, int *__restrict__ end16) {
+// The atom ranges of every tile from the sorted keys, in one launch and without clearing first.
+// Thread s in [0, n] looks at the keys either side of position s (key -1 before the first, the tile
+// count after the last): position s is the start of every tile k with key[s-1] < k <= key[s] and the
+// end of tile k - 1, so every tile's start and end is written once and an empty tile gets an empty
+// range.
+__global__ void k_tile_bounds(int n, const int *__restrict__ skey, int n8, int2 *__restrict__ range) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s > n) return;
     const int p8 = s > 0 ? skey[s - 1] : -1, c8 = s < n ? skey[s] : n8;
     for (int k = p8 + 1; k <= c8; ++k) {
-        if (k < n8) start8[k] = s;
-        if (k > 0 && k <= n8) end8[k - 1] = s;
-    }
-    const int p16 = s > 0 ? skey[s - 1] >> shift : -1, c16 = s < n ? skey[s] >> shift : n16;
-    for (int k = p16 + 1; k <= c16; ++k) {
-        if (k < n16) start16[k] = s;
-        if (k > 0 && k <= n16) end16[k - 1] = s;
+        if (k < n8) range[k].x = s;
+        if (k > 0 && k <= n8) range[k - 1].y = s;
     }
 }
 
-// Tiled spread: one wave per spread tile (fine key; block b * t.ntiles + key for bead b) accumulates
-// the stencils of its atoms into an LDS block of (T8 + P - 1)^3 points, written to `blocks` (merged
-// by k_merge_table).  The atoms'
-// spline weights, scaled dipoles, charges and local offsets are staged through LDS in chunks of
-// SPREAD_CHUNK (one parallel load instead of a chain of dependent loads per atom); the 64 lanes
-// cover the P^3 stencil points of one atom at a time, so no two lanes touch one point and the sum
-// is free of atomics and bitwise reproducible (an LDS float add, ds_add_f32, in place of the read and
-// write measured three times slower).
-constexpr int SPREAD_CHUNK = 8;  // atoms staged at a time: 10 KB of LDS per wave, 16 waves (all 8^3 tiles of 128^3) per CU
+// Tiled spread on the matrix cores: one wave per tile (fine key; block b * t.ntiles + key for bead b).
+// On the tile's block the sum over its atoms is, for every y, a product of two thin matrices,
+//   Q[x][z] = sum_a X1[x][a] (Y[y][a] Z[a][z]) + X2[x][a] (Y'[y][a] e2 Z[a][z] + Y[y][a] e3 Z'[a][z]),
+//   X1 = q theta_x + e1 theta'_x,  X2 = theta_x,
+// with the weights zero outside an atom's P points: 16 x 16 x 4 matrix instructions over four atoms at
+// a time (x the rows, z the columns; FP32 or FP64), the block held in accumulators of at most 15 rows y
+// until it is stored.  The atoms come in chunks of SPREAD_CHUNK: 3 x SPREAD_CHUNK lanes evaluate one
+// axis' spline of one atom each into dense rows in LDS.  All rows y are taken for every four atoms: a
+// test per row, to skip those out of reach, takes the independent products out of one stream and costs
+// more than it saves (50 us).  No atomics and a fixed order: bitwise reproducible.
+//
+// Bound by the matrix instructions (8 us at 4,096 tiles of 24 atoms) and by writing the blocks (44 MB at
+// 128^3).  Measured per launch (FP32, alone) at 32,768 waters and 128^3 / 512 waters and 32^3: 24.1 / 9.8
+// us; the earlier form, one atom at a time with a read-add-write of its 216 points in LDS, 26.8 / 13.7 us;
+// summing the eight tiles of a cube in LDS first (22 MB written) 30.0 / 19.3 us.
+constexpr int SPREAD_CHUNK = 16;
+constexpr int SPREAD_ROW = 17;  // LDS row of one atom's dense weights (16 points; odd: no bank conflicts)
+constexpr int SPREAD_PLANES = 7;  // X1, X2, Y, Y', Z, e2 Z, e3 Z'
 
-template <typename real, int P>
-PGM_DEV constexpr int spread_lds_atoms() {
-    return SPREAD_CHUNK * (6 * P + 4) * (int)sizeof(real) + SPREAD_CHUNK * (int)sizeof(int);
+template <typename real> struct mfma_acc;
+template <> struct mfma_acc<float> { typedef float type __attribute__((ext_vector_type(4))); };
+template <> struct mfma_acc<double> { typedef double type __attribute__((ext_vector_type(4))); };
+PGM_DEV mfma_acc<float>::type mfma_16x16x4(float a, float b, mfma_acc<float>::type c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
+PGM_DEV mfma_acc<double>::type mfma_16x16x4(double a, double b, mfma_acc<double>::type c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+// Row of result register r of lane group grp = lane / 16 (lane l holds column l % 16).
+template <typename real> PGM_DEV int mfma_row(int grp, int r) { return sizeof(real) == 4 ? 4 * grp + r : grp + 4 * r; }
 
 template <typename real, int P, bool WITHQ>
-__global__ __launch_bounds__(64) void k_spread_tiles(PMETiles t, PMEGeom g, const int *__restrict__ tstart,
-                                                     const int *__restrict__ tend, const int *__restrict__ sidx,
-                                                     const real *__restrict__ spl, const int *__restrict__ loc,
-                                                     const real4<real> *__restrict__ dq, real *__restrict__ blocks,
-                                                     const int *__restrict__ conv_it, int iter) {
-    if (cg_done(conv_it, blockIdx.x / t.ntiles, iter)) return;
-    extern __shared__ __align__(16) unsigned char lds_raw[];
-    constexpr int SW = 6 * P + 4;  // staged values per atom: splines, e0 e1 e2 q
-    real *sv = reinterpret_cast<real *>(lds_raw);
-    int *sl = reinterpret_cast<int *>(sv + SPREAD_CHUNK * SW);
-    real *blk = reinterpret_cast<real *>(lds_raw + spread_lds_atoms<real, P>());
-    const int lane = threadIdx.x;
-    const int key = blockIdx.x;
-    const int BY = t.B[1], BZ = t.B[2];
-    for (int k = lane; k < t.bsize; k += WAVE) blk[k] = real(0);
-    const int s0 = tstart[key], s1 = tend[key];
-    // this lane's stencil points p = lane + 64 u (the last pass only where p < P^3): axis indices
-    // and block offsets, the same for every atom
-    constexpr int NP = P * P * P, NPASS = (NP + WAVE - 1) / WAVE;
-    static_assert((NPASS - 1) * WAVE < NP, "every pass but the last is full");
-    int pix[NPASS], piy[NPASS], piz[NPASS], poff[NPASS];
-    const bool plast = lane + (NPASS - 1) * WAVE < NP;
+__global__ __launch_bounds__(64, sizeof(real) == 4 ? 4 : 2) void k_spread_tiles(PMETiles t, const int *__restrict__ corg, PMEGeom g,
+                                                     const int2 *__restrict__ range, const int *__restrict__ sidx,
+                                                     const real4<real> *__restrict__ sten, const real4<real> *__restrict__ dq,
+                                                     real *__restrict__ blocks, const int *__restrict__ conv_it, int iter) {
+    const int bead = blockIdx.x / t.ntiles, key = blockIdx.x - bead * t.ntiles;
+    if (cg_done(conv_it, bead, iter)) return;
+    int u8[3];
+    if (!octant_tile(corg[key >> 3], key & 7, t, u8)) return;  // no merge reads the block
+    using acc_t = typename mfma_acc<real>::type;
+    constexpr int MAXB = P + 7;  // tile rows at most (T <= 8)
+    constexpr int PLANE = SPREAD_CHUNK * SPREAD_ROW;
+    constexpr int NZ = (SPREAD_PLANES * PLANE * (int)sizeof(real) + 15) / 16;
+    __shared__ float4 w4[NZ];
+    real *w = reinterpret_cast<real *>(w4);
+    const int lane = threadIdx.x, grp = lane / 16, m = lane % 16;
+    const int2 rg = range[blockIdx.x];
+    const int s0 = rg.x, s1 = rg.y;
+    acc_t D[MAXB];
 #pragma unroll
-    for (int u = 0; u < NPASS; ++u) {
-        const int p = (u < NPASS - 1 || plast) ? lane + u * WAVE : 0;
-        pix[u] = p / (P * P);
-        piy[u] = (p / P) % P;
-        piz[u] = p % P;
-        poff[u] = (pix[u] * BY + piy[u]) * BZ + piz[u];
+    for (int y = 0; y < MAXB; ++y) D[y] = acc_t{0, 0, 0, 0};
+    const int ax = lane / SPREAD_CHUNK, a = lane % SPREAD_CHUNK;  // this lane's axis (0..2) and atom of a chunk
+    real4<real> st{}, d{};
+    if (ax < 3 && s0 + a < s1) {
+        st = sten[s0 + a];
+        d = dq[sidx[s0 + a]];
     }
     for (int c0 = s0; c0 < s1; c0 += SPREAD_CHUNK) {
-        const int m = min(SPREAD_CHUNK, s1 - c0);
-        __syncthreads();
-        for (int k = lane; k < m * 6 * P; k += WAVE) {  // (theta, dtheta) pairs per axis point
-            const int a = k / (6 * P), v = k - a * 6 * P;
-            const int ax = v / (2 * P), w = v - ax * 2 * P, which = w / P, i = w - which * P;
-            sv[a * SW + ax * 2 * P + 2 * i + which] = spl[(size_t)(c0 + a) * 6 * P + v];
-        }
-        if (lane < m) {
-            const real4<real> d = dq[sidx[c0 + lane]];
-            real e[3];
-            scaled_dipole<real>(d, g, e);
-            sv[lane * SW + 6 * P] = e[0];
-            sv[lane * SW + 6 * P + 1] = e[1];
-            sv[lane * SW + 6 * P + 2] = e[2];
-            sv[lane * SW + 6 * P + 3] = WITHQ ? d.w : real(0);
-            sl[lane] = loc[c0 + lane];
-        }
-        __syncthreads();
-        for (int a = 0; a < m; ++a) {
-            const real *v = sv + a * SW;
-            const int lc = sl[a];
-            const int lx = lc & 1023, ly = (lc >> 10) & 1023, lz = lc >> 20;
-            const real e0 = v[6 * P], e1 = v[6 * P + 1], e2 = v[6 * P + 2], q = v[6 * P + 3];
-            const int base = (lx * BY + ly) * BZ + lz;
-            real w[NPASS], old[NPASS];
+        const int mc = min(SPREAD_CHUNK, s1 - c0);
+        const bool on = ax < 3 && a < mc;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the previous chunk's rows have been read
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
-            for (int u = 0; u < NPASS; ++u) {
-                const real tx = v[2 * pix[u]], dx = v[2 * pix[u] + 1];
-                const real ty = v[2 * P + 2 * piy[u]], dy = v[2 * P + 2 * piy[u] + 1];
-                const real tz = v[4 * P + 2 * piz[u]], dz = v[4 * P + 2 * piz[u] + 1];
-                w[u] = (q * tx + e0 * dx) * ty * tz + tx * (e1 * dy * tz + e2 * ty * dz);
+        for (int k = 0; k < NZ; k += WAVE)
+            if (k + lane < NZ) w4[k + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (on) {
+            const int l = (unpack_loc(st.w) >> (5 * ax)) & 31;
+            double th[P], dth[P], e[3];
+            bspline<double, P, false>((double)(ax == 0 ? st.x : (ax == 1 ? st.y : st.z)), th, dth, nullptr);
+#pragma unroll
+            for (int b = 0; b < 3; ++b) e[b] = (double)d.x * g.escale[b] + (double)d.y * g.escale[3 + b] + (double)d.z * g.escale[6 + b];
+            const double q = WITHQ ? (double)d.w : 0.0;
+            real *row = w + a * SPREAD_ROW + l;
+            if (ax == 0) {
+#pragma unroll
+                for (int k = 0; k < P; ++k) {
+                    row[k] = (real)(q * th[k] + e[0] * dth[k]);
+                    row[PLANE + k] = (real)th[k];
+                }
+            } else if (ax == 1) {
+#pragma unroll
+                for (int k = 0; k < P; ++k) {
+                    row[2 * PLANE + k] = (real)th[k];
+                    row[3 * PLANE + k] = (real)dth[k];
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < P; ++k) {
+                    row[4 * PLANE + k] = (real)th[k];
+                    row[5 * PLANE + k] = (real)(e[1] * th[k]);
+                    row[6 * PLANE + k] = (real)(e[2] * dth[k]);
+                }
             }
+        }
+        if (ax < 3 && c0 + SPREAD_CHUNK + a < s1) {  // the next chunk's atoms, in flight with the products
+            st = sten[c0 + SPREAD_CHUNK + a];
+            d = dq[sidx[c0 + SPREAD_CHUNK + a]];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        for (int a0 = 0; a0 < mc; a0 += 4) {
+            const real *row = w + (a0 + grp) * SPREAD_ROW;
+            const real x1 = row[m], x2 = row[PLANE + m];
+            const real z0 = row[4 * PLANE + m], z1 = row[5 * PLANE + m], z2 = row[6 * PLANE + m];
 #pragma unroll
-            for (int u = 0; u < NPASS; ++u)
-                if (u < NPASS - 1 || plast) old[u] = blk[base + poff[u]];
-#pragma unroll
-            for (int u = 0; u < NPASS; ++u)
-                if (u < NPASS - 1 || plast) blk[base + poff[u]] = old[u] + w[u];
+            for (int y = 0; y < MAXB; ++y) {
+                const real ty = row[2 * PLANE + y], dy = row[3 * PLANE + y];
+                D[y] = mfma_16x16x4(x1, ty * z0, D[y]);
+                D[y] = mfma_16x16x4(x2, dy * z1 + ty * z2, D[y]);
+            }
         }
     }
-    __syncthreads();
-    real *out = blocks + (size_t)key * t.bsize;
-    for (int k = lane; k < t.bsize; k += WAVE) out[k] = blk[k];
+    real *out = blocks + (size_t)blockIdx.x * t.bsize + m;
+#pragma unroll
+    for (int y = 0; y < MAXB; ++y) {
+        if (y < t.B[1]) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int x = mfma_row<real>(grp, r);
+                if (x < t.B[0]) out[(x * t.B[1] + y) * PME_ZROW] = D[y][r];
+            }
+        }
+    }
 }
 
-// Block merge: grid point value = sum of the spread blocks covering it -- along each axis its own
-// spread tile (local l) and, when l <= P-2, the previous one (local l + width of that tile), in a
-// fixed order (deterministic).  Table driven: for grid coordinate g along axis a, tab_a[2 g] is the offset (in reals) of the
-// point in the block of its own spread tile's axis part -- A_a(u) bsize + l stride_a with
-// A_0(u) = ((u >> 1) nt16_1 nt16_2 8 + (u & 1) 4), A_1(u) = ((u >> 1) nt16_2 8 + (u & 1) 2),
-// A_2(u) = ((u >> 1) 8 + (u & 1)), strides B1 B2, B2, 1 -- and tab_a[2 g + 1] the same for the
-// previous tile (local l + its width) when l <= P-2, else -1.  Both the fine key and the in-block
-// offset are sums over the axes, so a grid point's up to 8 block values are
-// blocks[bead base + X + Y + Z] over the axes' candidates, summed in a fixed order.
+// Block merge: grid point value = sum of the tiles' blocks covering it -- along each axis its own tile
+// (local l) and, when l <= P-2, the previous one (local l + width of that tile), in a fixed order
+// (deterministic).  Table driven: for grid coordinate g along axis a, tab_a[2 g] is the offset (in reals)
+// of the point in the axis part of its own tile's block -- A_a(u) bsize + l stride_a with A_0(u) =
+// ((u >> 1) nc1 nc2 8 + (u & 1) 4), A_1(u) = ((u >> 1) nc2 8 + (u & 1) 2), A_2(u) = ((u >> 1) 8 + (u & 1)),
+// strides B1 PME_ZROW, PME_ZROW, 1 -- and tab_a[2 g + 1] the same for the previous tile (local l + its
+// width) when l <= P-2, else -1.  Both the fine key and the in-block offset are sums over the axes, so a
+// grid point's up to 8 block values are blocks[bead base + X + Y + Z] over the axes' candidates, summed
+// in a fixed order.
 // Launch: x = z-line (blockDim.x points), y = K2 rows, z = K1 planes times beads.
 template <typename real>
 __global__ __launch_bounds__(128) void k_merge_table(int K1, int K2, int K3, size_t bead_blocks, const int *__restrict__ tab,
@@ -438,114 +496,144 @@ PGM_DEV void combine_out(int mode, int i, real rx, real ry, real rz, const real4
     out[i] = o;
 }
 
-// Tiled gather + combine: one 512-thread workgroup per grid tile loads the potential on the
-// tile's (T + P - 1)^3 block (periodic wrap) into LDS once, then every atom binned to the tile
-// (two neighbouring threads per atom, sorted order s, atom sidx[s]: the first (P+1)/2 x planes of
-// its stencil and the rest, summed with one shuffle) sums its stencil values from LDS with the
-// spline weights stored by k_pme_splines, and the first thread's combine_out writes its result.  Per-block partials
-// of MODE_FIELD / MODE_AV go to part[tile].  Block b * t.ntiles + tile serves tile `tile` of bead
-// b (potential at phi + b K1 K2 K3).
-constexpr int GATHER_THREADS = 512;
-template <typename real, int P>
-__global__ __launch_bounds__(GATHER_THREADS) void k_gather_tiles(PMETiles t, PMEGeom g, const int *__restrict__ tstart,
-                                                      const int *__restrict__ tend, const int *__restrict__ sidx,
-                                                      const real *__restrict__ spl, const int *__restrict__ loc,
+// Tiled gather + combine: one wave per tile (fine key), GATHER_WAVES waves per workgroup.  The wave copies
+// the potential on the tile's (T + P - 1)^3 block (periodic wrap) into its part of the LDS, 16 bytes
+// per lane and load where the rows allow it (VEC: K3 and T2 multiples of 16 / sizeof(real)), then two
+// neighbouring lanes per atom (sorted order s, atom sidx[s]) sum its stencil from LDS, the first
+// (P+1)/2 x planes and the rest, and the first lane's combine_out writes the result.  Per-workgroup
+// partials of MODE_FIELD / MODE_AV go to part[blockIdx.x].  The potential of bead b is at phi + b K1 K2 K3.
+// Bound by latency and LDS reads.  Measured against one 512-thread workgroup per 16^3 points reading
+// stored splines (FP32, alone): 22 us at 32,768 waters and 128^3, 10.4 us at 64 waters and 32^3.
+template <typename real> constexpr int gather_waves() { return sizeof(real) == 4 ? 4 : 2; }
+template <typename real, int P, bool VEC>
+__global__ __launch_bounds__(WAVE * gather_waves<real>()) void k_gather_tiles(PMETiles t, const int *__restrict__ corg, PMEGeom g,
+                                                      const int2 *__restrict__ range, const int *__restrict__ sidx,
+                                                      const real4<real> *__restrict__ sten,
                                                       const real *__restrict__ phi, const real4<real> *__restrict__ dq,
                                                       const real4<real> *__restrict__ row, const real *__restrict__ alpha,
                                                       const real4<real> *__restrict__ extra, real cself, int mode,
                                                       real4<real> *__restrict__ out, double *__restrict__ part,
                                                       const int *__restrict__ conv_it, int iter) {
-    const int tile = blockIdx.x, tid = threadIdx.x;
-    const int bead = tile / t.ntiles, lt = tile - bead * t.ntiles;
+    constexpr int GW = gather_waves<real>();
+    const int bead = (blockIdx.x * GW) / t.ntiles;  // t.ntiles is a multiple of 8
     if (cg_done(conv_it, bead, iter)) return;
-    extern __shared__ __align__(16) unsigned char lds_raw[];
-    real *blk = reinterpret_cast<real *>(lds_raw);
+    constexpr int V = VEC ? 16 / (int)sizeof(real) : 1, LPR = 16 / V, RPI = WAVE / LPR;  // reals, lanes per row, rows per load
+    constexpr int MAXB = P + 7, SZ = MAXB | 1;
+    __shared__ real blk_all[GW][MAXB * MAXB * SZ];
     __shared__ double lds[16];
-    const int BX = t.B[0], BY = t.B[1], BZ = t.B[2];
-    const int u2 = lt % t.nt[2], u1 = (lt / t.nt[2]) % t.nt[1], u0 = lt / (t.nt[2] * t.nt[1]);
-    const int o0 = u0 * t.T[0], o1 = u1 * t.T[1], o2 = u2 * t.T[2];
-    const int K1 = g.K[0], K2 = g.K[1], K3 = g.K[2];
-    phi += (size_t)bead * K1 * K2 * K3;
-    // block load, four loads in flight per thread before the LDS stores
-    const int nth = blockDim.x, bs = t.bsize;
-    for (int k0 = tid; k0 < bs; k0 += 4 * nth) {
-        real v[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int k = k0 + u * nth < bs ? k0 + u * nth : 0;
-            const int bz = k % BZ, by = (k / BZ) % BY, bx = k / (BZ * BY);
-            int gx = o0 + bx, gy = o1 + by, gz = o2 + bz;
-            gx -= gx >= K1 ? K1 : 0;
-            gy -= gy >= K2 ? K2 : 0;
-            gz -= gz >= K3 ? K3 : 0;
-            v[u] = phi[((size_t)gx * K2 + gy) * K3 + gz];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (k0 + u * nth < bs) blk[k0 + u * nth] = v[u];
-    }
-    (void)BX;
-    __syncthreads();
-    const int s0 = tstart[tile], s1 = tend[tile];
+    const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE;
+    const int tile = blockIdx.x * GW + wv;
+    real *blk = blk_all[wv];
+    const int BY = t.B[1], BZ = t.B[2], nrow = t.B[0] * BY;
+    const int2 rg = range[tile];
+    const int s0 = rg.x, s1 = rg.y, lt = tile - bead * t.ntiles;
+    const int half = lane & 1;
     double acc[1] = {0.0};
-    const int half = tid & 1;
-    constexpr int PH = (P + 1) / 2;  // x planes of the first thread of a pair
-    for (int s = s0 + (tid >> 1); s < s1; s += blockDim.x >> 1) {  // both threads of a pair: same s
-        const real *v = spl + (size_t)s * 6 * P;
-        real t1[P], d1[P], t2[P], d2[P], t3[P], d3[P];
-#pragma unroll
-        for (int k = 0; k < P; ++k) {
-            t1[k] = v[k];
-            d1[k] = v[P + k];
-            t2[k] = v[2 * P + k];
-            d2[k] = v[3 * P + k];
-            t3[k] = v[4 * P + k];
-            d3[k] = v[5 * P + k];
+    int u8[3];
+    if (s0 < s1 && octant_tile(corg[lt >> 3], lt & 7, t, u8)) {
+        const int K1 = g.K[0], K2 = g.K[1], K3 = g.K[2];
+        phi += (size_t)bead * K1 * K2 * K3;
+        int s = s0 + (lane >> 1);
+        real4<real> st{};
+        int atom = 0;
+        if (s < s1) {  // in flight with the block
+            st = sten[s];
+            atom = sidx[s];
         }
-        const int lc = loc[s];
-        const int lx = lc & 1023, ly = (lc >> 10) & 1023, lz = lc >> 20;
-        real g1 = 0, g2 = 0, g3 = 0;
+        const int bz = V * (lane % LPR);
+        int gz = u8[2] * t.T[2] + bz;
+        gz -= gz >= K3 ? K3 : 0;
+        const int o0 = u8[0] * t.T[0], o1 = u8[1] * t.T[1];
+        const unsigned magic = 65536u / (unsigned)BY + 1u;  // row / BY for row < 256
+        constexpr int BATCH = 8;
+        for (int r0 = lane / LPR; r0 < nrow; r0 += BATCH * RPI) {
+            real v[BATCH][V];
 #pragma unroll
-        for (int ixh = 0; ixh < PH; ++ixh) {
-            const int ix = half ? PH + ixh : ixh;
-            if (ix >= P) break;
-            // spline weights picked with compile-time indices (registers, not scratch)
-            const int ih = PH + ixh < P ? PH + ixh : P - 1;
-            const real d1x = half ? d1[ih] : d1[ixh], t1x = half ? t1[ih] : t1[ixh];
-            real s_tt = 0, s_dt = 0, s_td = 0;
-#pragma unroll
-            for (int iy = 0; iy < P; ++iy) {
-                const real *line = blk + ((lx + ix) * BY + (ly + iy)) * BZ + lz;
-                real lt = 0, ld = 0;
-#pragma unroll
-                for (int iz = 0; iz < P; ++iz) {
-                    const real w = line[iz];
-                    lt += w * t3[iz];
-                    ld += w * d3[iz];
+            for (int u = 0; u < BATCH; ++u) {
+                const int rr = r0 + u * RPI < nrow ? r0 + u * RPI : 0;
+                const int bx = (int)(((unsigned)rr * magic) >> 16), by = rr - bx * BY;
+                int gx = o0 + bx, gy = o1 + by;
+                gx -= gx >= K1 ? K1 : 0;
+                gy -= gy >= K2 ? K2 : 0;
+                const real *src = phi + ((size_t)gx * K2 + gy) * K3 + gz;
+                if constexpr (V == 4) {
+                    const float4 q = *reinterpret_cast<const float4 *>(src);
+                    v[u][0] = q.x, v[u][1] = q.y, v[u][2] = q.z, v[u][3] = q.w;
+                } else if constexpr (V == 2) {
+                    const double2 q = *reinterpret_cast<const double2 *>(src);
+                    v[u][0] = q.x, v[u][1] = q.y;
+                } else {
+                    v[u][0] = bz < BZ ? *src : real(0);
                 }
-                s_tt += lt * t2[iy];
-                s_dt += lt * d2[iy];
-                s_td += ld * t2[iy];
             }
-            g1 += s_tt * d1x;
-            g2 += s_dt * t1x;
-            g3 += s_td * t1x;
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u)
+                if (r0 + u * RPI < nrow)
+#pragma unroll
+                    for (int k = 0; k < V; ++k)
+                        if (bz + k < BZ) blk[(r0 + u * RPI) * SZ + bz + k] = v[u][k];
         }
-        g1 += __shfl_xor(g1, 1, WAVE);
-        g2 += __shfl_xor(g2, 1, WAVE);
-        g3 += __shfl_xor(g3, 1, WAVE);
-        if (half) continue;
-        const double *es = g.escale;
-        const real rx = (real)es[0] * g1 + (real)es[1] * g2 + (real)es[2] * g3;
-        const real ry = (real)es[3] * g1 + (real)es[4] * g2 + (real)es[5] * g3;
-        const real rz = (real)es[6] * g1 + (real)es[7] * g2 + (real)es[8] * g3;
-        double a = 0.0;
-        combine_out<real>(mode, sidx[s], rx, ry, rz, dq, row, alpha, extra, cself, out, a);
-        acc[0] += a;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        constexpr int PH = (P + 1) / 2;  // x planes of the first lane of a pair
+        while (__ballot(s < s1)) {
+            if (s < s1) {
+                real t1[P], d1[P], t2[P], d2[P], t3[P], d3[P];
+                bspline_rounded<real, P, false>(st.x, t1, d1, nullptr);
+                bspline_rounded<real, P, false>(st.y, t2, d2, nullptr);
+                bspline_rounded<real, P, false>(st.z, t3, d3, nullptr);
+                const int lc = unpack_loc(st.w);
+                const int lx = lc & 31, ly = (lc >> 5) & 31, lz = (lc >> 10) & 31;
+                real g1 = 0, g2 = 0, g3 = 0;
+#pragma unroll
+                for (int ixh = 0; ixh < PH; ++ixh) {
+                    const int ix = half ? PH + ixh : ixh;
+                    if (ix >= P) break;
+                    // spline weights picked with compile-time indices (registers, not scratch)
+                    const int ih = PH + ixh < P ? PH + ixh : P - 1;
+                    const real d1x = half ? d1[ih] : d1[ixh], t1x = half ? t1[ih] : t1[ixh];
+                    real s_tt = 0, s_dt = 0, s_td = 0;
+#pragma unroll
+                    for (int iy = 0; iy < P; ++iy) {
+                        const real *line = blk + ((lx + ix) * BY + (ly + iy)) * SZ + lz;
+                        real lt = 0, ld = 0;
+#pragma unroll
+                        for (int iz = 0; iz < P; ++iz) {
+                            const real w = line[iz];
+                            lt += w * t3[iz];
+                            ld += w * d3[iz];
+                        }
+                        s_tt += lt * t2[iy];
+                        s_dt += lt * d2[iy];
+                        s_td += ld * t2[iy];
+                    }
+                    g1 += s_tt * d1x;
+                    g2 += s_dt * t1x;
+                    g3 += s_td * t1x;
+                }
+                g1 += __shfl_xor(g1, 1, WAVE);
+                g2 += __shfl_xor(g2, 1, WAVE);
+                g3 += __shfl_xor(g3, 1, WAVE);
+                if (!half) {
+                    const double *es = g.escale;
+                    const real rx = (real)es[0] * g1 + (real)es[1] * g2 + (real)es[2] * g3;
+                    const real ry = (real)es[3] * g1 + (real)es[4] * g2 + (real)es[5] * g3;
+                    const real rz = (real)es[6] * g1 + (real)es[7] * g2 + (real)es[8] * g3;
+                    double c = 0.0;
+                    combine_out<real>(mode, atom, rx, ry, rz, dq, row, alpha, extra, cself, out, c);
+                    acc[0] += c;
+                }
+            }
+            s += WAVE / 2;
+            if (s < s1) {
+                st = sten[s];
+                atom = sidx[s];
+            }
+        }
     }
     if (part) {
         block_sum<1>(acc, lds);
-        if (tid == 0) part[tile] = acc[0];
+        if (threadIdx.x == 0) part[blockIdx.x] = acc[0];
     }
 }
 
@@ -626,7 +714,7 @@ __global__ __launch_bounds__(256) void k_gather_forces(int n, int nper, const do
     stencil<real, P>(pos, i, g, base, f);
     real t[3][P], dt[3][P], d2t[3][P];
 #pragma unroll
-    for (int a = 0; a < 3; ++a) bspline<real, P, true>(f[a], t[a], dt[a], d2t[a]);
+    for (int a = 0; a < 3; ++a) bspline_rounded<real, P, true>(f[a], t[a], dt[a], d2t[a]);
     const real4<real> d = dq[i];
     real e[3];
     scaled_dipole<real>(d, g, e);
