@@ -143,6 +143,22 @@ PGM_DEV double sqrt_(double x) { return sqrt(x); }
 PGM_DEV float rsqrt_(float x) { return rsqrtf(x); }
 PGM_DEV double rsqrt_(double x) { return 1.0 / sqrt(x); }
 
+// exp(-s) for 0 <= s < 88 (FP32): the product s log2(e) in two parts, so that the rounding of the
+// argument of the hardware exp2 is corrected to first order; 5 instructions and the accuracy of expf (about
+// 1.5 units in the last place) without its handling of overflow and of arguments that cannot occur here
+// (larger s underflow to 0 as they should).
+PGM_DEV float exp_neg(float s) {
+    const float L = 1.44269502f, LL = 1.92596299e-8f;  // log2(e) rounded, and the rest
+    const float t = s * L;
+    const float d = __builtin_fmaf(s, LL, __builtin_fmaf(s, L, -t));
+    const float e = __builtin_amdgcn_exp2f(-t);
+    return __builtin_fmaf(e, d * -0.693147181f, e);
+}
+PGM_DEV double exp_neg(double s) { return exp(-s); }
+// 1/sqrt of a normal number (no denormals: squared distances and radii)
+PGM_DEV float rsqrt_n(float x) { return __builtin_amdgcn_rsqf(x); }
+PGM_DEV double rsqrt_n(double x) { return 1.0 / sqrt(x); }
+
 // erfc(x) for x >= 1 from e = exp(-x^2) and ix = 1/x, which the caller has anyway (the same
 // Gaussian enters the recursion below):  erfc(x) = e h(ix^2) ix / sqrt(pi), where h(u) =
 // sqrt(pi) x exp(x^2) erfc(x) at u = 1/x^2 is written h = 1 - u R(u) with R a (4,3) rational fitted
@@ -211,11 +227,11 @@ template <typename real, int NMAX> PGM_DEV void one_B(real a, real r, real ir, r
 
 // G_n when both (a r)^2 and (b r)^2 are >= 1 (the closed-form difference only).
 template <typename real, int NMAX> PGM_DEV void pair_G_far(real a, real b, real r2, real *G) {
-    const real ir = rsqrt_(r2);
+    const real ir = rsqrt_n(r2);
     const real r = r2 * ir;
     const real ir2 = ir * ir;
     const real sa = a * a * r2, sb = b * b * r2;
-    const real ea = exp_(-sa), eb = exp_(-sb);
+    const real ea = exp_neg(sa), eb = exp_neg(sb);
     const real ca = real(TWO_OVER_SQRTPI) * a * ea;
     const real cb = real(TWO_OVER_SQRTPI) * b * eb;
     G[0] = closed_G0(a, b, r, ir, ea, eb);
@@ -254,6 +270,41 @@ template <typename real, int NMAX> PGM_DEV void pair_G(real a, real b, real r2, 
         one_B<real, NMAX>(b, r, ir, ir2, Bb);
 #pragma unroll
         for (int n = 0; n < NMAX; ++n) G[n] = Ba[n] - Bb[n];
+    }
+}
+
+// B_n of phi_a through the Boys functions F_n(s) = int_0^1 t^2n exp(-s t^2) dt, s = (a r)^2:
+// B_n = (2a/sqrt(pi)) (2a^2)^n F_n.  The highest one by its series of positive terms (Shavitt, Methods in
+// Computational Physics 2, 1963), F_m = exp(-s) sum_k (2s)^k / ((2m+1)(2m+3)...(2m+2k+1)), the others by
+// F_(n-1) = (2s F_n + exp(-s)) / (2n-1), which is stable downwards.  In FP64 24 terms leave 1.5e-10 of F_n
+// for s < 6 and 12 terms 1e-11 for s < 1.25; in FP32 18 and 8 terms leave less than its rounding.
+template <typename real, int NMAX, int TERMS> PGM_DEV void boys_B(real a, real s, real *B) {
+    const real x = real(2) * s, e = exp_neg(s);
+    real S = real(1);
+#pragma unroll
+    for (int k = TERMS; k >= 1; --k) S = (S * x) * real(1.0 / double(2 * NMAX - 1 + 2 * k)) + real(1);
+    real F[NMAX];
+    F[NMAX - 1] = e * S * real(1.0 / double(2 * NMAX - 1));
+#pragma unroll
+    for (int n = NMAX - 1; n >= 1; --n) F[n - 1] = (x * F[n] + e) * real(1.0 / double(2 * n - 1));
+    real c = real(TWO_OVER_SQRTPI) * a;
+    const real f = real(2) * a * a;
+#pragma unroll
+    for (int n = 0; n < NMAX; ++n) {
+        B[n] = c * F[n];
+        c *= f;
+    }
+}
+template <typename real, int NMAX> PGM_DEV void near_B(real a, real r2, real *B) {
+    constexpr bool wide = sizeof(real) == 8;
+    const real s = a * a * r2;
+    if (s < real(1.25)) {
+        boys_B<real, NMAX, wide ? 12 : 8>(a, s, B);
+    } else if (s < real(6)) {
+        boys_B<real, NMAX, wide ? 24 : 18>(a, s, B);
+    } else {
+        const real ir = rsqrt_n(r2);
+        closed_B<real, NMAX>(a, r2 * ir, ir, ir * ir, B);
     }
 }
 

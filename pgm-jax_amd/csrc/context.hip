@@ -102,6 +102,7 @@ struct DevBuf {
     template <typename T> T *as() const { return (T *)p; }
 };
 
+constexpr int MOL_SPLIT = 2048;         // molecules from which the record pass takes one wave each
 constexpr int ROW_FIELD_WAVES = 2048;  // two waves per SIMD (row_field_lanes)
 
 struct pgm_ctx {
@@ -785,22 +786,28 @@ static int prepare(pgm_ctx *c, const double *pos, bool defer_records = false) {
         const double beta2 = c->s.ewald_beta * c->s.ewald_beta;
         hipStream_t rs = side_records ? c->side : st;
         const bool rows_too = c->mixed && c->rc_v > c->rc_e;
+        const auto go = [&](auto k, int per_block, auto *mg, auto beta, bool rows) {
+            k<<<nblk(nmol, per_block), 256, 0, rs>>>(nmol, c->mrows.as<int>(), c->mcount_full.as<int>(), c->mcap_full, c->mcap,
+                                                     c->xr.as<double4>(), c->box, rc2, rce2, beta, c->mj.as<int>(), mg,
+                                                     c->mcount.as<int>(), rows ? c->rows.as<int>() : nullptr, c->cap,
+                                                     rows ? c->count.as<int>() : nullptr, rows ? c->count_near.as<int>() : nullptr,
+                                                     beta2);
+        };
+        // four waves per molecule where one each would leave SIMDs idle behind its rounds of 64 candidates
+        const bool split = nmol < MOL_SPLIT;
+        float *mgf = c->mg.as<float>();
+        double *mgd = c->mg.as<double>();
+        const float bf = (float)c->s.ewald_beta;
         if (rows_too)
-            k_mol_tensors<float, true><<<nblk(nmol, 4), 256, 0, rs>>>(nmol, c->mrows.as<int>(), c->mcount_full.as<int>(), c->mcap_full,
-                                                               c->mcap, c->xr.as<double4>(), c->box, rc2, rce2,
-                                                               (float)c->s.ewald_beta, c->mj.as<int>(), c->mg.as<float>(),
-                                                               c->mcount.as<int>(), c->rows.as<int>(), c->cap,
-                                                               c->count.as<int>(), c->count_near.as<int>(), beta2);
+            go(k_mol_tensors<float, true, 1>, 4, mgf, bf, true);
+        else if (c->mixed && split)
+            go(k_mol_tensors<float, false, 4>, 1, mgf, bf, false);
         else if (c->mixed)
-            k_mol_tensors<float, false><<<nblk(nmol, 4), 256, 0, rs>>>(
-                nmol, c->mrows.as<int>(), c->mcount_full.as<int>(), c->mcap_full, c->mcap, c->xr.as<double4>(), c->box,
-                rc2, rce2, (float)c->s.ewald_beta, c->mj.as<int>(), c->mg.as<float>(), c->mcount.as<int>(), nullptr, 0, nullptr,
-                nullptr, beta2);
+            go(k_mol_tensors<float, false, 1>, 4, mgf, bf, false);
+        else if (split)
+            go(k_mol_tensors<double, false, 4>, 1, mgd, c->s.ewald_beta, false);
         else
-            k_mol_tensors<double, false><<<nblk(nmol, 4), 256, 0, rs>>>(
-                nmol, c->mrows.as<int>(), c->mcount_full.as<int>(), c->mcap_full, c->mcap, c->xr.as<double4>(), c->box,
-                rc2, rce2, c->s.ewald_beta, c->mj.as<int>(), c->mg.as<double>(), c->mcount.as<int>(), nullptr, 0, nullptr, nullptr,
-                beta2);
+            go(k_mol_tensors<double, false, 1>, 4, mgd, c->s.ewald_beta, false);
         c->atom_rows_fresh = rows_too;
         if (side_records) {
             LAUNCH_CHECK();

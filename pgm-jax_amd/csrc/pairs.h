@@ -691,54 +691,143 @@ __global__ __launch_bounds__(256) void k_mol_rows(int nmol, int nmol_bead, const
 // Records of the molecule blocks, once per geometry (the molecule form of k_compact_rows +
 // k_pair_tensors): every candidate J of I with at least one atom pair inside the electrostatics
 // cutoff (r^2 < rce2; pairs beyond it hold zeros, and rce2 = rc2 without a split cutoff) is kept, in candidate
-// order, its G1 / G2 by pair_G from the FP64 minimum-image displacement rounded to real.  One wave
-// per molecule, lanes over candidates, ballot compaction.  Divergence of pair_G's series branches is
-// kept out of the common path: the closed form (both screenings with (a r)^2, (beta r)^2 >= 1) is
-// evaluated for every pair at once, the other pairs are marked and then evaluated one per lane per
-// round, and the own molecule's record (J == I, six close pairs) is computed by six lanes together.
+// order, its G1 / G2 from the FP64 minimum-image displacement.  WPM waves per molecule, one lane per
+// candidate, ballot compaction (with WPM = 4 across the waves of the workgroup, in candidate order too).
+//
+// The lattice shift is found once per molecule pair, from the atoms 0: where that displacement plus the
+// extents of the two molecules stays within half the box along every axis, every atom pair has the same
+// shift (min_image would apply none to the shifted displacement), and J is moved by it once.  A wave with
+// a candidate near half the box, or a molecule split across the box, takes every pair's own minimum
+// image (only possible in boxes little wider than two cutoffs, or with such molecules).
+//
+// The closed form (both screenings with (a r)^2, (beta r)^2 >= 1) is evaluated for all nine pairs; the
+// others (the own molecule, hydrogen bonds: a few pairs per molecule) go to a queue in LDS and are
+// evaluated at the end, one per lane, so that a wave runs the series once and not once for every near
+// pair of its busiest lane.
 //
 // With ROWS the same pass also writes the compacted atom rows of the force pass (what
 // k_compact_rows makes from the full atom rows): for atom 3I + p every 3J + k with r^2 < rc^2,
 // the near pairs (r^2 < 1.05 * 2 (R_i^2 + R_j^2) or beta^2 r^2 < 1.05, FP64) from the front of the
 // row and the others from the back, in (k, candidate) order per wave chunk; count / count_near
-// as k_compact_rows gives them.  (Used for FP32; the FP64 variant keeps its registers for the
-// tensors and leaves the atom rows to k_compact_rows.)
-// FP32: four waves per SIMD (at most 128 VGPRs, no spills), 11 % faster than the three that the
-// unbounded register allocation gives (319 against 360 us at 32k waters); five spill, and so does
-// the FP64 variant at four.
-template <typename real, bool ROWS>
+// as k_compact_rows gives them.  (Used for FP32 with WPM = 1; the FP64 variant keeps its registers for
+// the tensors and leaves the atom rows to k_compact_rows.)
+//
+// VALU bound.
+constexpr int MOL_HELD = 64;                // near pairs a wave holds back for a later round
+constexpr int MOL_QUEUE = MOL_HELD + 9 * WAVE;  // and those of one round at most
+
+template <typename real>
+PGM_DEV void mol_near_pair(int I, int J, int e, int t, const double4 *__restrict__ xr, const Box &box, double rce2, real beta, int mcap,
+                           real *__restrict__ mg) {
+    const int p = t / 3, k = t - 3 * p;
+    const double4 a = xr[3 * I + p], b = xr[3 * J + k];
+    double dx = a.x - b.x, dy = a.y - b.y, dz = a.z - b.z;
+    min_image(dx, dy, dz, box);
+    const double r2d = dx * dx + dy * dy + dz * dz;
+    real G[3] = {real(0), real(0), real(0)};
+    if (r2d < rce2) {
+        const real x = (real)dx, y = (real)dy, z = (real)dz, r2 = x * x + y * y + z * z;
+        if constexpr (sizeof(real) == 4) {
+            real A[3], B[3];
+            near_B<real, 3>((real)(1.0 / sqrt(2.0 * (a.w + b.w))), r2, A);
+            near_B<real, 3>(beta, r2, B);
+            G[1] = A[1] - B[1];
+            G[2] = A[2] - B[2];
+        } else {
+            pair_G<real, 3>(rsqrt_(real(2) * (real)(a.w + b.w)), beta, r2, G);
+        }
+    }
+    real *g = mg + mchunk(e, I, mcap);
+    g[mslot<real>(e, t)] = G[1];
+    g[mslot<real>(e, 9 + t)] = G[2];
+}
+
+template <typename real, bool ROWS, int WPM>
 __global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_mol_tensors(int nmol, const int *__restrict__ mrows, const int *__restrict__ mcount_full,
                                                      int mcap_full, int mcap, const double4 *__restrict__ xr, Box box,
                                                      double rc2, double rce2, real beta, int *__restrict__ mj, real *__restrict__ mg,
                                                      int *__restrict__ mcount, int *__restrict__ rows, int acap,
                                                      int *__restrict__ acount, int *__restrict__ acount_near, double beta2) {
-    const int lane = threadIdx.x % WAVE;
-    const int I = blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
+    static_assert(!ROWS || WPM == 1, "atom rows are compacted by one wave per molecule");
+    __shared__ int2 nearq[4][MOL_QUEUE];
+    __shared__ int wsum[4];
+    const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE;
+    const int I = WPM == 1 ? blockIdx.x * 4 + wv : blockIdx.x;
     if (I >= nmol) return;
+    int2 *queue = nearq[wv];
     const double4 a[3] = {xr[3 * I], xr[3 * I + 1], xr[3 * I + 2]};
+    // half the box less this molecule's extent from its atom 0, per axis
+    const double hx = 0.5 * box.h[0] - fmax(fabs(a[1].x - a[0].x), fabs(a[2].x - a[0].x));
+    const double hy = 0.5 * box.h[4] - fmax(fabs(a[1].y - a[0].y), fabs(a[2].y - a[0].y));
+    const double hz = 0.5 * box.h[8] - fmax(fabs(a[1].z - a[0].z), fabs(a[2].z - a[0].z));
     const int cf = min(mcount_full[I], mcap_full);
     const int *cand = mrows + (size_t)I * mcap_full;
-    int kept = 0, self_slot = -1;
+    int kept = 0, qlen = 0;
     int on[3] = {0, 0, 0}, of[3] = {0, 0, 0};  // atom rows: near / far entries so far
     const unsigned long long below = (1ull << lane) - 1ull;
-    for (int e0 = 0; e0 < cf; e0 += WAVE) {
+    for (int e0 = WPM == 1 ? 0 : WAVE * wv; e0 < cf || (WPM > 1 && e0 - WAVE * wv < cf); e0 += WAVE * WPM) {
         const int e = e0 + lane;
         bool keep = false, own = false;
         int J = 0, code = MOL_OWN_IMAGES;
         unsigned near = 0u, akeep = 0u, anear = 0u;
         real G1[9], G2[9];
-        double4 b[3];
 #pragma unroll
         for (int t = 0; t < 9; ++t) G1[t] = G2[t] = real(0);
+        double4 b[3];
 #pragma unroll
         for (int k = 0; k < 3; ++k) b[k] = make_double4(0.0, 0.0, 0.0, 0.0);
+        int n0[3] = {0, 0, 0};
+        bool one = true;  // one shift for the nine pairs
         if (e < cf) {
             J = cand[e];
             own = J == I;
 #pragma unroll
             for (int k = 0; k < 3; ++k) b[k] = xr[3 * J + k];
-            int n0[3] = {0, 0, 0};
+            double dx = a[0].x - b[0].x, dy = a[0].y - b[0].y, dz = a[0].z - b[0].z;
+            min_image_n(dx, dy, dz, box, n0);
+            one = fabs(dx) + fmax(fabs(b[1].x - b[0].x), fabs(b[2].x - b[0].x)) <= hx &&
+                  fabs(dy) + fmax(fabs(b[1].y - b[0].y), fabs(b[2].y - b[0].y)) <= hy &&
+                  fabs(dz) + fmax(fabs(b[1].z - b[0].z), fabs(b[2].z - b[0].z)) <= hz;
+        }
+        const auto pair = [&](int p, int k, double r2d) {
+            const int t = 3 * p + k;
+            if (r2d >= rc2) return;
+            if (ROWS) {
+                akeep |= 1u << t;
+                if (r2d < 1.05 * 2.0 * (a[p].w + b[k].w) || beta2 * r2d < 1.05) anear |= 1u << t;
+            }
+            if (r2d >= rce2) return;  // records hold the electrostatic pairs only
+            keep = true;
+            const real r2 = (real)r2d;
+            const real aij = rsqrt_n(real(2) * (real)(a[p].w + b[k].w));
+            if (!own && aij * aij * r2 >= real(1) && beta * beta * r2 >= real(1)) {
+                real G[3];
+                pair_G_far<real, 3>(aij, beta, r2, G);
+                G1[t] = G[1];
+                G2[t] = G[2];
+            } else {
+                near |= 1u << t;
+            }
+        };
+        const bool small = n0[0] >= -1 && n0[0] <= 1 && n0[1] >= -1 && n0[1] <= 1 && n0[2] >= -1 && n0[2] <= 1;
+        if (!__ballot(!one)) {
+            const double f0 = n0[0], f1 = n0[1], f2 = n0[2];
+            const double sx = f0 * box.h[0] + f1 * box.h[3] + f2 * box.h[6], sy = f1 * box.h[4] + f2 * box.h[7], sz = f2 * box.h[8];
+            if (e < cf) {
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    const double bx = b[k].x + sx, by = b[k].y + sy, bz = b[k].z + sz;
+#pragma unroll
+                    for (int p = 0; p < 3; ++p) {
+                        const double dx = a[p].x - bx, dy = a[p].y - by, dz = a[p].z - bz;
+                        if (!(own && p == k)) pair(p, k, dx * dx + dy * dy + dz * dz);
+                    }
+                }
+                if (!own && small) code = (n0[0] + 1) | ((n0[1] + 1) << 2) | ((n0[2] + 1) << 4);
+            }
+        } else if (e < cf) {
             bool first = true, same = true;
+            int nc[3] = {0, 0, 0};
 #pragma unroll
             for (int p = 0; p < 3; ++p)
 #pragma unroll
@@ -748,55 +837,18 @@ __global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_mol_tensors(
                     int n[3];
                     min_image_n(dx, dy, dz, box, n);
                     const double r2d = dx * dx + dy * dy + dz * dz;
-                    if (r2d >= rc2) continue;
-                    if (ROWS) {
-                        akeep |= 1u << (3 * p + k);
-                        if (r2d < 1.05 * 2.0 * (a[p].w + b[k].w) || beta2 * r2d < 1.05) anear |= 1u << (3 * p + k);
+                    if (r2d < rce2) {
+                        if (first) {
+                            nc[0] = n[0], nc[1] = n[1], nc[2] = n[2];
+                            first = false;
+                        } else if (n[0] != nc[0] || n[1] != nc[1] || n[2] != nc[2]) {
+                            same = false;
+                        }
                     }
-                    if (r2d >= rce2) continue;  // records hold the electrostatic pairs only
-                    keep = true;
-                    if (own) continue;  // the own molecule's pairs come after the compaction
-                    if (first) {
-                        n0[0] = n[0], n0[1] = n[1], n0[2] = n[2];
-                        first = false;
-                    } else if (n[0] != n0[0] || n[1] != n0[1] || n[2] != n0[2]) {
-                        same = false;
-                    }
-                    const real x = (real)dx, y = (real)dy, z = (real)dz;
-                    const real r2 = x * x + y * y + z * z;
-                    const real aij = rsqrt_(real(2) * (real)(a[p].w + b[k].w));
-                    if (aij * aij * r2 >= real(1) && beta * beta * r2 >= real(1)) {
-                        real G[3];
-                        pair_G_far<real, 3>(aij, beta, r2, G);
-                        G1[3 * p + k] = G[1];
-                        G2[3 * p + k] = G[2];
-                    } else {
-                        near |= 1u << (3 * p + k);
-                    }
+                    pair(p, k, r2d);
                 }
-            const bool small = n0[0] >= -1 && n0[0] <= 1 && n0[1] >= -1 && n0[1] <= 1 && n0[2] >= -1 && n0[2] <= 1;
-            if (!own && same && small) code = (n0[0] + 1) | ((n0[1] + 1) << 2) | ((n0[2] + 1) << 4);
-        }
-        // pairs off the closed form: one per lane per round (the series branches run on useful lanes)
-        while (__ballot(near != 0u)) {
-            if (near) {
-                const int t = __ffs(near) - 1;
-                near &= near - 1u;
-                const int p = t / 3, k = t - 3 * p;
-                const double4 ap = xr[3 * I + p], bk = xr[3 * J + k];  // reloaded (cached) rather than selected
-                double dx = ap.x - bk.x, dy = ap.y - bk.y, dz = ap.z - bk.z;
-                min_image(dx, dy, dz, box);
-                const real x = (real)dx, y = (real)dy, z = (real)dz;
-                const real aij = rsqrt_(real(2) * (real)(ap.w + bk.w));
-                real G[3];
-                pair_G<real, 3>(aij, beta, x * x + y * y + z * z, G);
-#pragma unroll
-                for (int u = 0; u < 9; ++u)
-                    if (u == t) {
-                        G1[u] = G[1];
-                        G2[u] = G[2];
-                    }
-            }
+            const bool sm = nc[0] >= -1 && nc[0] <= 1 && nc[1] >= -1 && nc[1] <= 1 && nc[2] >= -1 && nc[2] <= 1;
+            if (!own && same && sm) code = (nc[0] + 1) | ((nc[1] + 1) << 2) | ((nc[2] + 1) << 4);
         }
         if (ROWS) {  // atom rows of the force pass
 #pragma unroll
@@ -816,41 +868,48 @@ __global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_mol_tensors(
             }
         }
         const unsigned long long m = __ballot(keep);
-        const int slot_e = kept + __popcll(m & below);
-        if (keep && slot_e < mcap) {
-            mj[(size_t)I * mcap + slot_e] = (int)((unsigned)J | ((unsigned)code << 26));
-            real *g = mg + mchunk(slot_e, I, mcap);
-            if (own) {  // the diagonal (p == k) only; the six pairs follow
+        int slot0 = kept;  // first slot of this wave's records in the round
+        if (WPM > 1) {
+            __syncthreads();
+            if (lane == 0) wsum[wv] = __popcll(m);
+            __syncthreads();
 #pragma unroll
-                for (int p = 0; p < 3; ++p) g[mslot<real>(slot_e, 4 * p)] = g[mslot<real>(slot_e, 9 + 4 * p)] = real(0);
-                self_slot = slot_e;
-            } else {
-                mstore(g, slot_e, G1, G2);
+            for (int w = 0; w < 4; ++w) {
+                if (w < wv) slot0 += wsum[w];
+                kept += wsum[w];
+            }
+        } else {
+            kept += __popcll(m);
+        }
+        const int slot_e = slot0 + __popcll(m & below);
+        const bool put = keep && slot_e < mcap;
+        if (put) {
+            mj[(size_t)I * mcap + slot_e] = (int)((unsigned)J | ((unsigned)code << 26));
+            mstore(mg + mchunk(slot_e, I, mcap), slot_e, G1, G2);
+        }
+        if (!put) near = 0u;
+        if (__ballot(near != 0u)) {
+#pragma unroll
+            for (int t = 0; t < 9; ++t) {
+                const bool q = (near >> t) & 1u;
+                const unsigned long long mq = __ballot(q);
+                if (q) queue[qlen + __popcll(mq & below)] = make_int2((slot_e << 4) | t, J);
+                qlen += __popcll(mq);
             }
         }
-        kept += __popcll(m);
-    }
-    // the own molecule's record: lanes 0..5 take the pairs (0,1) (0,2) (1,0) (1,2) (2,0) (2,1)
-    const unsigned long long hs = __ballot(self_slot >= 0);
-    if (hs) {
-        const int sslot = __shfl(self_slot, (int)__ffsll((long long)hs) - 1, WAVE);
-        if (lane < 6) {
-            const int p = lane / 2, k = (lane % 2) + (lane % 2 >= p ? 1 : 0);
-            const double4 ap = xr[3 * I + p], ak = xr[3 * I + k];
-            double dx = ap.x - ak.x, dy = ap.y - ak.y, dz = ap.z - ak.z;
-            min_image(dx, dy, dz, box);
-            real G[3] = {real(0), real(0), real(0)};
-            if (dx * dx + dy * dy + dz * dz < rce2) {
-                const real x = (real)dx, y = (real)dy, z = (real)dz;
-                const real aij = rsqrt_(real(2) * (real)(ap.w + ak.w));
-                pair_G<real, 3>(aij, beta, x * x + y * y + z * z, G);
+        const bool last = e0 + WAVE * WPM >= cf + (WPM == 1 ? 0 : WAVE * wv);
+        if (qlen > MOL_HELD || (last && qlen)) {  // the queued pairs, after the stores of their records
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+            __builtin_amdgcn_wave_barrier();
+            for (int u = lane; u < qlen; u += WAVE) {
+                const int2 q = queue[u];
+                mol_near_pair<real>(I, q.y, q.x >> 4, q.x & 15, xr, box, rce2, beta, mcap, mg);
             }
-            real *g = mg + mchunk(sslot, I, mcap);
-            g[mslot<real>(sslot, 3 * p + k)] = G[1];
-            g[mslot<real>(sslot, 9 + 3 * p + k)] = G[2];
+            __builtin_amdgcn_wave_barrier();
+            qlen = 0;
         }
     }
-    if (lane == 0) mcount[I] = kept < mcap ? kept : mcap;
+    if (WPM == 1 ? lane == 0 : threadIdx.x == 0) mcount[I] = kept < mcap ? kept : mcap;
     if (ROWS && lane < 3) {
         const int o = on[lane], f = of[lane];
         const int tot = o + f < acap ? o + f : acap;
