@@ -302,10 +302,29 @@ template <typename real, int NMAX> PGM_DEV void near_B(real a, real r2, real *B)
         boys_B<real, NMAX, wide ? 12 : 8>(a, s, B);
     } else if (s < real(6)) {
         boys_B<real, NMAX, wide ? 24 : 18>(a, s, B);
-    } else {
-        const real ir = rsqrt_n(r2);
-        closed_B<real, NMAX>(a, r2 * ir, ir, ir * ir, B);
+    } else {  // FP32: at these s neither erf nor the recursion loses accuracy (FP64 sums use pair_G)
+        const float fr2 = (float)r2, ir = rsqrt_n(fr2);
+        float C[NMAX];
+        closed_B<float, NMAX>((float)a, fr2 * ir, ir, ir * ir, C);
+#pragma unroll
+        for (int n = 0; n < NMAX; ++n) B[n] = (real)C[n];
     }
+}
+
+// G_n of a pair on or near a series branch for the force passes, evaluated in FP64 and rounded once.  These
+// are the pairs of a molecule with itself and its closest neighbours (a few per atom): their kernels are
+// the largest, and a rigid molecule repeats the same distances everywhere, so that the rounding of an
+// FP32 evaluation adds up with one sign over the system (7e-8 of the energy and 1.6e-6 of the strain
+// derivative of 2,744 waters; 3e-8 and 0.9e-6 with these).
+template <int NMAX> PGM_DEV void pair_G_near(double R2sum, double b, double r2, float *G) {
+    double Ba[NMAX], Bb[NMAX];
+    near_B<double, NMAX>(1.0 / sqrt(2.0 * R2sum), r2, Ba);
+    near_B<double, NMAX>(b, r2, Bb);
+#pragma unroll
+    for (int n = 0; n < NMAX; ++n) G[n] = (float)(Ba[n] - Bb[n]);
+}
+template <int NMAX> PGM_DEV void pair_G_near(double R2sum, double b, double r2, double *G) {
+    pair_G<double, NMAX>(1.0 / sqrt(2.0 * R2sum), b, r2, G);
 }
 
 // ---------------------------------------------------------------------------- B-splines

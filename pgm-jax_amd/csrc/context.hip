@@ -1715,7 +1715,7 @@ static int energy_forces_impl(pgm_ctx *c, const double *mu, pgm_energy *energy, 
     // or on the atom rows
     const bool mol_forces = c->layout == 1 && !vir && c->rc_v <= c->rc_e;
     if (!mol_forces && !c->atom_rows_fresh) PGM_TRY(compact_atom_rows(c));
-    const int npair = mol_forces ? nblk((long long)nper * MOL_FORCE_LANES, 256)
+    const int npair = mol_forces ? nblk(nper / 3, MOL_FORCE_MOLS)
                                  : nblk((long long)nper * rowl<real>(), 256);  // pair partials per bead
     const dim3 gpair(npair, B);
     const int nconv = conv_partials(c, vir);
@@ -1739,7 +1739,7 @@ static int energy_forces_impl(pgm_ctx *c, const double *mu, pgm_energy *energy, 
         LAUNCH_CHECK();
         k_pair_forces<real, true><<<gpair, 256, 0, st>>>(
             nper, c->rows.as<int>(), c->count.as<int>(), c->count_near.as<int>(), c->cap, c->xr.as<double4>(), dq, c->box,
-            (real)c->s.ewald_beta, c->rc_e * c->rc_e, c->rc_v * c->rc_v, c->ljp.as<double4>(), c->g_el.as<double>(),
+            c->s.ewald_beta, c->rc_e * c->rc_e, c->rc_v * c->rc_v, c->ljp.as<double4>(), c->g_el.as<double>(),
             c->g_lj.as<double>(), c->rowf.as<double>(), c->pair_part.as<double>(), c->off.as<double>(),
             c->vir_pair.as<double>());
     } else {
@@ -1752,14 +1752,14 @@ static int energy_forces_impl(pgm_ctx *c, const double *mu, pgm_energy *energy, 
             ps = c->side;
         }
         if (mol_forces)
-            k_pair_forces_mol<real, MOL_FORCE_LANES><<<gpair, 256, 0, ps>>>(
+            k_pair_forces_mol<real><<<gpair, 3 * WAVE, 0, ps>>>(
                 nper, c->mcap, c->mj.as<int>(), c->mg.as<real>(), c->mcount.as<int>(), c->xr.as<double4>(), dq, c->box,
-                (real)c->s.ewald_beta, c->rc_e * c->rc_e, c->rc_v * c->rc_v, c->rh.as<double>(), c->se.as<double>(),
+                c->s.ewald_beta, c->rc_e * c->rc_e, c->rc_v * c->rc_v, c->ljp.as<double4>(),
                 c->g_el.as<double>(), c->g_lj.as<double>(), c->rowf.as<double>(), c->pair_part.as<double>(), ext);
         else
             k_pair_forces<real, false><<<gpair, 256, 0, ps>>>(
                 nper, c->rows.as<int>(), c->count.as<int>(), c->count_near.as<int>(), c->cap, c->xr.as<double4>(), dq, c->box,
-                (real)c->s.ewald_beta, c->rc_e * c->rc_e, c->rc_v * c->rc_v, c->ljp.as<double4>(), c->g_el.as<double>(),
+                c->s.ewald_beta, c->rc_e * c->rc_e, c->rc_v * c->rc_v, c->ljp.as<double4>(), c->g_el.as<double>(),
                 c->g_lj.as<double>(), c->rowf.as<double>(), c->pair_part.as<double>(), nullptr, nullptr, ext);
         if (!c->ewald) HIP_TRY(hipEventRecord(c->ev_join, c->side));
     }

@@ -416,16 +416,16 @@ __global__ __launch_bounds__(256) void k_row_field(int n, int nper, const int *_
 // (each pair counted in both rows: the caller halves them).  With VIRIAL, also the per-block sums
 // of (KE de/dx + de_LJ/dx) (x) X, X = x - o_i + o_k with o the offsets of the atoms from their
 // molecules' centres of mass: the pair part of the molecular strain derivative (again twice).
+#define PAIR_NEAR pair_G_near<4>(a.w + b.w, beta64, r2d, G);
+#define PAIR_FAR pair_G_far<real, 4>(rsqrt_n(real(2) * (real)(a.w + b.w)), beta, (real)r2d, G);
 #define PAIR_FORCE_ENTRY(GFUN) \
             const double4 b = xr[j]; \
             double dx = a.x - b.x, dy = a.y - b.y, dz = a.z - b.z; \
             min_image(dx, dy, dz, box); \
             const real x = (real)dx, y = (real)dy, z = (real)dz; \
-            const real r2 = x * x + y * y + z * z; \
             const double r2d = dx * dx + dy * dy + dz * dz; \
-            const real aij = rsqrt_(real(2) * (real)(a.w + b.w)); \
             real G[4] = {real(0), real(0), real(0), real(0)}; \
-            if (r2d < rce2) GFUN<real, 4>(aij, beta, r2, G); \
+            if (r2d < rce2) { GFUN } \
             const real4<real> dk = dq[j]; \
             const real qk = dk.w; \
             const real dix = di.x * x + di.y * y + di.z * z; \
@@ -475,13 +475,14 @@ template <typename real, bool VIRIAL>
 __global__ __launch_bounds__(256) void k_pair_forces(int nper, const int *__restrict__ rows, const int *__restrict__ count,
                                                      const int *__restrict__ count_near, int cap,
                                                      const double4 *__restrict__ xr, const real4<real> *__restrict__ dq, Box box,
-                                                     real beta, double rce2, double rcv2, const double4 *__restrict__ ljp,
+                                                     double beta64, double rce2, double rcv2, const double4 *__restrict__ ljp,
                                                      double *__restrict__ g_el,
                                                      double *__restrict__ g_lj, double *__restrict__ rowf,
                                                      double *__restrict__ epart, const double *__restrict__ off,
                                                      double *__restrict__ wpart, Ext3 ext = {}) {
     __shared__ double lds[9 * 16];
     constexpr int RL_ = rowl<real>();
+    const real beta = (real)beta64;
     const int lane = threadIdx.x % RL_;
     const int li = blockIdx.x * (blockDim.x / RL_) + threadIdx.x / RL_;
     const int i = blockIdx.y * nper + li;
@@ -507,11 +508,11 @@ __global__ __launch_bounds__(256) void k_pair_forces(int nper, const int *__rest
         const int cn = count_near[i];
         for (int e = lane; e < cn; e += RL_) {
             const int j = row[e];
-            PAIR_FORCE_ENTRY(pair_G)
+            PAIR_FORCE_ENTRY(PAIR_NEAR)
         }
         for (int e = cap - (c - cn) + lane; e < cap; e += RL_) {
             const int j = row[e];
-            PAIR_FORCE_ENTRY(pair_G_far)
+            PAIR_FORCE_ENTRY(PAIR_FAR)
         }
         gx = group_sum<RL_>(gx);
         gy = group_sum<RL_>(gy);
@@ -550,8 +551,8 @@ __global__ __launch_bounds__(256) void k_pair_forces(int nper, const int *__rest
 
 // ---------------------------------------------------------------------------- molecule-blocked field rows
 // For systems of 3-site molecules (atoms 3I, 3I+1, 3I+2) the CG row field runs on molecule pairs:
-// record (I, J) holds the 9 atom pairs (p of I, k of J) as G1[3p+k], G2[3p+k] (zero beyond the
-// cutoff and for p == k when J == I), so one lane fetches J's three positions and dipoles once for
+// record (I, J) holds the 9 atom pairs (p of I, k of J), real 6p + k = G1 and 6p + 3 + k = G2 (zero beyond
+// the cutoff and for p == k when J == I), so one lane fetches J's three positions and dipoles once for
 // nine pair terms instead of one gather per pair.  The record's word (mj[I mcap + e]) is
 // J | code << 26: code = the lattice shifts (n_a + 1 in two bits per axis) shared by every pair
 // within the cutoff, or MOL_OWN_IMAGES when they differ (the pairs then take min_image each).
@@ -562,7 +563,7 @@ __global__ __launch_bounds__(256) void k_pair_forces(int nper, const int *__rest
 // segments.  One 72-byte record per lane in a row made every load instruction of a wave touch 36
 // cache lines instead of 8.  The layout does not depend on how many lanes share a molecule.
 constexpr int MOL_OWN_IMAGES = 63;
-constexpr int MOL_REC = 18;  // reals per record: G1 of the 9 pairs, then G2
+constexpr int MOL_REC = 18;  // reals per record: for each atom of I, G1 and G2 of its three pairs
 constexpr int MCH = 16;      // records per chunk
 // First real of the chunk of record e of molecule I (mcap a multiple of MCH).
 PGM_DEV size_t mchunk(int e, int I, int mcap) { return ((size_t)I * (mcap / MCH) + e / MCH) * (size_t)(MCH * MOL_REC); }
@@ -595,23 +596,43 @@ PGM_DEV void mload(const double *__restrict__ g, int e, double (&G)[MOL_REC]) {
 PGM_DEV void mstore(float *__restrict__ g, int e, const float (&A)[9], const float (&B)[9]) {
     const int s = e % MCH;
     float4 *q = reinterpret_cast<float4 *>(g) + s;
-    q[0] = make_float4(A[0], A[1], A[2], A[3]);
-    q[MCH] = make_float4(A[4], A[5], A[6], A[7]);
-    q[2 * MCH] = make_float4(A[8], B[0], B[1], B[2]);
-    q[3 * MCH] = make_float4(B[3], B[4], B[5], B[6]);
+    q[0] = make_float4(A[0], A[1], A[2], B[0]);
+    q[MCH] = make_float4(B[1], B[2], A[3], A[4]);
+    q[2 * MCH] = make_float4(A[5], B[3], B[4], B[5]);
+    q[3 * MCH] = make_float4(A[6], A[7], A[8], B[6]);
     reinterpret_cast<float2 *>(g + 16 * MCH)[s] = make_float2(B[7], B[8]);
 }
 PGM_DEV void mstore(double *__restrict__ g, int e, const double (&A)[9], const double (&B)[9]) {
     double2 *q = reinterpret_cast<double2 *>(g) + e % MCH;
-    q[0] = make_double2(A[0], A[1]);
-    q[MCH] = make_double2(A[2], A[3]);
-    q[2 * MCH] = make_double2(A[4], A[5]);
-    q[3 * MCH] = make_double2(A[6], A[7]);
-    q[4 * MCH] = make_double2(A[8], B[0]);
-    q[5 * MCH] = make_double2(B[1], B[2]);
-    q[6 * MCH] = make_double2(B[3], B[4]);
-    q[7 * MCH] = make_double2(B[5], B[6]);
-    q[8 * MCH] = make_double2(B[7], B[8]);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+        q[(3 * p) * MCH] = make_double2(A[3 * p], A[3 * p + 1]);
+        q[(3 * p + 1) * MCH] = make_double2(A[3 * p + 2], B[3 * p]);
+        q[(3 * p + 2) * MCH] = make_double2(B[3 * p + 1], B[3 * p + 2]);
+    }
+}
+// G1 and G2 of atom p's three pairs of record e (p the same for the whole wave).
+PGM_DEV void mload_atom(const float *__restrict__ g, int e, int p, float (&G1)[3], float (&G2)[3]) {
+    const int s = e % MCH;
+    const float4 *q = reinterpret_cast<const float4 *>(g) + s;
+    if (p == 0) {
+        const float4 a = q[0];
+        const float2 b = *reinterpret_cast<const float2 *>(q + MCH);
+        G1[0] = a.x, G1[1] = a.y, G1[2] = a.z, G2[0] = a.w, G2[1] = b.x, G2[2] = b.y;
+    } else if (p == 1) {
+        const float2 a = *(reinterpret_cast<const float2 *>(q + MCH) + 1);
+        const float4 b = q[2 * MCH];
+        G1[0] = a.x, G1[1] = a.y, G1[2] = b.x, G2[0] = b.y, G2[1] = b.z, G2[2] = b.w;
+    } else {
+        const float4 a = q[3 * MCH];
+        const float2 b = reinterpret_cast<const float2 *>(g + 16 * MCH)[s];
+        G1[0] = a.x, G1[1] = a.y, G1[2] = a.z, G2[0] = a.w, G2[1] = b.x, G2[2] = b.y;
+    }
+}
+PGM_DEV void mload_atom(const double *__restrict__ g, int e, int p, double (&G1)[3], double (&G2)[3]) {
+    const double2 *q = reinterpret_cast<const double2 *>(g) + e % MCH + 3 * p * MCH;
+    const double2 a = q[0], b = q[MCH], c = q[2 * MCH];
+    G1[0] = a.x, G1[1] = a.y, G1[2] = b.x, G2[0] = b.y, G2[1] = c.x, G2[2] = c.y;
 }
 
 // Candidate partner molecules of molecule I: the molecules of the atoms in the full (cutoff + skin)
@@ -738,8 +759,8 @@ PGM_DEV void mol_near_pair(int I, int J, int e, int t, const double4 *__restrict
         }
     }
     real *g = mg + mchunk(e, I, mcap);
-    g[mslot<real>(e, t)] = G[1];
-    g[mslot<real>(e, 9 + t)] = G[2];
+    g[mslot<real>(e, 6 * p + k)] = G[1];
+    g[mslot<real>(e, 6 * p + 3 + k)] = G[2];
 }
 
 template <typename real, bool ROWS, int WPM>
@@ -965,7 +986,7 @@ __global__ __launch_bounds__(256) void k_row_field_mol(int nmol, int nmol_bead, 
                 double dx = a[p].x - b[k].x, dy = a[p].y - b[k].y, dz = a[p].z - b[k].z;
                 if (own) min_image(dx, dy, dz, box);
                 const real x = (real)dx, y = (real)dy, z = (real)dz;
-                const real g1 = G[3 * p + k], g2 = G[9 + 3 * p + k];
+                const real g1 = G[6 * p + k], g2 = G[6 * p + 3 + k];
                 const real dkx = d[k].x * x + d[k].y * y + d[k].z * z;
                 real cf = -g2 * dkx;
                 if (WITHQ) cf -= d[k].w * g1;
@@ -997,17 +1018,19 @@ __global__ __launch_bounds__(256) void k_row_field_mol(int nmol, int nmol_bead, 
 // The force pass of k_pair_forces (the same per-atom sums g_el, g_lj, rowf and per-block energy
 // partials, each pair again counted from both sides) on the molecule-block records, for 3-site
 // molecules when the van der Waals cutoff does not exceed the electrostatic one (every LJ pair then
-// lies in a record) and no strain derivative is asked for.  FL lanes per atom i = 3I + p walk the
-// records of its molecule I and take the three pairs (p, k) of each: J's positions, dipoles, charges
-// and LJ parameters are the same loads for the three atoms of I (one cache line for the lanes of
-// a wave), and the record's G1, G2 are reused.  On the closed-form branch ((a r)^2, (b r)^2 >= 1)
-// the other two radial functions follow from them and the two Gaussians c_a = 2a/sqrt(pi)
-// exp(-a^2 r^2), c_b likewise: G0 = r^2 G1 + (c_a - c_b) and G3 = (5 G2 - ((2a^2)^2 c_a -
+// lies in a record) and no strain derivative is asked for.  A workgroup takes MOL_FORCE_MOLS molecules, one
+// wave for each of their three atoms p, MOL_FORCE_LANES lanes per molecule: with p the same over a wave a
+// record's six reals of the atom are two coalesced loads, and the waves of the hydrogens (no LJ) never enter
+// the LJ branch.  The partners' atoms go through LDS, wave k fetching atom k of the round's 64 partners (one
+// round ahead) for all three: one lane per (atom, record) fetching them itself was bound by the gathers, 576
+// address cycles per 64 of them (400 us at 32,768 waters).  On the closed-form
+// branch ((a r)^2, (b r)^2 >= 1) the other two radial functions follow from G1, G2 and the two Gaussians
+// c_a = 2a/sqrt(pi) exp(-a^2 r^2), c_b likewise: G0 = r^2 G1 + (c_a - c_b) and G3 = (5 G2 - ((2a^2)^2 c_a -
 // (2b^2)^2 c_b)) / r^2, the recursion B_n = ((2n-1) B_(n-1) - (2a^2)^(n-1) c) / r^2 of the closed
 // form read down and up (no erfc).  Pairs off it (a few per atom: its own molecule, hydrogen bonds)
-// are queued per lane in LDS and take pair_G (series) after the record loop, one per lane per round,
-// so that the wave runs the series branch a few times per atom and not in most record rounds.  The
-// terms of a record are summed in `real`, then added to FP64 sums.  Grid (blocks per bead, beads).
+// are queued per atom in LDS and evaluated after the record loop over the molecule's lanes, in FP64 (see
+// pair_G_near).  The terms of a record are summed in `real`, then added to FP64 sums.  Grid (blocks per
+// bead, beads).  VALU bound.
 #define MOL_FORCE_TERMS(G0_, G1_, G2_, G3_)                                                            \
     {                                                                                                  \
         const real dix = di.x * x + di.y * y + di.z * z;                                               \
@@ -1028,99 +1051,114 @@ __global__ __launch_bounds__(256) void k_row_field_mol(int nmol, int nmol_bead, 
     }
 
 constexpr int MOL_FORCE_LANES = 8;
-constexpr int MOL_NEAR_QUEUE = 8;  // queued series pairs per lane (more are evaluated at once)
-// Launched with 256 threads per block (the LDS queue has 256 columns).  FP32: at most 128 VGPRs
-// (four waves per SIMD); FP64 unbounded.
-template <typename real, int FL>
-__global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_pair_forces_mol(int nper, int mcap, const int *__restrict__ mj,
+constexpr int MOL_FORCE_MOLS = WAVE / MOL_FORCE_LANES;  // molecules per workgroup of three waves
+constexpr int MOL_NEAR_QUEUE = 64;  // queued series pairs per molecule and atom: drained above 64 - 3 MOL_FORCE_LANES
+template <typename real>
+__global__ __launch_bounds__(3 * WAVE, sizeof(real) == 4 ? 3 : 1) void k_pair_forces_mol(int nper, int mcap, const int *__restrict__ mj,
                                                          const real *__restrict__ mg, const int *__restrict__ mcount,
                                                          const double4 *__restrict__ xr, const real4<real> *__restrict__ dq,
-                                                         Box box, real beta, double rce2, double rcv2,
-                                                         const double *__restrict__ rh, const double *__restrict__ se,
-                                                         double *__restrict__ g_el, double *__restrict__ g_lj,
-                                                         double *__restrict__ rowf, double *__restrict__ epart, Ext3 ext = {}) {
+                                                         Box box, double beta64, double rce2, double rcv2,
+                                                         const double4 *__restrict__ ljp, double *__restrict__ g_el,
+                                                         double *__restrict__ g_lj, double *__restrict__ rowf,
+                                                         double *__restrict__ epart, Ext3 ext = {}) {
+    constexpr int FL = MOL_FORCE_LANES;
     __shared__ double lds[2 * 16];
-    __shared__ int nq[MOL_NEAR_QUEUE * 256];  // (record index << 2 | k) of the lane's series pairs
-    const int lane = threadIdx.x % FL;
-    const int li = blockIdx.x * (blockDim.x / FL) + threadIdx.x / FL;
-    const int i = blockIdx.y * nper + li;
+    __shared__ int nq[3 * MOL_FORCE_MOLS][MOL_NEAR_QUEUE];  // (record index << 2 | k) of the series pairs of an atom
+    __shared__ double2 s_xy[2][3][WAVE], s_zr[2][3][WAVE], s_lj[2][3][WAVE];  // partner atoms, shifted; (rmin/2, sqrt eps)
+    __shared__ real4<real> s_d[2][3][WAVE];
+    const int lane = threadIdx.x % FL, wl = threadIdx.x % WAVE;
+    const int p = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int lm = blockIdx.x * MOL_FORCE_MOLS + wl / FL;  // molecule of the bead
+    const bool in = 3 * lm < nper;
+    const int I = blockIdx.y * (nper / 3) + (in ? lm : 0), i = 3 * I + p;
     const int pb = blockIdx.y * gridDim.x + blockIdx.x;
-    int *queue = nq + threadIdx.x;  // entry u at queue[256 u]
-    double esum[2] = {0.0, 0.0};
-    if (li < nper) {
-        const int I = i / 3, p = i - 3 * I;
-        const double4 a = xr[i];
-        const real4<real> di = dq[i];
-        const real qi = di.w;
-        const double rhi = rh[i], sei = se[i];
-        const real fb = real(2) * beta * beta;
-        double gx = 0, gy = 0, gz = 0, lx = 0, ly = 0, lz = 0, fx = 0, fy = 0, fz = 0, ee = 0, el = 0;
-        const int c = mcount[I];
-        int qlen = 0;
-        // the pair (p, k) of record e on the series branch
-        auto near_pair = [&](int e, int k, real &pe, real &pg0, real &pg1, real &pg2, real &pf0, real &pf1, real &pf2) {
-            const unsigned word = (unsigned)mj[(size_t)I * mcap + e];
-            const int J = (int)(word & ((1u << 26) - 1u)), code = (int)(word >> 26);
-            const int n[3] = {(code & 3) - 1, ((code >> 2) & 3) - 1, ((code >> 4) & 3) - 1};
-            const double4 b = xr[3 * J + k];
-            const real4<real> dk = dq[3 * J + k];
-            double dx = a.x - b.x, dy = a.y - b.y, dz = a.z - b.z;
-            if (code == MOL_OWN_IMAGES)
-                min_image(dx, dy, dz, box);
-            else
-                apply_shift(dx, dy, dz, box, n);
-            const real x = (real)dx, y = (real)dy, z = (real)dz;
-            const real aij = rsqrt_(real(2) * (real)(a.w + b.w));
-            real G[4];
-            pair_G<real, 4>(aij, beta, x * x + y * y + z * z, G);
-            MOL_FORCE_TERMS(G[0], G[1], G[2], G[3])
-        };
-        for (int e = lane; e < c; e += FL) {
-            const unsigned word = (unsigned)mj[(size_t)I * mcap + e];
-            const int J = (int)(word & ((1u << 26) - 1u)), code = (int)(word >> 26);
-            const bool own = J == I;
-            const real *gr = mg + mchunk(e, I, mcap);
-            real G1[3], G2[3];
+    int *queue = nq[threadIdx.x / FL];
+    const double4 a = xr[i];
+    const real4<real> di = dq[i];
+    const real qi = di.w;
+    const double rhi = ljp[i].x, sei = ljp[i].y;
+    const real beta = (real)beta64, fb = real(2) * beta * beta;
+    double gx = 0, gy = 0, gz = 0, lx = 0, ly = 0, lz = 0, fx = 0, fy = 0, fz = 0, ee = 0, el = 0;
+    const int c = in ? mcount[I] : 0;
+    int cmax = c;  // the same for the three waves
 #pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                G1[k] = gr[mslot<real>(e, 3 * p + k)];
-                G2[k] = gr[mslot<real>(e, 9 + 3 * p + k)];
-            }
-            const int n[3] = {(code & 3) - 1, ((code >> 2) & 3) - 1, ((code >> 4) & 3) - 1};
+    for (int o = WAVE / 2; o >= FL; o >>= 1) cmax = max(cmax, __shfl_xor(cmax, o, WAVE));
+    const int *words = mj + (size_t)I * mcap;
+    int qlen = 0;
+    // the lattice shift of a record's word, 0 where the pairs take their own images (returns whether)
+    const auto shift = [&](unsigned word, double &sx, double &sy, double &sz) {
+        const int code = (int)(word >> 26);
+        const bool own = code == MOL_OWN_IMAGES;
+        const double n0 = own ? 0.0 : (double)((code & 3) - 1), n1 = own ? 0.0 : (double)(((code >> 2) & 3) - 1),
+                     n2 = own ? 0.0 : (double)(((code >> 4) & 3) - 1);
+        sx = n0 * box.h[0] + n1 * box.h[3] + n2 * box.h[6];
+        sy = n1 * box.h[4] + n2 * box.h[7];
+        sz = n2 * box.h[8];
+        return own;
+    };
+    unsigned word = 0u;
+    const auto stage = [&](int buf, unsigned w) {  // atom p of the partner of word w
+        const int j = 3 * (int)(w & ((1u << 26) - 1u)) + p;
+        const double4 b = xr[j];
+        const real4<real> d = dq[j];
+        const double2 l = *reinterpret_cast<const double2 *>(ljp + j);
+        double sx, sy, sz;
+        shift(w, sx, sy, sz);
+        s_xy[buf][p][wl] = make_double2(b.x + sx, b.y + sy);
+        s_zr[buf][p][wl] = make_double2(b.z + sz, b.w);
+        s_lj[buf][p][wl] = l;
+        s_d[buf][p][wl] = d;
+    };
+    if (lane < c) {
+        word = (unsigned)words[lane];
+        stage(0, word);
+    }
+    for (int e0 = 0, buf = 0; e0 < cmax; e0 += FL, buf ^= 1) {
+        const int e = e0 + lane;
+        __syncthreads();  // this round's partners are in; the other buffer's readers are done
+        unsigned next = 0u;
+        if (e + FL < c) {
+            next = (unsigned)words[e + FL];
+            stage(buf ^ 1, next);
+        }
+        unsigned nearm = 0u;
+        if (e < c) {
+            const bool own = (int)(word & ((1u << 26) - 1u)) == I, images = (int)(word >> 26) == MOL_OWN_IMAGES;
+            real G1[3], G2[3];
+            mload_atom(mg + mchunk(e, I, mcap), e, p, G1, G2);
             real pg0 = 0, pg1 = 0, pg2 = 0, pf0 = 0, pf1 = 0, pf2 = 0, pe = 0;
-            unsigned nearm = 0u;
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
                 if (own && k == p) continue;
-                const double4 b = xr[3 * J + k];
-                const real4<real> dk = dq[3 * J + k];
-                double dx = a.x - b.x, dy = a.y - b.y, dz = a.z - b.z;
-                if (code == MOL_OWN_IMAGES)
-                    min_image(dx, dy, dz, box);
-                else
-                    apply_shift(dx, dy, dz, box, n);
+                const double2 bxy = s_xy[buf][k][wl], bzr = s_zr[buf][k][wl];
+                const real4<real> dk = s_d[buf][k][wl];
+                double dx = a.x - bxy.x, dy = a.y - bxy.y, dz = a.z - bzr.x;
+                if (images) min_image(dx, dy, dz, box);
                 const double r2d = dx * dx + dy * dy + dz * dz;
-                const double eps = sei * se[3 * J + k];
-                if (!own && eps != 0.0 && r2d < rcv2) {  // LJ, FP64 as in k_pair_forces
-                    const double rmin = rhi + rh[3 * J + k];
-                    const double ir2 = 1.0 / r2d;
-                    const double s2 = rmin * rmin * ir2;
-                    const double s6 = s2 * s2 * s2;
-                    el += eps * (s6 * s6 - 2.0 * s6);
-                    const double dl = eps * 12.0 * (s6 - s6 * s6) * ir2;
-                    lx += dl * dx;
-                    ly += dl * dy;
-                    lz += dl * dz;
+                if (sei != 0.0) {  // LJ, FP64 as in k_pair_forces
+                    const double2 lj = s_lj[buf][k][wl];
+                    const double eps = sei * lj.y;
+                    if (!own && eps != 0.0 && r2d < rcv2) {
+                        const double rmin = rhi + lj.x;
+                        const double ir2 = 1.0 / r2d;
+                        const double s2 = rmin * rmin * ir2;
+                        const double s6 = s2 * s2 * s2;
+                        el += eps * (s6 * s6 - 2.0 * s6);
+                        const double dl = eps * 12.0 * (s6 - s6 * s6) * ir2;
+                        lx += dl * dx;
+                        ly += dl * dy;
+                        lz += dl * dz;
+                    }
                 }
                 if (r2d >= rce2) continue;
                 const real x = (real)dx, y = (real)dy, z = (real)dz;
-                const real r2 = x * x + y * y + z * z;
-                const real aij = rsqrt_(real(2) * (real)(a.w + b.w));
+                const real r2 = (real)r2d;
+                const real aij = rsqrt_n(real(2) * (real)(a.w + bzr.y));
                 const real sa = aij * aij * r2, sb = beta * beta * r2;
                 if (sa >= real(1) && sb >= real(1)) {
-                    const real ir = rsqrt_(r2), ir2 = ir * ir;
-                    const real ca = real(TWO_OVER_SQRTPI) * aij * exp_(-sa);
-                    const real cb = real(TWO_OVER_SQRTPI) * beta * exp_(-sb);
+                    const real ir = rsqrt_n(r2), ir2 = ir * ir;
+                    const real ca = real(TWO_OVER_SQRTPI) * aij * exp_neg(sa);
+                    const real cb = real(TWO_OVER_SQRTPI) * beta * exp_neg(sb);
                     const real fa = real(2) * aij * aij;
                     const real g1 = G1[k], g2 = G2[k];
                     const real g0 = r2 * g1 + (ca - cb);
@@ -1130,14 +1168,6 @@ __global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_pair_forces_
                     nearm |= 1u << k;
                 }
             }
-            while (nearm) {  // queue the series pairs (evaluate at once when the queue is full)
-                const int k = __ffs(nearm) - 1;
-                nearm &= nearm - 1u;
-                if (qlen < MOL_NEAR_QUEUE)
-                    queue[256 * qlen++] = (e << 2) | k;
-                else
-                    near_pair(e, k, pe, pg0, pg1, pg2, pf0, pf1, pf2);
-            }
             gx += (double)pg0;
             gy += (double)pg1;
             gz += (double)pg2;
@@ -1146,11 +1176,35 @@ __global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_pair_forces_
             fz += (double)pf2;
             ee += (double)pe;
         }
-        for (int u = 0; __ballot(u < qlen); ++u) {  // the queued series pairs, one per lane per round
+        word = next;
+        if (__ballot(nearm != 0u)) {  // queue the series pairs with those of the molecule's other lanes
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const bool q = (nearm >> k) & 1u;
+                const unsigned g = (unsigned)(__ballot(q) >> (wl - lane)) & ((1u << FL) - 1u);
+                if (q) queue[qlen + __popc(g & ((1u << lane) - 1u))] = (e << 2) | k;
+                qlen += __popc(g);
+            }
+        }
+        if (e0 + FL < cmax && !__ballot(qlen > MOL_NEAR_QUEUE - 3 * FL)) continue;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        for (int u = lane; __ballot(u < qlen); u += FL) {  // the queued series pairs, over the molecule's lanes
             if (u < qlen) {
-                const int v = queue[256 * u];
+                const int v = queue[u], k = v & 3;
+                const unsigned wn = (unsigned)words[v >> 2];
+                const int j = 3 * (int)(wn & ((1u << 26) - 1u)) + k;
+                const double4 b = xr[j];
+                const real4<real> dk = dq[j];
+                double sx, sy, sz;
+                const bool im = shift(wn, sx, sy, sz);
+                double dx = a.x - (b.x + sx), dy = a.y - (b.y + sy), dz = a.z - (b.z + sz);
+                if (im) min_image(dx, dy, dz, box);
+                const real x = (real)dx, y = (real)dy, z = (real)dz;
+                real G[4];
+                pair_G_near<4>(a.w + b.w, beta64, dx * dx + dy * dy + dz * dz, G);
                 real pg0 = 0, pg1 = 0, pg2 = 0, pf0 = 0, pf1 = 0, pf2 = 0, pe = 0;
-                near_pair(v >> 2, v & 3, pe, pg0, pg1, pg2, pf0, pf1, pf2);
+                MOL_FORCE_TERMS(G[0], G[1], G[2], G[3])
                 gx += (double)pg0;
                 gy += (double)pg1;
                 gz += (double)pg2;
@@ -1160,29 +1214,30 @@ __global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_pair_forces_
                 ee += (double)pe;
             }
         }
-        gx = group_sum<FL>(gx);
-        gy = group_sum<FL>(gy);
-        gz = group_sum<FL>(gz);
-        lx = group_sum<FL>(lx);
-        ly = group_sum<FL>(ly);
-        lz = group_sum<FL>(lz);
-        fx = group_sum<FL>(fx);
-        fy = group_sum<FL>(fy);
-        fz = group_sum<FL>(fz);
-        if (lane == 0) {
-            g_el[3 * i] = gx;
-            g_el[3 * i + 1] = gy;
-            g_el[3 * i + 2] = gz;
-            g_lj[3 * i] = lx;
-            g_lj[3 * i + 1] = ly;
-            g_lj[3 * i + 2] = lz;
-            rowf[3 * i] = fx - ext.x;  // a uniform external field: its dU/dd is -ext
-            rowf[3 * i + 1] = fy - ext.y;
-            rowf[3 * i + 2] = fz - ext.z;
-        }
-        esum[0] = ee;
-        esum[1] = el;
+        __builtin_amdgcn_wave_barrier();
+        qlen = 0;
     }
+    gx = group_sum<FL>(gx);
+    gy = group_sum<FL>(gy);
+    gz = group_sum<FL>(gz);
+    lx = group_sum<FL>(lx);
+    ly = group_sum<FL>(ly);
+    lz = group_sum<FL>(lz);
+    fx = group_sum<FL>(fx);
+    fy = group_sum<FL>(fy);
+    fz = group_sum<FL>(fz);
+    if (in && lane == 0) {
+        g_el[3 * i] = gx;
+        g_el[3 * i + 1] = gy;
+        g_el[3 * i + 2] = gz;
+        g_lj[3 * i] = lx;
+        g_lj[3 * i + 1] = ly;
+        g_lj[3 * i + 2] = lz;
+        rowf[3 * i] = fx - ext.x;  // a uniform external field: its dU/dd is -ext
+        rowf[3 * i + 1] = fy - ext.y;
+        rowf[3 * i + 2] = fz - ext.z;
+    }
+    double esum[2] = {ee, el};
     block_sum<2>(esum, lds);
     if (threadIdx.x == 0) {
         epart[2 * pb] = esum[0];
