@@ -176,9 +176,9 @@ struct pgm_ctx {
     DevBuf grid, cgrid, Gc, fft_work;
     rocfft_plan fwd = nullptr, bwd = nullptr;
     rocfft_execution_info info = nullptr;
-    // fused transform of the CG field evaluations (fft.h): available for power-of-two grids with
+    // fused transform of the CG field evaluations (fft.h): available for grids of 2^k {1, 3, 5, 15} points per axis with
     // tiled spreading; pme_fused selects it over the library plans
-    bool fused_ok = false, pme_fused = false;
+    bool fused_ok = false, pme_fused = false, pfft_odd = false;  // pfft_odd: an axis has a factor 3 or 5
     // where a CG field evaluation forks the row field onto the side stream: 0 before the spread,
     // 1 after the spread, 2 after the forward planes, 3 before the spread with the forward planes
     // waiting for it (2 and 3: fused transform only), 4 no side stream; set from the size at creation
@@ -584,15 +584,17 @@ static int make_plans(pgm_ctx *c) {
     return PGM_OK;
 }
 
-// Fused transform of the CG field evaluations (fft.h): every grid axis a power of two in 8..256,
+// Fused transform of the CG field evaluations (fft.h): every grid axis 2^k {1, 3, 5, 15} in 8..256,
 // the plane of K2 (K3/2 + 1) complex values within 160 KB of LDS, no Ewald sum.  Twiddles
 // W_N^t = exp(-2 pi i t / N) for N = K3/2, K3, K2, K1 in FP64, rounded to the context's precision.
 template <typename real> static int fused_lds(pgm_ctx *c) {
     const int plane = (int)pfft_plane_lds<real>(c->pfg), xc = (int)pfft_xconv_lds<real>(c->pfg);
-    HIP_TRY(hipFuncSetAttribute((const void *)k_pme_fwd_plane<real>, hipFuncAttributeMaxDynamicSharedMemorySize, plane));
-    HIP_TRY(hipFuncSetAttribute((const void *)k_pme_bwd_plane<real>, hipFuncAttributeMaxDynamicSharedMemorySize, plane));
-    HIP_TRY(hipFuncSetAttribute((const void *)k_pme_x_conv<real>, hipFuncAttributeMaxDynamicSharedMemorySize, xc));
-    HIP_TRY(hipFuncSetAttribute((const void *)k_pme_x_conv<real, true>, hipFuncAttributeMaxDynamicSharedMemorySize, xc));
+    for (const void *k : {(const void *)k_pme_fwd_plane<real, false>, (const void *)k_pme_fwd_plane<real, true>,
+                          (const void *)k_pme_bwd_plane<real, false>, (const void *)k_pme_bwd_plane<real, true>})
+        HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, plane));
+    for (const void *k : {(const void *)k_pme_x_conv<real, false>, (const void *)k_pme_x_conv<real, true>,
+                          (const void *)k_pme_x_conv<real, false, true>, (const void *)k_pme_x_conv<real, true, true>})
+        HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, xc));
     std::vector<real> tw;
     int *offs[4] = {&c->pfg.twM, &c->pfg.twK3, &c->pfg.twK2, &c->pfg.twK1};
     const int lens[4] = {c->pfg.M, c->pfg.K3, c->pfg.K2, c->pfg.K1};
@@ -611,10 +613,15 @@ template <typename real> static int fused_lds(pgm_ctx *c) {
 static int setup_fused(pgm_ctx *c) {
     c->fused_ok = false;
     c->pme_fused = false;
+    c->pfft_odd = false;
     if (c->ewald) return PGM_OK;
     const int *K = c->s.grid;
-    for (int a = 0; a < 3; ++a)
-        if (K[a] < 8 || K[a] > 256 || (K[a] & (K[a] - 1))) return PGM_OK;
+    for (int a = 0; a < 3; ++a) {
+        int odd = K[a];
+        while (odd % 2 == 0) odd /= 2;
+        if (K[a] < 8 || K[a] > 256 || K[a] == odd || (odd != 1 && odd != 3 && odd != 5 && odd != 15)) return PGM_OK;
+        c->pfft_odd = c->pfft_odd || odd != 1;
+    }
     const PFFTGeom f{K[0], K[1], K[2], K[2] / 2, K[2] / 2 + 1, 0, 0, 0, 0};
     const size_t plane = c->mixed ? pfft_plane_lds<float>(f) : pfft_plane_lds<double>(f);
     if (plane > 160 * 1024) return PGM_OK;
@@ -904,17 +911,16 @@ static int fused_transform(pgm_ctx *c, const int *conv, int iter, hipStream_t st
     const int nth = f.K2 * f.K3 >= 8192 ? pfft_plane_threads<real>() : 256;
     const C *tw = c->pfft_tw.as<C>();
     if (fork && c->fork_stage == 3) HIP_TRY(hipStreamWaitEvent(st, c->ev_join, 0));  // planes after the row field
-    k_pme_fwd_plane<real><<<f.K1 * B, nth, plane, st>>>(f, (size_t)c->tiles.ntiles * c->tiles.bsize, c->merge_tab.as<int>(),
-                                                         c->blocks.as<real>(), c->cgrid.as<C>(), tw, conv, iter);
+    const auto fwd = c->pfft_odd ? k_pme_fwd_plane<real, true> : k_pme_fwd_plane<real, false>;
+    const auto bwd = c->pfft_odd ? k_pme_bwd_plane<real, true> : k_pme_bwd_plane<real, false>;
+    fwd<<<f.K1 * B, nth, plane, st>>>(f, (size_t)c->tiles.ntiles * c->tiles.bsize, c->merge_tab.as<int>(), c->blocks.as<real>(),
+                                      c->cgrid.as<C>(), tw, conv, iter);
     if (fork && c->fork_stage == 2) PGM_TRY((*fork)());
-    const dim3 gx(nblk((long long)f.K2 * f.K3h, PFFT_COLS), B);
-    if (epart)
-        k_pme_x_conv<real, true><<<gx, 256, pfft_xconv_lds<real>(f), st>>>(f, c->cgrid.as<C>(), c->Gc.as<real>(), tw + f.twK1,
-                                                                          conv, iter, epart);
-    else
-        k_pme_x_conv<real><<<gx, 256, pfft_xconv_lds<real>(f), st>>>(f, c->cgrid.as<C>(), c->Gc.as<real>(), tw + f.twK1, conv,
-                                                                     iter);
-    k_pme_bwd_plane<real><<<f.K1 * B, nth, plane, st>>>(f, c->cgrid.as<C>(), c->grid.as<real>(), tw, conv, iter);
+    const auto xc = c->pfft_odd ? (epart ? k_pme_x_conv<real, true, true> : k_pme_x_conv<real, true, false>)
+                                : (epart ? k_pme_x_conv<real, false, true> : k_pme_x_conv<real, false, false>);
+    xc<<<dim3(nblk((long long)f.K2 * f.K3h, PFFT_COLS), B), 256, pfft_xconv_lds<real>(f), st>>>(
+        f, c->cgrid.as<C>(), c->Gc.as<real>(), tw + f.twK1, conv, iter, epart);
+    bwd<<<f.K1 * B, nth, plane, st>>>(f, c->cgrid.as<C>(), c->grid.as<real>(), tw, conv, iter);
     LAUNCH_CHECK();
     return PGM_OK;
 }
@@ -3467,18 +3473,18 @@ template <typename real> static int time_impl(pgm_ctx *c, const double *pos, int
         const C *tw = c->pfft_tw.as<C>();
         ms[0] = 0.0;
         rc = timed(2, [&] {
-            k_pme_fwd_plane<real><<<f.K1 * c->nbead, nth, plane, st>>>(f, (size_t)c->tiles.ntiles * c->tiles.bsize,
+            (c->pfft_odd ? k_pme_fwd_plane<real, true> : k_pme_fwd_plane<real, false>)<<<f.K1 * c->nbead, nth, plane, st>>>(f, (size_t)c->tiles.ntiles * c->tiles.bsize,
                                                                         c->merge_tab.as<int>(), c->blocks.as<real>(),
                                                                         c->cgrid.as<C>(), tw, nullptr, -1);
         });
         if (rc < 0) return rc;
         rc = timed(3, [&] {
-            k_pme_x_conv<real><<<dim3(nblk((long long)f.K2 * f.K3h, PFFT_COLS), c->nbead), 256, pfft_xconv_lds<real>(f), st>>>(
-                f, c->cgrid.as<C>(), c->Gc.as<real>(), tw + f.twK1, nullptr, -1);
+            (c->pfft_odd ? k_pme_x_conv<real, true> : k_pme_x_conv<real, false>)<<<dim3(nblk((long long)f.K2 * f.K3h, PFFT_COLS), c->nbead), 256, pfft_xconv_lds<real>(f), st>>>(
+                f, c->cgrid.as<C>(), c->Gc.as<real>(), tw + f.twK1, nullptr, -1, nullptr);
         });
         if (rc < 0) return rc;
         rc = timed(4, [&] {
-            k_pme_bwd_plane<real><<<f.K1 * c->nbead, nth, plane, st>>>(f, c->cgrid.as<C>(), c->grid.as<real>(), tw, nullptr, -1);
+            (c->pfft_odd ? k_pme_bwd_plane<real, true> : k_pme_bwd_plane<real, false>)<<<f.K1 * c->nbead, nth, plane, st>>>(f, c->cgrid.as<C>(), c->grid.as<real>(), tw, nullptr, -1);
         });
         if (rc < 0) return rc;
     } else {
@@ -3657,7 +3663,7 @@ template <typename real> static int autotune_impl(pgm_ctx *c, const double *pos,
 extern "C" int pgm_set_pme_transform(pgm_ctx *c, int fused) {
     if (!c) return PGM_ERR_ARG;
     if (fused && !(c->fused_ok && c->tiled)) {
-        g_err = "pgm_set_pme_transform: the fused transform needs power-of-two grids of 8..256 points per axis, tiled "
+        g_err = "pgm_set_pme_transform: the fused transform needs grids of 8..256 points per axis (2^k times 1, 3, 5 or 15), tiled "
                 "spreading and a plane of K2 (K3/2 + 1) complex values within 160 KB";
         return PGM_ERR_ARG;
     }

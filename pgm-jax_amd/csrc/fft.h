@@ -1,8 +1,8 @@
 // fft.h -- the PME reciprocal-space convolution of one field (or energy) evaluation as three fused kernels.
 //
 // phi = c2r(Gc * r2c(Q)) over a K1 x K2 x K3 grid (z = K3 fastest; half spectrum of K3h = K3/2 + 1
-// points along z, the layout [x][y][kz] of the library's FFT plans), pme.py:373-376, with each K a
-// power of two (8..256):
+// points along z, the layout [x][y][kz] of the library's FFT plans), pme.py:373-376, with each K in
+// 8..256 a power of two times 1, 3, 5 or 15:
 //   k_pme_fwd_plane  one workgroup per x-plane: the spread-block merge of the plane (the sums of
 //                    k_merge_table), the real transform along z (a K3/2-point complex transform of
 //                    (x_2m, x_2m+1) and the split into the half spectrum), the transform along y;
@@ -10,7 +10,7 @@
 //                    inverse transform along x (with ENERGY also the sum of w Gc |F Q|^2);
 //   k_pme_bwd_plane  one workgroup per x-plane: the inverse along y, the merge of the half
 //                    spectrum into a K3/2-point complex sequence, the inverse along z -> real plane.
-// Every transform runs in LDS as radix-16/8/4/2 Stockham stages (autosort, in place: a stage reads all
+// Every transform runs in LDS as radix-16/8/4/2 and then radix-3/5 Stockham stages (autosort, in place: a stage reads all
 // its inputs into registers, then writes) with twiddles exp(-2 pi i t / N) tabulated in FP64 on the
 // host.  Unnormalised in both directions, like the library plans it replaces.
 #pragma once
@@ -101,19 +101,49 @@ template <bool INV, typename C> PGM_DEV void dft16(C *v) {
 #pragma unroll
     for (int k = 0; k < 16; ++k) v[k] = y[k];
 }
+template <bool INV, typename C> PGM_DEV void dft3(C *v) {
+    using R = decltype(C{}.x);
+    const R s = R(0.86602540378443864676);  // sin 60 deg
+    const C t = cadd(v[1], v[2]), d = csub(v[1], v[2]);
+    const C m = cmk<C>(v[0].x - R(0.5) * t.x, v[0].y - R(0.5) * t.y), n = cmi<INV>(cmk<C>(s * d.x, s * d.y));
+    v[0] = cadd(v[0], t);
+    v[1] = cadd(m, n);
+    v[2] = csub(m, n);
+}
+template <bool INV, typename C> PGM_DEV void dft5(C *v) {
+    using R = decltype(C{}.x);
+    const R c1 = R(0.30901699437494742410), c2 = R(-0.80901699437494742410);  // cos 72, cos 144 deg
+    const R s1 = R(0.95105651629515357212), s2 = R(0.58778525229247312917);   // sin 72, sin 144 deg
+    const C a = cadd(v[1], v[4]), b = cadd(v[2], v[3]), c = csub(v[1], v[4]), d = csub(v[2], v[3]);
+    const C m1 = cmk<C>(v[0].x + c1 * a.x + c2 * b.x, v[0].y + c1 * a.y + c2 * b.y);
+    const C m2 = cmk<C>(v[0].x + c2 * a.x + c1 * b.x, v[0].y + c2 * a.y + c1 * b.y);
+    const C n1 = cmi<INV>(cmk<C>(s1 * c.x + s2 * d.x, s1 * c.y + s2 * d.y));
+    const C n2 = cmi<INV>(cmk<C>(s2 * c.x - s1 * d.x, s2 * c.y - s1 * d.y));
+    v[0] = cadd(v[0], cadd(a, b));
+    v[1] = cadd(m1, n1);
+    v[4] = csub(m1, n1);
+    v[2] = cadd(m2, n2);
+    v[3] = csub(m2, n2);
+}
 template <int R, bool INV, typename C> PGM_DEV void dft(C *v) {
     if constexpr (R == 16) dft16<INV>(v);
+    else if constexpr (R == 5) dft5<INV>(v);
+    else if constexpr (R == 3) dft3<INV>(v);
     else if constexpr (R == 8) dft8<INV>(v);
     else if constexpr (R == 4) dft4<INV>(v[0], v[1], v[2], v[3]);
     else dft2<INV>(v);
 }
 
-// Radix of the next Stockham stage for a remaining length n (a power of two): 16 for n = 16 and
-// n >= 128, else 8 while it divides n, then 4, then 2 (128 = 16 x 8, 256 = 16 x 16, 64 = 8 x 8,
-// 32 = 8 x 4).
-PGM_DEV int fft_radix(int n) {
-    if (n == 16 || (n >= 128 && n % 16 == 0)) return 16;
-    return n % 8 == 0 ? 8 : (n % 4 == 0 ? 4 : 2);
+// Radix of the next Stockham stage for a remaining length n = 2^a {1, 3, 5, 15}: the power of two first
+// (16 for 2^a = 16 and 2^a >= 128, else 8 while it divides, then 4, then 2: 128 = 16 x 8, 256 = 16 x 16,
+// 64 = 8 x 8, 32 = 8 x 4), then 3, then 5.  ODD: lengths with a factor 3 or 5; kernels without it leave
+// those stages out (with them a transform of 32^3 took 24 instead of 22.5 us).
+template <bool ODD> PGM_DEV int fft_radix(int n) {
+    const int two = ODD ? n & -n : n;
+    if (two == 16 || two >= 128) return 16;
+    if (two >= 8) return 8;
+    if (!ODD || two > 1) return two;
+    return n % 3 == 0 ? 3 : 5;
 }
 
 // One Stockham stage (radix R, sub-transform length L -> L R) of nlines length-N transforms held in
@@ -141,7 +171,7 @@ PGM_DEV void fft_stage(C *buf, int N, int L, int nlines, int es, int ls, const C
             if (item < items) {
                 const int line = contiguous ? item / nb : item % nl;
                 const int j = contiguous ? item - line * nb : item / nl;
-                const int k = j & (L - 1);
+                const int k = R == 5 ? j % L : j & (L - 1);  // L is a power of two before a radix-5 stage
                 base[it] = (l0 + line) * ls;
                 jj[it] = j;
 #pragma unroll
@@ -160,7 +190,7 @@ PGM_DEV void fft_stage(C *buf, int N, int L, int nlines, int es, int ls, const C
 #pragma unroll
         for (int it = 0; it < IT; ++it) {
             if (base[it] >= 0) {
-                const int j = jj[it], k = j & (L - 1);
+                const int j = jj[it], k = R == 5 ? j % L : j & (L - 1);
                 const int o = (j - k) * R + k;
 #pragma unroll
                 for (int m = 0; m < R; ++m) buf[base[it] + (o + m * L) * es] = v[it][m];
@@ -172,12 +202,14 @@ PGM_DEV void fft_stage(C *buf, int N, int L, int nlines, int es, int ls, const C
 
 // Full length-N transform (forward: exp(-2 pi i ...), inverse: exp(+...), unnormalised) of nlines
 // lines in LDS; tw = W_N^t for t < N.
-template <bool INV, typename C> PGM_DEV void fft_lds(C *buf, int N, int nlines, int es, int ls, const C *__restrict__ tw) {
+template <bool INV, bool ODD, typename C> PGM_DEV void fft_lds(C *buf, int N, int nlines, int es, int ls, const C *__restrict__ tw) {
     for (int L = 1; L < N;) {
-        const int R = fft_radix(N / L);
+        const int R = fft_radix<ODD>(N / L);
         if (R == 16) fft_stage<16, INV, 1>(buf, N, L, nlines, es, ls, tw);
         else if (R == 8) fft_stage<8, INV, 2>(buf, N, L, nlines, es, ls, tw);
         else if (R == 4) fft_stage<4, INV, 2>(buf, N, L, nlines, es, ls, tw);
+        else if (ODD && R == 3) fft_stage<3, INV, 4>(buf, N, L, nlines, es, ls, tw);
+        else if (ODD && R == 5) fft_stage<5, INV, 2>(buf, N, L, nlines, es, ls, tw);
         else fft_stage<2, INV, 4>(buf, N, L, nlines, es, ls, tw);
         L *= R;
     }
@@ -188,6 +220,9 @@ struct PFFTGeom {
     int K1, K2, K3, M, K3h;
     int twM, twK3, twK2, twK1;
 };
+
+// p / K for p < 2^16, K <= 256 by a multiplication (m = 2^32 / K rounded up).
+PGM_DEV int div_small(int p, unsigned m) { return (int)__umulhi((unsigned)p, m); }
 
 // Threads of a plane workgroup at most: 1024 (FP32), 512 (FP64: twice the registers per value).
 template <typename real> constexpr int pfft_plane_threads() { return sizeof(real) == 4 ? 1024 : 512; }
@@ -215,7 +250,7 @@ template <typename real> inline size_t pfft_plane_lds(const PFFTGeom &f) {
 // store the plane's K2 K3h complex values at spec[(b K1 + x) K2 K3h ...].  Launch: K1 B blocks,
 // pfft_plane_lds bytes of dynamic LDS.  The twiddle tables of lengths K3/2, K3, K2 lie one after
 // the other from tw (offsets twM = 0, twK3 = K3/2, twK2 = K3/2 + K3).
-template <typename real>
+template <typename real, bool ODD>
 __global__ __launch_bounds__(pfft_plane_threads<real>()) void k_pme_fwd_plane(PFFTGeom f, size_t bead_blocks, const int *__restrict__ tab,
                                                         const real *__restrict__ blocks, cplx<real> *__restrict__ spec,
                                                         const cplx<real> *__restrict__ tw, const int *__restrict__ conv_it,
@@ -232,7 +267,7 @@ __global__ __launch_bounds__(pfft_plane_threads<real>()) void k_pme_fwd_plane(PF
     const int *tx = tab, *ty = tab + 2 * K1, *tz = tab + 2 * (K1 + K2);
     const int X0 = tx[2 * gx], X1 = tx[2 * gx + 1];
     const real *b = blocks + bead_blocks * bead;
-    const int lg3 = __ffs(K3) - 1;
+    const unsigned m3 = 0xffffffffu / (unsigned)K3 + 1u;
     const int nth = blockDim.x, npt = K2 * K3;
     // 1. merge (fixed order per point: the table candidates x, y, z in turn), four points per
     //    thread per pass with all their loads issued first; real line y at plr[2 y K3h ...]
@@ -241,7 +276,7 @@ __global__ __launch_bounds__(pfft_plane_threads<real>()) void k_pme_fwd_plane(PF
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int p = p0 + u * nth;
-            const int y = (p < npt ? p : 0) >> lg3, z = p & (K3 - 1);
+            const int pc = p < npt ? p : 0, y = div_small(pc, m3), z = pc - y * K3;
             const int X[2] = {X0, X1}, Y[2] = {ty[2 * y], ty[2 * y + 1]}, Z[2] = {tz[2 * z], tz[2 * z + 1]};
 #pragma unroll
             for (int i0 = 0; i0 < 2; ++i0)
@@ -260,13 +295,14 @@ __global__ __launch_bounds__(pfft_plane_threads<real>()) void k_pme_fwd_plane(PF
                 real acc = real(0);
 #pragma unroll
                 for (int c = 0; c < 8; ++c) acc += v[u][c];
-                plr[2 * (p >> lg3) * K3h + (p & (K3 - 1))] = acc;
+                const int y = div_small(p, m3);
+                plr[2 * y * K3h + (p - y * K3)] = acc;
             }
         }
     }
     __syncthreads();
     // 2. M-point transforms of z_m = x_2m + i x_2m+1 along every line
-    fft_lds<false>(pl, M, K2, 1, K3h, tws);
+    fft_lds<false, ODD>(pl, M, K2, 1, K3h, tws);
     // 3. half spectrum: X_k = E_k + W_K3^k O_k, E_k = (Z_k + conj Z_M-k) / 2, O_k = (Z_k - conj Z_M-k) / 2i
     const C *wk = tws + M;
     const int half = M / 2 + 1;
@@ -295,7 +331,7 @@ __global__ __launch_bounds__(pfft_plane_threads<real>()) void k_pme_fwd_plane(PF
     }
     __syncthreads();
     // 4. K2-point transforms along y (columns kz: stride K3h)
-    fft_lds<false>(pl, K2, K3h, K3h, 1, tws + M + K3);
+    fft_lds<false, ODD>(pl, K2, K3h, K3h, 1, tws + M + K3);
     // 5. store the plane
     C *out = spec + ((size_t)bead * K1 + gx) * (size_t)(K2 * K3h);
     for (int p = threadIdx.x; p < K2 * K3h; p += nth) out[p] = pl[p];
@@ -313,7 +349,7 @@ template <typename real> inline size_t pfft_xconv_lds(const PFFTGeom &f) {
 // Nyquist planes of the half spectrum, 1 elsewhere: the sum of k_convolve's ENERGY branch) to
 // epart[b * gridDim.x + blockIdx.x].  Launch: (ceil(K2 K3h / 16), B) blocks of 256 threads,
 // pfft_xconv_lds bytes of dynamic LDS; twx = the K1 twiddles.
-template <typename real, bool ENERGY = false>
+template <typename real, bool ODD, bool ENERGY = false>
 __global__ __launch_bounds__(256) void k_pme_x_conv(PFFTGeom f, cplx<real> *__restrict__ spec, const real *__restrict__ Gc,
                                                     const cplx<real> *__restrict__ twx, const int *__restrict__ conv_it, int iter,
                                                     double *__restrict__ epart = nullptr) {
@@ -343,7 +379,7 @@ __global__ __launch_bounds__(256) void k_pme_x_conv(PFFTGeom f, cplx<real> *__re
             if (p0 + u * nth < nv) col[p0 + u * nth] = v[u];
     }
     __syncthreads();
-    fft_lds<false>(col, K1, nc, PFFT_COLS, 1, tws);
+    fft_lds<false, ODD>(col, K1, nc, PFFT_COLS, 1, tws);
     double e[1] = {0.0};
     for (int p0 = threadIdx.x; p0 < nv; p0 += 4 * nth) {
         real g[4];
@@ -371,7 +407,7 @@ __global__ __launch_bounds__(256) void k_pme_x_conv(PFFTGeom f, cplx<real> *__re
         if (threadIdx.x == 0) epart[(size_t)bead * gridDim.x + blockIdx.x] = e[0];
     }
     __syncthreads();
-    fft_lds<true>(col, K1, nc, PFFT_COLS, 1, tws);
+    fft_lds<true, ODD>(col, K1, nc, PFFT_COLS, 1, tws);
     for (int p = threadIdx.x; p < nv; p += nth) {
         const int x = p / PFFT_COLS, cc = p - x * PFFT_COLS;
         if (cc < nc) s[(size_t)x * ncol + c0 + cc] = col[p];
@@ -383,7 +419,7 @@ __global__ __launch_bounds__(256) void k_pme_x_conv(PFFTGeom f, cplx<real> *__re
 // dropped), the inverse M-point transform gives (x_2m, x_2m+1); the real plane goes to
 // grid[(b K1 + x) K2 K3 ...].  Launch: K1 B blocks, pfft_plane_lds bytes of dynamic LDS, tw as
 // for the forward plane.
-template <typename real>
+template <typename real, bool ODD>
 __global__ __launch_bounds__(pfft_plane_threads<real>()) void k_pme_bwd_plane(PFFTGeom f, const cplx<real> *__restrict__ spec, real *__restrict__ grid,
                                                         const cplx<real> *__restrict__ tw, const int *__restrict__ conv_it,
                                                         int iter) {
@@ -398,7 +434,7 @@ __global__ __launch_bounds__(pfft_plane_threads<real>()) void k_pme_bwd_plane(PF
     copy_in(tws, tw, M + K3 + K2);
     copy_in(pl, spec + ((size_t)bead * K1 + gx) * (size_t)(K2 * K3h), K2 * K3h);
     __syncthreads();
-    fft_lds<true>(pl, K2, K3h, K3h, 1, tws + M + K3);
+    fft_lds<true, ODD>(pl, K2, K3h, K3h, 1, tws + M + K3);
     const C *wk = tws + M;
     const int half = M / 2 + 1;
     for (int p = threadIdx.x; p < K2 * half; p += blockDim.x) {
@@ -424,11 +460,11 @@ __global__ __launch_bounds__(pfft_plane_threads<real>()) void k_pme_bwd_plane(PF
         }
     }
     __syncthreads();
-    fft_lds<true>(pl, M, K2, 1, K3h, tws);
+    fft_lds<true, ODD>(pl, M, K2, 1, K3h, tws);
     real *out = grid + ((size_t)bead * K1 + gx) * (size_t)(K2 * K3);
-    const int lg3 = __ffs(K3) - 1;
+    const unsigned m3 = 0xffffffffu / (unsigned)K3 + 1u;
     for (int p = threadIdx.x; p < K2 * K3; p += blockDim.x) {
-        const int y = p >> lg3, z = p & (K3 - 1);
+        const int y = div_small(p, m3), z = p - y * K3;
         out[p] = plr[2 * y * K3h + z];
     }
 }
