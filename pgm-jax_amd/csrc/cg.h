@@ -513,6 +513,121 @@ __global__ __launch_bounds__(MOLP_BLOCK) void k_cg_update1_mol(int nper, const d
     }
 }
 
+// Both halves of an iteration in one launch, one workgroup per bead, for beads of at most CG_ONE_ATOMS atoms:
+// k_cg_update1 (with MOLP k_cg_update1_mol) and k_cg_update2 with the sums taken inside the workgroup
+// and r', z' and p kept in registers.  For such sizes each half is a launch of a few workgroups that waits
+// for the one before; one workgroup is through both in less time (FP32 alone, 512 waters: 4.1 + 4.6 us
+// and the gap between them against 6 us).
+constexpr int CG_ONE_THREADS = 1024, CG_ONE_STRIDE = 1023, CG_ONE_PER = 4;  // 341 whole molecules per round
+constexpr int CG_ONE_ATOMS = CG_ONE_STRIDE * CG_ONE_PER;
+template <typename real, bool MOLP>
+__global__ __launch_bounds__(CG_ONE_THREADS) void k_cg_update_one(int nper, const double *__restrict__ pap_part, int np, double *__restrict__ rz,
+                                                       double *__restrict__ err, int rzs, int k, real4<real> *__restrict__ x,
+                                                       real4<real> *__restrict__ r, real4<real> *__restrict__ z,
+                                                       real4<real> *__restrict__ p, const real4<real> *__restrict__ Ap,
+                                                       const real *__restrict__ alpha, const real *__restrict__ minv, CGState *st,
+                                                       double tol, int max_iter, unsigned long long *mirror) {
+    const int b = blockIdx.x;
+    const int conv0 = st[b].conv_it;
+    if (k >= conv0) {
+        if (threadIdx.x == 0) cg_mirror(mirror, gridDim.x, b, st[b].seq, k + 1, conv0);
+        return;
+    }
+    __shared__ double lds[2 * 16 + 16];
+    __shared__ double shared_beta;
+    __shared__ real sr[MOLP ? 3 * CG_ONE_STRIDE : 1];
+    rz += (size_t)b * rzs;
+    err += (size_t)b * rzs;
+    const int base = b * nper, t = threadIdx.x;
+    real4<real> r0[CG_ONE_PER], z1[CG_ONE_PER], pp[CG_ONE_PER], ap[CG_ONE_PER], xx[CG_ONE_PER];
+    real al0[CG_ONE_PER];
+#pragma unroll
+    for (int u = 0; u < CG_ONE_PER; ++u) {  // the vectors, in flight with the sum of p . Ap
+        const int li = u * CG_ONE_STRIDE + t;
+        if (t < CG_ONE_STRIDE && li < nper) {
+            pp[u] = p[base + li];
+            ap[u] = Ap[base + li];
+            r0[u] = r[base + li];
+            xx[u] = x[base + li];
+            al0[u] = alpha[base + li];
+        }
+    }
+    const double pap = block_reduce_partials(pap_part + (size_t)b * np, np, 1, 0, lds, false);
+    const double rzk = rz[k];
+    const real al = (real)(rzk / fmax(pap, 1e-300));
+    double s[2] = {0.0, 0.0};
+    double m = 0.0;
+#pragma unroll
+    for (int u = 0; u < CG_ONE_PER; ++u) {
+        const int li = u * CG_ONE_STRIDE + t;
+        const bool in = t < CG_ONE_STRIDE && li < nper;
+        real4<real> r1;
+        r1.x = r1.y = r1.z = r1.w = real(0);
+        if (in) {
+            xx[u].x += al * pp[u].x;
+            xx[u].y += al * pp[u].y;
+            xx[u].z += al * pp[u].z;
+            x[base + li] = xx[u];
+            r1.x = r0[u].x - al * ap[u].x;
+            r1.y = r0[u].y - al * ap[u].y;
+            r1.z = r0[u].z - al * ap[u].z;
+            r[base + li] = r1;
+        }
+        const real a = in ? al0[u] : real(0);
+        if constexpr (MOLP) {
+            if (u * CG_ONE_STRIDE < nper) {  // uniform
+                __syncthreads();
+                if (t < CG_ONE_STRIDE) {
+                    sr[3 * t] = r1.x;
+                    sr[3 * t + 1] = r1.y;
+                    sr[3 * t + 2] = r1.z;
+                }
+                __syncthreads();
+                if (in) {
+                    const int q = t / 3;
+                    z1[u] = mol_apply<real>(minv + (size_t)81 * ((base + li) / 3), t - 3 * q, sr + 9 * q);
+                }
+            }
+        } else {
+            z1[u].x = r1.x * a;
+            z1[u].y = r1.y * a;
+            z1[u].z = r1.z * a;
+            z1[u].w = 0;
+        }
+        if (in) {
+            z[base + li] = z1[u];
+            s[0] += (double)(z1[u].x * (r1.x - r0[u].x)) + (double)(z1[u].y * (r1.y - r0[u].y)) + (double)(z1[u].z * (r1.z - r0[u].z));
+            s[1] += (double)(r1.x * z1[u].x) + (double)(r1.y * z1[u].y) + (double)(r1.z * z1[u].z);
+            m = fmax(m, fmax(fmax(fabs((double)(a * r1.x)), fabs((double)(a * r1.y))), fabs((double)(a * r1.z))));
+        }
+    }
+    block_sum<2>(s, lds);
+    m = block_max(m, lds + 32);
+    if (t == 0) {
+        shared_beta = s[0] / fmax(rzk, 1e-300);
+        rz[k + 1] = s[1];
+        const double e = m / st[b].norm;
+        err[k + 1] = e;
+        const int conv = (e > tol && k + 1 < max_iter) ? conv0 : k + 1;
+        if (conv != conv0) st[b].conv_it = conv;
+        cg_mirror(mirror, gridDim.x, b, st[b].seq, k + 1, conv);
+    }
+    __syncthreads();
+    const real beta = (real)shared_beta;
+#pragma unroll
+    for (int u = 0; u < CG_ONE_PER; ++u) {
+        const int li = u * CG_ONE_STRIDE + t;
+        if (t < CG_ONE_STRIDE && li < nper) {
+            real4<real> v;
+            v.x = z1[u].x + beta * pp[u].x;
+            v.y = z1[u].y + beta * pp[u].y;
+            v.z = z1[u].z + beta * pp[u].z;
+            v.w = 0;
+            p[base + li] = v;
+        }
+    }
+}
+
 // Per bead b: iterations it_b = min(conv_it_b, launched) and the final residual err_b[it_b]
 // (bead_it, bead_res); stats slot = the largest of the residuals (kept on the device).  One block.
 __global__ void k_record_residual(int nbead, const double *__restrict__ err, int rzs, const CGState *__restrict__ st,

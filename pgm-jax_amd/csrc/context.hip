@@ -103,6 +103,7 @@ struct DevBuf {
 };
 
 constexpr int MOL_SPLIT = 2048;         // molecules from which the record pass takes one wave each
+constexpr int SPREAD_ROWS_LANES = 32;  // lanes per molecule of the row field beside the spread (k_spread_rows)
 constexpr int ROW_FIELD_WAVES = 2048;  // two waves per SIMD (row_field_lanes)
 
 struct pgm_ctx {
@@ -935,13 +936,15 @@ static int conv_partials(const pgm_ctx *c, bool vir) {
     return use_fused(c, vir) ? nblk((long long)c->pfg.K2 * c->pfg.K3h, PFFT_COLS) : nblk((long long)c->ncplx, 256);
 }
 
+template <typename real> static SpreadArgs<real> spread_args(const pgm_ctx *c) {
+    return {c->tiles, c->pg, c->corg.as<int>(), c->trange.as<int2>(), c->psidx.as<int>(), c->sten.as<real4<real>>(), c->blocks.as<real>()};
+}
+
 // The tiled spread of dq into the blocks.
 template <typename real>
 static int spread_tiles(pgm_ctx *c, const real4<real> *dq, bool withq, const int *conv, int iter, hipStream_t st, TimedPair tp = {}) {
-    const PMETiles &t = c->tiles;
     const auto go = [&](auto k) {
-        launch_timed(tp, k, dim3(c->nbead * t.ntiles), dim3(WAVE), 0, st, t, c->corg.as<int>(), c->pg,
-                     c->trange.as<int2>(), c->psidx.as<int>(), c->sten.as<real4<real>>(), dq, c->blocks.as<real>(), conv, iter);
+        launch_timed(tp, k, dim3(c->nbead * c->tiles.ntiles), dim3(WAVE), 0, st, spread_args<real>(c), dq, conv, iter);
     };
     if (withq) {
         ORDER_SWITCH(c->s.order, go(k_spread_tiles<real, PO, true>));
@@ -952,18 +955,18 @@ static int spread_tiles(pgm_ctx *c, const real4<real> *dq, bool withq, const int
     return PGM_OK;
 }
 
-// fork: called once the spread (fork_stage 1 and 4) or the forward planes (fork_stage 2) are enqueued.
+// spread_done: the (tiled) spread is already in the blocks.  fork: called once the spread (fork_stage 1 and 4) or the forward planes (fork_stage 2) are enqueued.
 template <typename real>
 static int spread_fft(pgm_ctx *c, const real4<real> *dq, bool withq, bool energy, const int *conv, int iter,
-                      double *vir_part = nullptr, const std::function<int()> *fork = nullptr) {
+                      double *vir_part = nullptr, const std::function<int()> *fork = nullptr, bool spread_done = false) {
     const int n = c->n;
     hipStream_t st = c->stream;
     const int P = c->s.order;
-    const TimedPair tp = energy ? TimedPair{} : timing_pair(c, 1);  // the spread kernel
+    const TimedPair tp = energy || spread_done ? TimedPair{} : timing_pair(c, 1);  // the spread kernel
     const int B = c->nbead;
     if (c->tiled) {
         const PMETiles &t = c->tiles;
-        PGM_TRY(spread_tiles<real>(c, dq, withq, conv, iter, st, tp));
+        if (!spread_done) PGM_TRY(spread_tiles<real>(c, dq, withq, conv, iter, st, tp));
         if (use_fused(c, vir_part != nullptr)) {  // merge + transforms + Gc fused (fft.h)
             if (fork && (c->fork_stage == 1 || c->fork_stage == 4)) PGM_TRY((*fork)());
             return fused_transform<real>(c, conv, iter, st, fork, energy ? c->conv_part.as<double>() : nullptr);
@@ -1061,14 +1064,16 @@ static int gather_combine(pgm_ctx *c, const real4<real> *dq, int mode, const rea
 }
 
 // Lanes that share a molecule's records in the row field: 16 (a chunk of records is read in whole
-// 256-byte segments), more while the launch has fewer than ROW_FIELD_WAVES waves and would leave SIMDs
+// 256-byte segments), 32 while the launch would have fewer than ROW_FIELD_WAVES waves and leave SIMDs
 // idle behind a few long chains of dependent gathers.  Measured alone (FP32, us per launch, with 4 / 16
 // / 32 / 64 lanes): 512 waters 31.6 / 10.3 / 7.4 / 5.9, 4,096: 39.4 / 14.8 / 12.2 / 13.6, 12,167: 43.7 /
-// 27.2 / 28.0 / 32.3, 32,768: 111.6 / 84.9 / 86.9 / 100.6.
-static int row_field_lanes(const pgm_ctx *c) {
-    int lanes = std::max(c->rlm, 16);
-    while (lanes < 64 && (long long)(c->n / 3) * lanes < 64LL * ROW_FIELD_WAVES) lanes *= 2;
-    return lanes;
+// 27.2 / 28.0 / 32.3, 32,768: 111.6 / 84.9 / 86.9 / 100.6.  (Where 64 would be faster the row field runs
+// beside the longer spread, spread_rows.)
+static int row_field_lanes(const pgm_ctx *c) { return (long long)(c->n / 3) * 16 < 64LL * ROW_FIELD_WAVES ? SPREAD_ROWS_LANES : 16; }
+
+template <typename real> static RowArgs<real> row_args(const pgm_ctx *c, Ext3 ext) {
+    return {c->n / 3, c->nper / 3, c->mcap, c->mj.as<int>(), c->mg.as<real>(), c->mcount.as<int>(), c->xr.as<double4>(), c->box,
+            c->vrow.as<real4<real>>(), ext};
 }
 
 // The CG row field of dq into vrow on stream st, in the context's layout.
@@ -1077,24 +1082,45 @@ static int row_field_launch(pgm_ctx *c, const real4<real> *dq, const int *conv, 
                             Ext3 ext = {}) {
     using R4 = real4<real>;
     if (c->layout == 1) {
-        const int nmol = c->n / 3, nb = c->nper / 3;
-        const int *mj = c->mj.as<int>(), *mc = c->mcount.as<int>();
-        const real *mg = c->mg.as<real>();
-        const double4 *xr = c->xr.as<double4>();
-        R4 *out = c->vrow.as<R4>();
         const auto go = [&](auto k, int lanes) {
-            launch_timed(tp, k, dim3(nblk((long long)nmol * lanes, 256)), dim3(256), 0, st, nmol, nb, c->mcap, mj, mg, mc, xr, dq, c->box, out,
-                         conv, iter, ext);
+            launch_timed(tp, k, dim3(nblk((long long)(c->n / 3) * lanes, 256)), dim3(256), 0, st, row_args<real>(c, ext), dq, conv, iter);
         };
-        switch (row_field_lanes(c)) {
-            case 16: go(k_row_field_mol<real, WITHQ, 16>, 16); break;
-            case 32: go(k_row_field_mol<real, WITHQ, 32>, 32); break;
-            default: go(k_row_field_mol<real, WITHQ, 64>, 64); break;
-        }
+        if (row_field_lanes(c) == 16)
+            go(k_row_field_mol<real, WITHQ, 16>, 16);
+        else
+            go(k_row_field_mol<real, WITHQ, SPREAD_ROWS_LANES>, SPREAD_ROWS_LANES);
     } else {
         launch_timed(tp, k_row_field<real, WITHQ>, dim3(nblk((long long)c->n * RL, 256)), dim3(256), 0, st, c->n, c->nper,
                      c->jell.as<int>(), c->count.as<int>(), c->G1.as<real>(), c->G2.as<real>(), c->xr.as<double4>(), dq, c->box,
                      c->vrow.as<R4>(), conv, iter, ext);
+    }
+    LAUNCH_CHECK();
+    return PGM_OK;
+}
+
+// The row field and the tiled spread of dq as one launch: the two read only dq and the geometry, each of
+// them leaves most of a small system's time to latency, and side by side in one grid they need neither
+// a second launch nor the events of the side stream.  A workgroup is four tiles of the spread or 256 threads
+// of the row field; the spread's come first, being the longer chain.
+template <typename real, int P, bool WITHQ>
+__global__ __launch_bounds__(256) void k_spread_rows(SpreadArgs<real> S, RowArgs<real> R, int nspread, const real4<real> *__restrict__ dq,
+                                                     const int *__restrict__ conv_it, int iter) {
+    __shared__ float4 w4[4][spread_lds16<real>()];
+    const int b = blockIdx.x, w = threadIdx.x / WAVE;
+    if (b < nspread)
+        spread_tile<real, P, WITHQ>(S, 4 * b + w, w4[w], dq, conv_it, iter);
+    else
+        row_field_mol<real, WITHQ, SPREAD_ROWS_LANES>(R, b - nspread, dq, conv_it, iter);
+}
+template <typename real>
+static int spread_rows(pgm_ctx *c, const real4<real> *dq, bool withq, const int *conv, int iter, Ext3 ext) {
+    const int ns = c->nbead * c->tiles.ntiles / 4;  // tiles come in cubes of eight
+    const dim3 grid(ns + nblk((long long)(c->n / 3) * SPREAD_ROWS_LANES, 256));
+    const auto go = [&](auto k) { k<<<grid, 256, 0, c->stream>>>(spread_args<real>(c), row_args<real>(c, ext), ns, dq, conv, iter); };
+    if (withq) {
+        ORDER_SWITCH(c->s.order, go(k_spread_rows<real, PO, true>));
+    } else {
+        ORDER_SWITCH(c->s.order, go(k_spread_rows<real, PO, false>));
     }
     LAUNCH_CHECK();
     return PGM_OK;
@@ -1152,7 +1178,11 @@ static int field_eval(pgm_ctx *c, const real4<real> *dq, bool withq, int mode, c
         LAUNCH_CHECK();
         return PGM_OK;
     }
-    PGM_TRY(spread_fft<real>(c, dq, withq, false, conv, iter, nullptr, late || (fused && c->fork_stage == 3) ? &fork : nullptr));
+    // in one launch where nothing separates the two: molecule records written on this stream, no live timing
+    const bool together = serial && late && c->layout == 1 && row_field_lanes(c) == SPREAD_ROWS_LANES && !c->rec_pending && !c->timing;
+    if (together) PGM_TRY(spread_rows<real>(c, dq, withq, conv, iter, withq ? ext : Ext3{}));
+    PGM_TRY(spread_fft<real>(c, dq, withq, false, conv, iter, nullptr,
+                             !together && (late || (fused && c->fork_stage == 3)) ? &fork : nullptr, together));
     if (!serial) {
         HIP_TRY(hipStreamWaitEvent(st, c->ev_join, 0));
         c->rec_pending = false;  // the row field followed the record pass on the side stream
@@ -1468,6 +1498,14 @@ static int cg_iterate(pgm_ctx *c, double tol, int expect, bool graphs, int *laun
     auto iteration = [&](int k) -> int {
         hipStream_t cs = c->stream;
         PGM_TRY(field_eval<real>(c, p, false, MODE_AV, nullptr, Ap, c->partA.as<double>(), k));
+        unsigned long long *mir = mirror ? c->h_mirror : nullptr;
+        if (nper <= CG_ONE_ATOMS) {
+            const auto k1 = c->molp ? k_cg_update_one<real, true> : k_cg_update_one<real, false>;
+            k1<<<B, CG_ONE_THREADS, 0, cs>>>(nper, c->partA.as<double>(), gather_parts(c), rz, err, c->rzs, k, x, r, z, p, Ap,
+                                             c->alpha_r.as<real>(), c->molp ? c->pinv.as<real>() : nullptr, S, tol, max_iter, mir);
+            LAUNCH_CHECK();
+            return PGM_OK;
+        }
         if (c->molp)
             k_cg_update1_mol<real><<<gM, MOLP_BLOCK, 0, cs>>>(nper, c->partA.as<double>(), gather_parts(c), rz, c->rzs, k, x, r, z,
                                                                p, Ap, c->alpha_r.as<real>(), c->pinv.as<real>(),
@@ -1476,7 +1514,7 @@ static int cg_iterate(pgm_ctx *c, double tol, int expect, bool graphs, int *laun
             k_cg_update1<real><<<gB, 256, 0, cs>>>(nper, c->partA.as<double>(), gather_parts(c), rz, c->rzs, k, x, r, z, p, Ap,
                                                    c->alpha_r.as<real>(), c->partB.as<double>(), S);
         k_cg_update2<real><<<gB, 256, 0, cs>>>(nper, c->partB.as<double>(), npb, rz, err, c->rzs, k, z, p, S, tol,
-                                               max_iter, mirror ? c->h_mirror : nullptr);
+                                               max_iter, mir);
         LAUNCH_CHECK();
         return PGM_OK;
     };

@@ -941,14 +941,31 @@ __global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_mol_tensors(
 
 // Row field of the molecule blocks: out_i for the three atoms of I (the same sum as k_row_field over
 // the pairs within rc, in molecule-pair order).  RLM lanes per molecule take its records in turn.
+template <typename real> struct RowArgs {
+    int nmol, nmol_bead, mcap;
+    const int *mj;
+    const real *mg;
+    const int *mcount;
+    const double4 *xr;
+    Box box;
+    real4<real> *out;
+    Ext3 ext;
+};
+
+// Workgroup `block` of the row field.
 template <typename real, bool WITHQ, int RLM>
-__global__ __launch_bounds__(256) void k_row_field_mol(int nmol, int nmol_bead, int mcap, const int *__restrict__ mj,
-                                                       const real *__restrict__ mg, const int *__restrict__ mcount,
-                                                       const double4 *__restrict__ xr, const real4<real> *__restrict__ dq,
-                                                       Box box, real4<real> *__restrict__ out, const int *__restrict__ conv_it,
-                                                       int iter, Ext3 ext = {}) {
+PGM_DEV void row_field_mol(const RowArgs<real> &A, int block, const real4<real> *__restrict__ dq, const int *__restrict__ conv_it,
+                           int iter) {
+    const int nmol = A.nmol, nmol_bead = A.nmol_bead, mcap = A.mcap;
+    const int *__restrict__ mj = A.mj;
+    const real *__restrict__ mg = A.mg;
+    const int *__restrict__ mcount = A.mcount;
+    const double4 *__restrict__ xr = A.xr;
+    const Box &box = A.box;
+    real4<real> *__restrict__ out = A.out;
+    const Ext3 &ext = A.ext;
     const int lane = threadIdx.x % RLM;
-    const int I = blockIdx.x * (blockDim.x / RLM) + threadIdx.x / RLM;
+    const int I = block * (blockDim.x / RLM) + threadIdx.x / RLM;
     if (I >= nmol || cg_done(conv_it, I / nmol_bead, iter)) return;
     const double4 a[3] = {xr[3 * I], xr[3 * I + 1], xr[3 * I + 2]};
     real acc[9];
@@ -1012,6 +1029,12 @@ __global__ __launch_bounds__(256) void k_row_field_mol(int nmol, int nmol_bead, 
             }
             out[3 * I + p] = v;
         }
+}
+
+template <typename real, bool WITHQ, int RLM>
+__global__ __launch_bounds__(256) void k_row_field_mol(RowArgs<real> A, const real4<real> *__restrict__ dq,
+                                                       const int *__restrict__ conv_it, int iter) {
+    row_field_mol<real, WITHQ, RLM>(A, blockIdx.x, dq, conv_it, iter);
 }
 
 // ---------------------------------------------------------------------------- molecule-blocked force pass

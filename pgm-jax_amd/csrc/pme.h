@@ -236,23 +236,41 @@ PGM_DEV mfma_acc<double>::type mfma_16x16x4(double a, double b, mfma_acc<double>
 // Row of result register r of lane group grp = lane / 16 (lane l holds column l % 16).
 template <typename real> PGM_DEV int mfma_row(int grp, int r) { return sizeof(real) == 4 ? 4 * grp + r : grp + 4 * r; }
 
+// LDS of one wave of the spread, in 16-byte units.
+template <typename real> constexpr int spread_lds16() {
+    return (SPREAD_PLANES * SPREAD_CHUNK * SPREAD_ROW * (int)sizeof(real) + 15) / 16;
+}
+template <typename real> struct SpreadArgs {
+    PMETiles t;
+    PMEGeom g;
+    const int *corg;
+    const int2 *range;
+    const int *sidx;
+    const real4<real> *sten;
+    real *blocks;
+};
+
+// Tile `tile` (bead * t.ntiles + key) by one wave, its rows in w4.
 template <typename real, int P, bool WITHQ>
-__global__ __launch_bounds__(64, sizeof(real) == 4 ? 4 : 2) void k_spread_tiles(PMETiles t, const int *__restrict__ corg, PMEGeom g,
-                                                     const int2 *__restrict__ range, const int *__restrict__ sidx,
-                                                     const real4<real> *__restrict__ sten, const real4<real> *__restrict__ dq,
-                                                     real *__restrict__ blocks, const int *__restrict__ conv_it, int iter) {
-    const int bead = blockIdx.x / t.ntiles, key = blockIdx.x - bead * t.ntiles;
+PGM_DEV void spread_tile(const SpreadArgs<real> &A, int tile, float4 *w4, const real4<real> *__restrict__ dq,
+                         const int *__restrict__ conv_it, int iter) {
+    const PMETiles &t = A.t;
+    const PMEGeom &g = A.g;
+    const int *__restrict__ corg = A.corg;
+    const int2 *__restrict__ range = A.range;
+    const int *__restrict__ sidx = A.sidx;
+    const real4<real> *__restrict__ sten = A.sten;
+    real *__restrict__ blocks = A.blocks;
+    const int bead = tile / t.ntiles, key = tile - bead * t.ntiles;
     if (cg_done(conv_it, bead, iter)) return;
     int u8[3];
     if (!octant_tile(corg[key >> 3], key & 7, t, u8)) return;  // no merge reads the block
     using acc_t = typename mfma_acc<real>::type;
-    constexpr int MAXB = P + 7;  // tile rows at most (T <= 8)
-    constexpr int PLANE = SPREAD_CHUNK * SPREAD_ROW;
-    constexpr int NZ = (SPREAD_PLANES * PLANE * (int)sizeof(real) + 15) / 16;
-    __shared__ float4 w4[NZ];
+    constexpr int MAXB = P + 7;  // block rows at most (T <= 8)
+    constexpr int PLANE = SPREAD_CHUNK * SPREAD_ROW, NZ = spread_lds16<real>();
     real *w = reinterpret_cast<real *>(w4);
-    const int lane = threadIdx.x, grp = lane / 16, m = lane % 16;
-    const int2 rg = range[blockIdx.x];
+    const int lane = threadIdx.x % WAVE, grp = lane / 16, m = lane % 16;
+    const int2 rg = range[tile];
     const int s0 = rg.x, s1 = rg.y;
     acc_t D[MAXB];
 #pragma unroll
@@ -320,7 +338,7 @@ __global__ __launch_bounds__(64, sizeof(real) == 4 ? 4 : 2) void k_spread_tiles(
             }
         }
     }
-    real *out = blocks + (size_t)blockIdx.x * t.bsize + m;
+    real *out = blocks + (size_t)tile * t.bsize + m;
 #pragma unroll
     for (int y = 0; y < MAXB; ++y) {
         if (y < t.B[1]) {
@@ -331,6 +349,13 @@ __global__ __launch_bounds__(64, sizeof(real) == 4 ? 4 : 2) void k_spread_tiles(
             }
         }
     }
+}
+
+template <typename real, int P, bool WITHQ>
+__global__ __launch_bounds__(64, sizeof(real) == 4 ? 4 : 2) void k_spread_tiles(SpreadArgs<real> A, const real4<real> *__restrict__ dq,
+                                                     const int *__restrict__ conv_it, int iter) {
+    __shared__ float4 w4[spread_lds16<real>()];
+    spread_tile<real, P, WITHQ>(A, blockIdx.x, w4, dq, conv_it, iter);
 }
 
 // Block merge: grid point value = sum of the tiles' blocks covering it -- along each axis its own tile

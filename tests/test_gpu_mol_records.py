@@ -1,7 +1,7 @@
 """The molecule-block records at the edges of their choices (GPU): their field against the atom rows'.
 
 Sizes either side of the switch from four waves per molecule to one (2,048 molecules), sizes either side
-of the row field's lane counts (64 / 32 / 16 per molecule), and a box whose half is hardly more than the
+of the row field's lane counts (32 or 16 per molecule; 32 beside the spread in one launch), and a box whose half is hardly more than the
 cutoff, where the pairs of a molecule pair can have different lattice shifts; molecules whole and
 wrapped into the box atom by atom.  Same sums in another order, FP64 to 1e-12 and FP32 to 1e-6 relative RMS
 (the row layouts' own test).
