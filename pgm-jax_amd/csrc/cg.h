@@ -515,12 +515,15 @@ __global__ __launch_bounds__(MOLP_BLOCK) void k_cg_update1_mol(int nper, const d
 
 // Both halves of an iteration in one launch, one workgroup per bead, for beads of at most CG_ONE_ATOMS atoms:
 // k_cg_update1 (with MOLP k_cg_update1_mol) and k_cg_update2 with the sums taken inside the workgroup
-// and r', z' and p kept in registers.  For such sizes each half is a launch of a few workgroups that waits
-// for the one before; one workgroup is through both in less time (FP32 alone, 512 waters: 4.1 + 4.6 us
-// and the gap between them against 6 us).
-constexpr int CG_ONE_THREADS = 1024, CG_ONE_STRIDE = 1023, CG_ONE_PER = 4;  // 341 whole molecules per round
-constexpr int CG_ONE_ATOMS = CG_ONE_STRIDE * CG_ONE_PER;
-template <typename real, bool MOLP>
+// and z' and p kept in registers, PER atoms per thread.  For such sizes each half is a launch of a few
+// workgroups that waits for the one before.  Bound by latency: every wave sums the partials of p . Ap by
+// itself, and the three sums of the update cross the workgroup with one barrier (with the block sums of
+// the two kernels, ten barriers of sixteen waves, it took 14 us where the two kernels take 10).  Measured
+// against the two kernels without the gap between them: 192 atoms, FP32 4.7 / 8.2 us, 1,536, FP64 8.6 / 8.7,
+// 3,993, FP32 10.2 / 9.1, where the line is drawn.
+constexpr int CG_ONE_THREADS = 1024, CG_ONE_STRIDE = 1023;  // 341 whole molecules per round
+constexpr int CG_ONE_ATOMS = 2 * CG_ONE_STRIDE;
+template <typename real, bool MOLP, int PER>
 __global__ __launch_bounds__(CG_ONE_THREADS) void k_cg_update_one(int nper, const double *__restrict__ pap_part, int np, double *__restrict__ rz,
                                                        double *__restrict__ err, int rzs, int k, real4<real> *__restrict__ x,
                                                        real4<real> *__restrict__ r, real4<real> *__restrict__ z,
@@ -533,89 +536,85 @@ __global__ __launch_bounds__(CG_ONE_THREADS) void k_cg_update_one(int nper, cons
         if (threadIdx.x == 0) cg_mirror(mirror, gridDim.x, b, st[b].seq, k + 1, conv0);
         return;
     }
-    __shared__ double lds[2 * 16 + 16];
-    __shared__ double shared_beta;
+    constexpr int NW = CG_ONE_THREADS / WAVE;
+    __shared__ double lds[3][NW];
     __shared__ real sr[MOLP ? 3 * CG_ONE_STRIDE : 1];
     rz += (size_t)b * rzs;
     err += (size_t)b * rzs;
-    const int base = b * nper, t = threadIdx.x;
-    real4<real> r0[CG_ONE_PER], z1[CG_ONE_PER], pp[CG_ONE_PER], ap[CG_ONE_PER], xx[CG_ONE_PER];
-    real al0[CG_ONE_PER];
+    pap_part += (size_t)b * np;
+    const int base = b * nper, t = threadIdx.x, lane = t % WAVE, wv = t / WAVE;
+    double pap = 0.0;
+    for (int c = lane; c < np; c += WAVE) pap += pap_part[c];
+    const double rzk = rz[k];
+    real4<real> pp[PER], z1[PER], r0[PER], r1[PER];
 #pragma unroll
-    for (int u = 0; u < CG_ONE_PER; ++u) {  // the vectors, in flight with the sum of p . Ap
+    for (int u = 0; u < PER; ++u) {
         const int li = u * CG_ONE_STRIDE + t;
         if (t < CG_ONE_STRIDE && li < nper) {
             pp[u] = p[base + li];
-            ap[u] = Ap[base + li];
             r0[u] = r[base + li];
-            xx[u] = x[base + li];
-            al0[u] = alpha[base + li];
+            r1[u] = Ap[base + li];
         }
     }
-    const double pap = block_reduce_partials(pap_part + (size_t)b * np, np, 1, 0, lds, false);
-    const double rzk = rz[k];
+    pap = wave_sum(pap);
     const real al = (real)(rzk / fmax(pap, 1e-300));
-    double s[2] = {0.0, 0.0};
-    double m = 0.0;
+    double s0 = 0.0, s1 = 0.0, m = 0.0;
 #pragma unroll
-    for (int u = 0; u < CG_ONE_PER; ++u) {
+    for (int u = 0; u < PER; ++u) {
         const int li = u * CG_ONE_STRIDE + t;
         const bool in = t < CG_ONE_STRIDE && li < nper;
-        real4<real> r1;
-        r1.x = r1.y = r1.z = r1.w = real(0);
         if (in) {
-            xx[u].x += al * pp[u].x;
-            xx[u].y += al * pp[u].y;
-            xx[u].z += al * pp[u].z;
-            x[base + li] = xx[u];
-            r1.x = r0[u].x - al * ap[u].x;
-            r1.y = r0[u].y - al * ap[u].y;
-            r1.z = r0[u].z - al * ap[u].z;
-            r[base + li] = r1;
+            real4<real> xx = x[base + li];
+            xx.x += al * pp[u].x;
+            xx.y += al * pp[u].y;
+            xx.z += al * pp[u].z;
+            x[base + li] = xx;
+            r1[u].x = r0[u].x - al * r1[u].x;
+            r1[u].y = r0[u].y - al * r1[u].y;
+            r1[u].z = r0[u].z - al * r1[u].z;
+            r1[u].w = 0;
+            r[base + li] = r1[u];
         }
-        const real a = in ? al0[u] : real(0);
+        const real a = in ? alpha[base + li] : real(0);
         if constexpr (MOLP) {
-            if (u * CG_ONE_STRIDE < nper) {  // uniform
-                __syncthreads();
-                if (t < CG_ONE_STRIDE) {
-                    sr[3 * t] = r1.x;
-                    sr[3 * t + 1] = r1.y;
-                    sr[3 * t + 2] = r1.z;
-                }
-                __syncthreads();
-                if (in) {
-                    const int q = t / 3;
-                    z1[u] = mol_apply<real>(minv + (size_t)81 * ((base + li) / 3), t - 3 * q, sr + 9 * q);
-                }
+            __syncthreads();
+            if (in) {
+                sr[3 * t] = r1[u].x;
+                sr[3 * t + 1] = r1[u].y;
+                sr[3 * t + 2] = r1[u].z;
             }
-        } else {
-            z1[u].x = r1.x * a;
-            z1[u].y = r1.y * a;
-            z1[u].z = r1.z * a;
+            __syncthreads();
+            if (in) {
+                const int q = t / 3;
+                z1[u] = mol_apply<real>(minv + (size_t)81 * ((base + li) / 3), t - 3 * q, sr + 9 * q);
+            }
+        } else if (in) {
+            z1[u].x = r1[u].x * a;
+            z1[u].y = r1[u].y * a;
+            z1[u].z = r1[u].z * a;
             z1[u].w = 0;
         }
         if (in) {
             z[base + li] = z1[u];
-            s[0] += (double)(z1[u].x * (r1.x - r0[u].x)) + (double)(z1[u].y * (r1.y - r0[u].y)) + (double)(z1[u].z * (r1.z - r0[u].z));
-            s[1] += (double)(r1.x * z1[u].x) + (double)(r1.y * z1[u].y) + (double)(r1.z * z1[u].z);
-            m = fmax(m, fmax(fmax(fabs((double)(a * r1.x)), fabs((double)(a * r1.y))), fabs((double)(a * r1.z))));
+            s0 += (double)(z1[u].x * (r1[u].x - r0[u].x)) + (double)(z1[u].y * (r1[u].y - r0[u].y)) +
+                  (double)(z1[u].z * (r1[u].z - r0[u].z));
+            s1 += (double)(r1[u].x * z1[u].x) + (double)(r1[u].y * z1[u].y) + (double)(r1[u].z * z1[u].z);
+            m = fmax(m, fmax(fmax(fabs((double)(a * r1[u].x)), fabs((double)(a * r1[u].y))), fabs((double)(a * r1[u].z))));
         }
     }
-    block_sum<2>(s, lds);
-    m = block_max(m, lds + 32);
-    if (t == 0) {
-        shared_beta = s[0] / fmax(rzk, 1e-300);
-        rz[k + 1] = s[1];
-        const double e = m / st[b].norm;
-        err[k + 1] = e;
-        const int conv = (e > tol && k + 1 < max_iter) ? conv0 : k + 1;
-        if (conv != conv0) st[b].conv_it = conv;
-        cg_mirror(mirror, gridDim.x, b, st[b].seq, k + 1, conv);
+    s0 = wave_sum(s0);
+    s1 = wave_sum(s1);
+    m = wave_max(m);
+    if (lane == 0) {
+        lds[0][wv] = s0;
+        lds[1][wv] = s1;
+        lds[2][wv] = m;
     }
     __syncthreads();
-    const real beta = (real)shared_beta;
+    s0 = group_sum<NW>(lds[0][lane % NW]);
+    const real beta = (real)(s0 / fmax(rzk, 1e-300));
 #pragma unroll
-    for (int u = 0; u < CG_ONE_PER; ++u) {
+    for (int u = 0; u < PER; ++u) {
         const int li = u * CG_ONE_STRIDE + t;
         if (t < CG_ONE_STRIDE && li < nper) {
             real4<real> v;
@@ -624,6 +623,18 @@ __global__ __launch_bounds__(CG_ONE_THREADS) void k_cg_update_one(int nper, cons
             v.z = z1[u].z + beta * pp[u].z;
             v.w = 0;
             p[base + li] = v;
+        }
+    }
+    if (wv == 0) {
+        s1 = group_sum<NW>(lds[1][lane % NW]);
+        m = wave_max(lds[2][lane % NW]);
+        if (lane == 0) {
+            rz[k + 1] = s1;
+            const double e = m / st[b].norm;
+            err[k + 1] = e;
+            const int conv = (e > tol && k + 1 < max_iter) ? conv0 : k + 1;
+            if (conv != conv0) st[b].conv_it = conv;
+            cg_mirror(mirror, gridDim.x, b, st[b].seq, k + 1, conv);
         }
     }
 }

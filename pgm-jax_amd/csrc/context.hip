@@ -188,12 +188,13 @@ struct pgm_ctx {
     PFFTGeom pfg{};
     DevBuf pfft_tw;
     // tiled spread (atoms sorted by grid tile)
-    // tiles of T points per axis (one fine key each) in cubes of 2 x 2 x 2; trange (start, end) by fine key
+    // tiles of T points per axis (one fine key each) in cubes of 2 x 2 x 2; trange (start, end) by fine key;
+    // tcount: atoms per tile, zero between binnings
     bool tiled = false;
     int tile_cap = 8;  // largest spread-tile width tried per axis (pgm_autotune lowers it)
     PMETiles tiles{};
     DevBuf corg;  // packed cube coordinates (octant_tile)
-    DevBuf pkey, pidx, pskey, psidx, trange, sten, blocks, pme_sort_tmp, merge_tab;
+    DevBuf pkey, pidx, pskey, psidx, trange, tcount, sten, blocks, pme_sort_tmp, merge_tab;
     // vectors (real4 N) and FP64 (N, 3) work arrays
     DevBuf vx, vr, vz, vp, vAp, vb, vx0, vrow, vdq, vtmp;
     DevBuf pperm, dd, g_el, g_lj, rowf, rec_dr, gp;
@@ -488,6 +489,9 @@ static int setup_tiles(pgm_ctx *c) {
     PGM_TRY(c->pskey.ensure(sizeof(int) * n));
     PGM_TRY(c->psidx.ensure(sizeof(int) * n));
     PGM_TRY(c->trange.ensure(sizeof(int2) * B * t.ntiles));
+    PGM_TRY(c->tcount.ensure(sizeof(int) * B * t.ntiles));
+    k_fill_int<<<nblk((long long)B * t.ntiles, 256), 256, 0, c->stream>>>((int)(B * t.ntiles), c->tcount.as<int>(), 0);
+    LAUNCH_CHECK();
     PGM_TRY(c->sten.ensure(c->rsize * 4 * (size_t)n));
     PGM_TRY(c->blocks.ensure(c->rsize * B * t.ntiles * t.bsize));
     {  // per-axis offsets of the block merge (k_merge_table, k_pme_fwd_plane)
@@ -527,19 +531,29 @@ template <typename real> static int pme_bin(pgm_ctx *c, const double *pos) {
     hipStream_t st = c->stream;
     const PMETiles &t = c->tiles;
     const int nk = c->nbead * t.ntiles;
-    k_pme_bin<<<nblk(n, 256), 256, 0, st>>>(n, c->nper, pos, c->pg, t, c->pkey.as<int>(), c->pidx.as<int>());
+    real4<real> *sten = c->sten.as<real4<real>>();
+    // key and arrival number in pkey / pidx; slots (arrival order) in pskey; the sorted atoms in psidx
+    k_pme_bin<<<nblk(n, 256), 256, 0, st>>>(n, c->nper, pos, c->pg, t, c->pkey.as<int>(), c->pidx.as<int>(), c->tcount.as<int>());
     LAUNCH_CHECK();
-    int bits = 1;
-    while ((1 << bits) < nk) ++bits;
-    size_t tmp = 0;
-    HIP_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, c->pkey.as<int>(), c->pskey.as<int>(), c->pidx.as<int>(),
-                                               c->psidx.as<int>(), n, 0, bits, st));
-    PGM_TRY(c->pme_sort_tmp.ensure(tmp));
-    HIP_TRY(hipcub::DeviceRadixSort::SortPairs(c->pme_sort_tmp.p, tmp, c->pkey.as<int>(), c->pskey.as<int>(), c->pidx.as<int>(),
-                                               c->psidx.as<int>(), n, 0, bits, st));
-    k_tile_bounds<<<nblk(n + 1, 256), 256, 0, st>>>(n, c->pskey.as<int>(), nk, c->trange.as<int2>());
-    LAUNCH_CHECK();
-    k_pme_stencils<real><<<nblk(n, 256), 256, 0, st>>>(n, pos, c->pg, t, c->psidx.as<int>(), c->sten.as<real4<real>>());
+    if (nk <= PME_SCAN_MAX) {
+        k_pme_scan<<<1, 1024, 0, st>>>(nk, c->tcount.as<int>(), c->trange.as<int2>());
+        k_pme_place<<<nblk(n, 256), 256, 0, st>>>(n, c->pkey.as<int>(), c->pidx.as<int>(), c->trange.as<int2>(), c->pskey.as<int>());
+        k_pme_order<real><<<nblk(nk, 4), 256, 0, st>>>(nk, c->trange.as<int2>(), c->pskey.as<int>(), pos, c->pg, t, c->psidx.as<int>(),
+                                                       sten);
+    } else {
+        int bits = 1;
+        while ((1 << bits) < nk) ++bits;
+        k_iota<<<nblk(n, 256), 256, 0, st>>>(n, c->pidx.as<int>());
+        size_t tmp = 0;
+        HIP_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, c->pkey.as<int>(), c->pskey.as<int>(), c->pidx.as<int>(),
+                                                   c->psidx.as<int>(), n, 0, bits, st));
+        PGM_TRY(c->pme_sort_tmp.ensure(tmp));
+        HIP_TRY(hipcub::DeviceRadixSort::SortPairs(c->pme_sort_tmp.p, tmp, c->pkey.as<int>(), c->pskey.as<int>(), c->pidx.as<int>(),
+                                                   c->psidx.as<int>(), n, 0, bits, st));
+        k_pme_sorted<real><<<nblk(n + 1, 256), 256, 0, st>>>(n, c->pskey.as<int>(), nk, c->psidx.as<int>(), pos, c->pg, t,
+                                                             c->trange.as<int2>(), sten);
+        k_fill_int<<<nblk(nk, 256), 256, 0, st>>>(nk, c->tcount.as<int>(), 0);
+    }
     LAUNCH_CHECK();
     return PGM_OK;
 }
@@ -1500,9 +1514,15 @@ static int cg_iterate(pgm_ctx *c, double tol, int expect, bool graphs, int *laun
         PGM_TRY(field_eval<real>(c, p, false, MODE_AV, nullptr, Ap, c->partA.as<double>(), k));
         unsigned long long *mir = mirror ? c->h_mirror : nullptr;
         if (nper <= CG_ONE_ATOMS) {
-            const auto k1 = c->molp ? k_cg_update_one<real, true> : k_cg_update_one<real, false>;
-            k1<<<B, CG_ONE_THREADS, 0, cs>>>(nper, c->partA.as<double>(), gather_parts(c), rz, err, c->rzs, k, x, r, z, p, Ap,
-                                             c->alpha_r.as<real>(), c->molp ? c->pinv.as<real>() : nullptr, S, tol, max_iter, mir);
+            const auto go = [&](auto k1) {
+                k1<<<B, CG_ONE_THREADS, 0, cs>>>(nper, c->partA.as<double>(), gather_parts(c), rz, err, c->rzs, k, x, r, z, p, Ap,
+                                                 c->alpha_r.as<real>(), c->molp ? c->pinv.as<real>() : nullptr, S, tol, max_iter, mir);
+            };
+            const bool one = nper <= CG_ONE_STRIDE;
+            if (c->molp)
+                one ? go(k_cg_update_one<real, true, 1>) : go(k_cg_update_one<real, true, 2>);
+            else
+                one ? go(k_cg_update_one<real, false, 1>) : go(k_cg_update_one<real, false, 2>);
             LAUNCH_CHECK();
             return PGM_OK;
         }
@@ -2183,7 +2203,7 @@ extern "C" int pgm_ctx_destroy(pgm_ctx *c) {
                      &c->pair_part, &c->pack_part, &c->conv_part, &c->st, &c->rz, &c->err, &c->energy, &c->bead_it, &c->bead_res,
                      &c->mrows, &c->mcount_full, &c->mcount, &c->mj, &c->mg, &c->pinv,
                      &c->pos_build, &c->minv, &c->mass, &c->d2, &c->md_part, &c->md_fail, &c->heat,
-                     &c->pkey, &c->pidx, &c->pskey, &c->psidx, &c->trange, &c->corg, &c->sten,
+                     &c->pkey, &c->pidx, &c->pskey, &c->psidx, &c->trange, &c->tcount, &c->corg, &c->sten,
                      &c->blocks, &c->merge_tab, &c->pfft_tw,
                      &c->pme_sort_tmp, &c->stats, &c->mol_ptr, &c->mol_atoms, &c->com, &c->off, &c->rec_dd,
                      &c->vir_pair, &c->vir_conv, &c->vir_atoms, &c->vir_cov, &c->vir_out, &c->kvec, &c->sk,

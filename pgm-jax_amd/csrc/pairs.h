@@ -47,6 +47,11 @@ __global__ void k_fill_int(int n, int *__restrict__ p, int v) {
     if (i < n) p[i] = v;
 }
 
+__global__ void k_iota(int n, int *__restrict__ p) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = i;
+}
+
 // cell_start[c] / cell_end[c] from the sorted keys.
 __global__ void k_cell_bounds(int n, const int *__restrict__ skey, int *__restrict__ start, int *__restrict__ end) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
