@@ -31,6 +31,14 @@ template <typename real> using real4 = typename vec4<real>::type;
 constexpr int CG_STRIDE = 4;
 PGM_DEV bool cg_done(const int *conv, int bead, int iter) { return conv && iter >= conv[bead * CG_STRIDE]; }
 
+// Workgroups are dealt to the eight XCDs in turn, each with an L2 of its own.  With consecutive work on
+// one XCD (workgroup b of nb takes item (b mod 8) (nb / 8) + b / 8) neighbours in space, which mostly are
+// neighbours in index, share an L2 instead of having their surroundings fetched into all eight.
+PGM_DEV int xcd_block(int b, int nb) {
+    const int per = nb / 8;
+    return b < 8 * per ? (b & 7) * per + (b >> 3) : b;
+}
+
 // Reduced lower-triangular box: lattice vectors as rows, h[3a+b].
 struct Box {
     double h[9];

@@ -580,20 +580,29 @@ template <typename real> PGM_DEV int mslot(int e, int t) {
     return t < FULL ? (t / V) * (V * MCH) + s * V + t % V : FULL * MCH + s * (MOL_REC - FULL) + (t - FULL);
 }
 // The 18 reals of record e of the chunk at g, to or from registers.
-PGM_DEV void mload(const float *__restrict__ g, int e, float (&G)[MOL_REC]) {
+// STREAM: non-temporal loads, for records that are not read again before they leave the caches.
+template <bool STREAM, typename V> PGM_DEV V stream_load(const V *p) {
+    if constexpr (STREAM) return __builtin_nontemporal_load(p);
+    return *p;
+}
+template <bool STREAM> PGM_DEV void mload(const float *__restrict__ g, int e, float (&G)[MOL_REC]) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    typedef float f2 __attribute__((ext_vector_type(2)));
     const int s = e % MCH;
-    const float4 *q = reinterpret_cast<const float4 *>(g) + s;
-    const float4 a = q[0], b = q[MCH], c = q[2 * MCH], d = q[3 * MCH];
-    const float2 t = reinterpret_cast<const float2 *>(g + 16 * MCH)[s];
+    const f4 *q = reinterpret_cast<const f4 *>(g) + s;
+    const f4 a = stream_load<STREAM>(q), b = stream_load<STREAM>(q + MCH), c = stream_load<STREAM>(q + 2 * MCH),
+             d = stream_load<STREAM>(q + 3 * MCH);
+    const f2 t = stream_load<STREAM>(reinterpret_cast<const f2 *>(g + 16 * MCH) + s);
     const float v[MOL_REC] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, c.x, c.y, c.z, c.w, d.x, d.y, d.z, d.w, t.x, t.y};
 #pragma unroll
     for (int k = 0; k < MOL_REC; ++k) G[k] = v[k];
 }
-PGM_DEV void mload(const double *__restrict__ g, int e, double (&G)[MOL_REC]) {
-    const double2 *q = reinterpret_cast<const double2 *>(g) + e % MCH;
+template <bool STREAM> PGM_DEV void mload(const double *__restrict__ g, int e, double (&G)[MOL_REC]) {
+    typedef double d2 __attribute__((ext_vector_type(2)));
+    const d2 *q = reinterpret_cast<const d2 *>(g) + e % MCH;
 #pragma unroll
     for (int k = 0; k < MOL_REC / 2; ++k) {
-        const double2 v = q[k * MCH];
+        const d2 v = stream_load<STREAM>(q + k * MCH);
         G[2 * k] = v.x;
         G[2 * k + 1] = v.y;
     }
@@ -778,7 +787,8 @@ __global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_mol_tensors(
     __shared__ int2 nearq[4][MOL_QUEUE];
     __shared__ int wsum[4];
     const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE;
-    const int I = WPM == 1 ? blockIdx.x * 4 + wv : blockIdx.x;
+    const int blk = xcd_block(blockIdx.x, gridDim.x);
+    const int I = WPM == 1 ? blk * 4 + wv : blk;
     if (I >= nmol) return;
     int2 *queue = nearq[wv];
     const double4 a[3] = {xr[3 * I], xr[3 * I + 1], xr[3 * I + 2]};
@@ -945,7 +955,9 @@ __global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_mol_tensors(
 }
 
 // Row field of the molecule blocks: out_i for the three atoms of I (the same sum as k_row_field over
-// the pairs within rc, in molecule-pair order).  RLM lanes per molecule take its records in turn.
+// the pairs within rc, in molecule-pair order).  RLM lanes per molecule take its records in turn.  Bound by the
+// record stream in large systems (32,768 waters: 338 MB in 81 us, 4.2 TB/s, where a copy reaches 4.8), by
+// the partners' gathers and latency in smaller ones.
 template <typename real> struct RowArgs {
     int nmol, nmol_bead, mcap;
     const int *mj;
@@ -958,7 +970,7 @@ template <typename real> struct RowArgs {
 };
 
 // Workgroup `block` of the row field.
-template <typename real, bool WITHQ, int RLM>
+template <typename real, bool WITHQ, int RLM, bool STREAM>
 PGM_DEV void row_field_mol(const RowArgs<real> &A, int block, const real4<real> *__restrict__ dq, const int *__restrict__ conv_it,
                            int iter) {
     const int nmol = A.nmol, nmol_bead = A.nmol_bead, mcap = A.mcap;
@@ -982,7 +994,7 @@ PGM_DEV void row_field_mol(const RowArgs<real> &A, int block, const real4<real> 
         const unsigned word = (unsigned)words[e];
         const int J = (int)(word & ((1u << 26) - 1u)), code = (int)(word >> 26);
         real G[MOL_REC];
-        mload(mg + mchunk(e, I, mcap), e, G);
+        mload<STREAM>(mg + mchunk(e, I, mcap), e, G);
         double4 b[3];
         real4<real> d[3];
 #pragma unroll
@@ -1036,10 +1048,10 @@ PGM_DEV void row_field_mol(const RowArgs<real> &A, int block, const real4<real> 
         }
 }
 
-template <typename real, bool WITHQ, int RLM>
+template <typename real, bool WITHQ, int RLM, bool STREAM>
 __global__ __launch_bounds__(256) void k_row_field_mol(RowArgs<real> A, const real4<real> *__restrict__ dq,
                                                        const int *__restrict__ conv_it, int iter) {
-    row_field_mol<real, WITHQ, RLM>(A, blockIdx.x, dq, conv_it, iter);
+    row_field_mol<real, WITHQ, RLM, STREAM>(A, xcd_block(blockIdx.x, gridDim.x), dq, conv_it, iter);
 }
 
 // ---------------------------------------------------------------------------- molecule-blocked force pass
@@ -1096,7 +1108,7 @@ __global__ __launch_bounds__(3 * WAVE, sizeof(real) == 4 ? 3 : 1) void k_pair_fo
     __shared__ real4<real> s_d[2][3][WAVE];
     const int lane = threadIdx.x % FL, wl = threadIdx.x % WAVE;
     const int p = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const int lm = blockIdx.x * MOL_FORCE_MOLS + wl / FL;  // molecule of the bead
+    const int lm = xcd_block(blockIdx.x, gridDim.x) * MOL_FORCE_MOLS + wl / FL;  // molecule of the bead
     const bool in = 3 * lm < nper;
     const int I = blockIdx.y * (nper / 3) + (in ? lm : 0), i = 3 * I + p;
     const int pb = blockIdx.y * gridDim.x + blockIdx.x;

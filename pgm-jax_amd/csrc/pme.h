@@ -159,13 +159,15 @@ __global__ void k_pme_bin(int n, int nper, const double *__restrict__ pos, PMEGe
     arrival[i] = atomicAdd(count + k, 1);
 }
 
-// One workgroup of 1024 threads; PME_SCAN_MAX tiles at most (more are sorted by the library).
-constexpr int PME_SCAN_MAX = 1 << 17;
-__global__ __launch_bounds__(1024) void k_pme_scan(int nk, int *__restrict__ count, int2 *__restrict__ range) {
-    __shared__ int wsum[16];
+// One workgroup; PME_SCAN_MAX tiles at most (more are sorted by the library).  Four waves: a workgroup of
+// sixteen waited 160 us for a CU with room beside the record pass.
+constexpr int PME_SCAN_MAX = 1 << 17, PME_SCAN_THREADS = 256;
+__global__ __launch_bounds__(PME_SCAN_THREADS) void k_pme_scan(int nk, int *__restrict__ count, int2 *__restrict__ range) {
+    constexpr int NW = PME_SCAN_THREADS / WAVE;
+    __shared__ int wsum[NW];
     const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE;
     int carry = 0;
-    for (int k0 = 0; k0 < nk; k0 += 4096) {
+    for (int k0 = 0; k0 < nk; k0 += 4 * PME_SCAN_THREADS) {
         const int k = k0 + 4 * threadIdx.x;
         int c[4], sum = 0;
 #pragma unroll
@@ -184,7 +186,7 @@ __global__ __launch_bounds__(1024) void k_pme_scan(int nk, int *__restrict__ cou
         __syncthreads();
         int before = carry, total = 0;
 #pragma unroll
-        for (int w = 0; w < 16; ++w) {
+        for (int w = 0; w < NW; ++w) {
             if (w < wv) before += wsum[w];
             total += wsum[w];
         }
