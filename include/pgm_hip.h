@@ -106,6 +106,11 @@ int pgm_set_box(pgm_ctx *ctx, const double *H);
  * the device positions pos (N,3).  Returns PGM_ROW_OVERFLOW after growing the capacity. */
 int pgm_build_rows(pgm_ctx *ctx, const double *pos);
 
+/* Largest displacement [nm] of an atom of pos (all beads, device) since the rows were built (no minimum
+ * image: molecules move continuously); infinity while there are no valid rows.  The caller's test for
+ * pgm_build_rows, against half the skin (MDEngine's list update).  Synchronises. */
+int pgm_rows_displacement(pgm_ctx *ctx, const double *pos, double *displacement);
+
 /* Number of stored row entries (pairs counted twice) within cutoff at the last compute. */
 long long pgm_row_entries(pgm_ctx *ctx);
 
@@ -192,8 +197,8 @@ int pgm_set_graphs(pgm_ctx *ctx, int on);
 /* Layout of the CG row field (the data of PGMForceField._row_field, forcefield.py:1395-1402): 0 atom
  * rows (partner index, G1, G2 per pair in sliced ELL), 1 molecule blocks (contexts of consecutive
  * 3-atom molecules: per molecule pair the 9 atom pairs' G1, G2, `lanes` = 4, 8 or 16: at least so many
- * lanes per molecule (the launch takes 16 to 64 by the size of the system); the default where it applies).  Same sums in another order; rows are rebuilt at the
- * next evaluation.  pgm_row_layout reports the layout and its lanes. */
+ * lanes per molecule, of which the launch takes 16 or 32 by the size of the system; the default where
+ * it applies).  Same sums in another order; rows are rebuilt at the next evaluation.  pgm_row_layout reports the layout and its lanes. */
 int pgm_set_row_layout(pgm_ctx *ctx, int layout, int lanes);
 int pgm_row_layout(const pgm_ctx *ctx, int *layout, int *lanes);
 

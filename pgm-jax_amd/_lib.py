@@ -25,6 +25,7 @@ EXPORTS = (
     "pgm_set_stream",
     "pgm_set_box",
     "pgm_build_rows",
+    "pgm_rows_displacement",
     "pgm_row_entries",
     "pgm_row_blocks",
     "pgm_perm_dipoles",
@@ -181,6 +182,7 @@ def lib() -> C.CDLL:
     L.pgm_set_stream.argtypes = [P, P]
     L.pgm_set_box.argtypes = [P, C.POINTER(D)]
     L.pgm_build_rows.argtypes = [P, P]
+    L.pgm_rows_displacement.argtypes = [P, P, C.POINTER(C.c_double)]
     L.pgm_row_entries.argtypes = [P]
     L.pgm_row_entries.restype = C.c_longlong
     L.pgm_row_blocks.argtypes = [P]

@@ -25,7 +25,7 @@ import dataclasses
 import numpy as np
 
 from . import _lib
-from .forcefield import InductionState, _autotune, _dev, _make_context, _ptr, _set_transform, _torch, _transform
+from .forcefield import InductionState, _autotune, _dev, _displacement, _make_context, _ptr, _set_transform, _torch, _transform
 from .settings import MDSettings, grid_size
 from .system import System
 
@@ -74,7 +74,7 @@ class PGMBeads:
         self.K = tuple(int(k) for k in (settings.pme_grid or grid_size(H, settings.pme_spacing)))
         self._ctx, self._stream = _make_context(sys, H, settings, self.K, self.P)
         self._H = H.copy()
-        self._built_at = None
+        self._rows_built = False
 
     def __del__(self) -> None:
         ctx = getattr(self, "_ctx", None)
@@ -99,21 +99,18 @@ class PGMBeads:
         if not np.array_equal(H, self._H):
             _lib.check(_lib.lib().pgm_set_box(self._ctx, _ptr(H, C.c_double)), "pgm_set_box")
             self._H = H.copy()
-            self._built_at = None
+            self._rows_built = False
 
     def _ensure_rows(self, q) -> None:
-        torch = _torch()
-        if self._built_at is not None:
-            disp = torch.max(torch.linalg.norm((q - self._built_at).reshape(-1, 3), dim=1)).item()
-            if disp <= 0.5 * self.s.skin:
-                return
+        if self._rows_built and _displacement(self._ctx, self._stream, q) <= 0.5 * self.s.skin:
+            return
         _lib.check(_lib.lib().pgm_build_rows(self._ctx, C.c_void_p(q.data_ptr())), "pgm_build_rows")
-        self._built_at = q.clone()
+        self._rows_built = True
 
     def autotune(self, q, reps: int = 20) -> dict:
         """Time every row-field layout, PME spread-tile width and reciprocal transform on the beads q (P, N, 3); keep the fastest."""
         q = _dev(q, (self.P, self.n, 3))
-        self._built_at = None
+        self._rows_built = False
         return _autotune(self._ctx, q, reps)
 
     def set_pme_transform(self, transform: str = "fused") -> None:

@@ -327,6 +327,19 @@ __global__ __launch_bounds__(256) void k_max_disp(int n, const double *__restric
     if (threadIdx.x == 0) part[blockIdx.x] = d;
 }
 
+// The same over all atoms by one workgroup of 1024 threads, to *out (pinned host memory).
+__global__ __launch_bounds__(1024) void k_max_disp_one(int n, const double *__restrict__ pos, const double *__restrict__ ref,
+                                                       double *__restrict__ out) {
+    __shared__ double lds[32];
+    double d2 = 0.0;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+        const double dx = pos[3 * i] - ref[3 * i], dy = pos[3 * i + 1] - ref[3 * i + 1], dz = pos[3 * i + 2] - ref[3 * i + 2];
+        d2 = fmax(d2, dx * dx + dy * dy + dz * dz);
+    }
+    d2 = block_max(d2, lds);
+    if (threadIdx.x == 0) *out = sqrt(d2);
+}
+
 __global__ void k_scale3(int n3, double *__restrict__ v, double f) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n3) v[i] *= f;

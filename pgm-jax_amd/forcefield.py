@@ -125,6 +125,17 @@ def _transform(ctx) -> tuple[str, bool]:
     return ("library", "fused")[fused.value], bool(avail.value)
 
 
+def _displacement(ctx, stream, pos) -> float:
+    """Largest displacement [nm] of an atom of pos since the context's rows were built (pgm_rows_displacement)."""
+    torch = _torch()
+    now = torch.cuda.current_stream()
+    if now.cuda_stream != stream.cuda_stream:  # the context's stream reads what this one has queued
+        now.synchronize()
+    d = C.c_double()
+    _lib.check(_lib.lib().pgm_rows_displacement(ctx, C.c_void_p(pos.data_ptr()), C.byref(d)), "pgm_rows_displacement")
+    return d.value
+
+
 class PGMForceField:
     """The pGM + LJ force field of one system on the GPU (forcefield.py:810-1000)."""
 
@@ -136,7 +147,7 @@ class PGMForceField:
         self.K = tuple(int(k) for k in (settings.pme_grid or grid_size(H, settings.pme_spacing)))
         self._ctx, self._stream = _make_context(sys, H, settings, self.K)
         self._H = H.copy()
-        self._built_at = None
+        self._rows_built = False
 
     def __del__(self) -> None:
         ctx = getattr(self, "_ctx", None)
@@ -161,20 +172,15 @@ class PGMForceField:
         if not np.array_equal(H, self._H):
             _lib.check(_lib.lib().pgm_set_box(self._ctx, _ptr(H, C.c_double)), "pgm_set_box")
             self._H = H.copy()
-            self._built_at = None
+            self._rows_built = False
 
     def build_rows(self, pos) -> None:
         """Rebuild the neighbour rows (cell list, cutoff + skin) at pos."""
         _lib.check(_lib.lib().pgm_build_rows(self._ctx, C.c_void_p(pos.data_ptr())), "pgm_build_rows")
-        self._built_at = pos.clone()
+        self._rows_built = True
 
     def _ensure_rows(self, pos) -> None:
-        torch = _torch()
-        if self._built_at is None:
-            self.build_rows(pos)
-            return
-        disp = torch.max(torch.linalg.norm(pos - self._built_at, dim=1)).item()
-        if disp > 0.5 * self.s.skin:
+        if not self._rows_built or _displacement(self._ctx, self._stream, pos) > 0.5 * self.s.skin:
             self.build_rows(pos)
 
     def _efield(self, efield) -> bool:
@@ -507,12 +513,12 @@ class PGMForceField:
         """Choose the CG row-field layout: "atom" rows or "molecule" blocks (3-site molecules; 4, 8 or 16 lanes)."""
         code = {"atom": 0, "molecule": 1}[layout]
         _lib.check(_lib.lib().pgm_set_row_layout(self._ctx, code, int(lanes)), "pgm_set_row_layout")
-        self._built_at = None
+        self._rows_built = False
 
     def autotune(self, pos, reps: int = 20) -> dict:
         """Time every row-field layout, PME spread-tile width and reciprocal transform at pos; keep the fastest."""
         pos = _dev(pos, (self.n, 3))
-        self._built_at = None
+        self._rows_built = False
         return _autotune(self._ctx, pos, reps)
 
     def set_graphs(self, on: bool = True) -> None:
