@@ -1078,6 +1078,32 @@ static int gather_combine(pgm_ctx *c, const real4<real> *dq, int mode, const rea
     return PGM_OK;
 }
 
+// The force evaluation's gather, on the tiles that its spread has binned where the grid is tiled.
+template <typename real> static int gather_forces(pgm_ctx *c, const real4<real> *dq, double *rec_dd) {
+    hipStream_t st = c->stream;
+    const double *dd = c->dd.as<double>(), *rowf = c->rowf.as<double>();
+    double *rec_dr = c->rec_dr.as<double>(), *gp = c->gp.as<double>();
+    if (c->tiled) {
+        const PMETiles &t = c->tiles;
+        constexpr int GW = gather_waves<real>(), V = 16 / (int)sizeof(real);
+        const auto go = [&](auto k) {
+            k<<<c->nbead * t.ntiles / GW, WAVE * GW, 0, st>>>(t, c->corg.as<int>(), c->pg, c->trange.as<int2>(), c->psidx.as<int>(),
+                                                              c->sten.as<real4<real>>(), c->grid.as<real>(), dq, dd, rowf, c_self(c),
+                                                              rec_dr, gp, rec_dd);
+        };
+        if (c->s.grid[2] % V == 0 && t.T[2] % V == 0) {
+            ORDER_SWITCH(c->s.order, go(k_gather_forces_tiles<real, PO, true>));
+        } else {
+            ORDER_SWITCH(c->s.order, go(k_gather_forces_tiles<real, PO, false>));
+        }
+    } else {
+        ORDER_SWITCH(c->s.order, (k_gather_forces<real, PO><<<nblk(c->n, 256), 256, 0, st>>>(
+                                     c->n, c->nper, c->pos, c->pg, c->grid.as<real>(), dq, dd, rowf, c_self(c), rec_dr, gp, rec_dd)));
+    }
+    LAUNCH_CHECK();
+    return PGM_OK;
+}
+
 // Lanes that share a molecule's records in the row field: 16 (a chunk of records is read in whole
 // 256-byte segments), 32 while the launch would have fewer than ROW_FIELD_WAVES waves and leave SIMDs
 // idle behind a few long chains of dependent gathers.  Measured alone (FP32, us per launch, with 4 / 16
@@ -1850,10 +1876,7 @@ static int energy_forces_impl(pgm_ctx *c, const double *mu, pgm_energy *energy, 
     } else {
         PGM_TRY(spread_fft<real>(c, dq, true, true, nullptr, -1, vir ? c->vir_conv.as<double>() : nullptr));
         if (!vir) HIP_TRY(hipStreamWaitEvent(st, c->ev_join, 0));  // the pair pass's row field
-        ORDER_SWITCH(c->s.order, (k_gather_forces<real, PO><<<nb, 256, 0, st>>>(
-                                     n, nper, c->pos, c->pg, c->grid.as<real>(), dq, c->dd.as<double>(), c->rowf.as<double>(),
-                                     c_self(c), c->rec_dr.as<double>(), c->gp.as<double>(),
-                                     vir ? c->rec_dd.as<double>() : nullptr)));
+        PGM_TRY(gather_forces<real>(c, dq, vir ? c->rec_dd.as<double>() : nullptr));
     }
     LAUNCH_CHECK();
     if (vir) {
@@ -3607,7 +3630,7 @@ template <typename real> static int time_impl(pgm_ctx *c, const double *pos, int
 // Time the CG matvec's pieces for every applicable shape on this context's own system and keep the
 // fastest: the row-field layout (molecule blocks with 4, 8 or 16 lanes per molecule, atom rows) by
 // the row field alone, then the spread-tile width (the largest valid width up to 8, 7, 6, ... P-1
-// per axis; gather tiles are 2 x 2 x 2 spread tiles) by spread + merge + gather.
+// per axis; the gather uses the same tiles) by spread + merge + gather.
 template <typename real> static int autotune_impl(pgm_ctx *c, const double *pos, int reps, double *out) {
     using R4 = real4<real>;
     hipStream_t st = c->stream;

@@ -596,6 +596,50 @@ PGM_DEV void combine_out(int mode, int i, real rx, real ry, real rz, const real4
     out[i] = o;
 }
 
+// One wave copies the potential on a tile's (T + P - 1)^3 block (periodic wrap) into blk, 16 bytes per lane
+// and load where the rows allow it (VEC: K3 and T2 multiples of 16 / sizeof(real)), and waits for its writes.
+template <typename real, int P, bool VEC>
+PGM_DEV void load_tile_block(const PMETiles &t, const PMEGeom &g, const int *u8, const real *__restrict__ phi, real *blk, int lane) {
+    constexpr int V = VEC ? 16 / (int)sizeof(real) : 1, LPR = 16 / V, RPI = WAVE / LPR;  // reals, lanes per row, rows per load
+    constexpr int SZ = (P + 7) | 1;
+    const int K1 = g.K[0], K2 = g.K[1], K3 = g.K[2], BY = t.B[1], BZ = t.B[2], nrow = t.B[0] * BY;
+    const int bz = V * (lane % LPR);
+    int gz = u8[2] * t.T[2] + bz;
+    gz -= gz >= K3 ? K3 : 0;
+    const int o0 = u8[0] * t.T[0], o1 = u8[1] * t.T[1];
+    const unsigned magic = 65536u / (unsigned)BY + 1u;  // row / BY for row < 256
+    constexpr int BATCH = 8;
+    for (int r0 = lane / LPR; r0 < nrow; r0 += BATCH * RPI) {
+        real v[BATCH][V];
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) {
+            const int rr = r0 + u * RPI < nrow ? r0 + u * RPI : 0;
+            const int bx = (int)(((unsigned)rr * magic) >> 16), by = rr - bx * BY;
+            int gx = o0 + bx, gy = o1 + by;
+            gx -= gx >= K1 ? K1 : 0;
+            gy -= gy >= K2 ? K2 : 0;
+            const real *src = phi + ((size_t)gx * K2 + gy) * K3 + gz;
+            if constexpr (V == 4) {
+                const float4 q = *reinterpret_cast<const float4 *>(src);
+                v[u][0] = q.x, v[u][1] = q.y, v[u][2] = q.z, v[u][3] = q.w;
+            } else if constexpr (V == 2) {
+                const double2 q = *reinterpret_cast<const double2 *>(src);
+                v[u][0] = q.x, v[u][1] = q.y;
+            } else {
+                v[u][0] = bz < BZ ? *src : real(0);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u)
+            if (r0 + u * RPI < nrow)
+#pragma unroll
+                for (int k = 0; k < V; ++k)
+                    if (bz + k < BZ) blk[(r0 + u * RPI) * SZ + bz + k] = v[u][k];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Tiled gather + combine: one wave per tile (fine key), GATHER_WAVES waves per workgroup.  The wave copies
 // the potential on the tile's (T + P - 1)^3 block (periodic wrap) into its part of the LDS, 16 bytes
 // per lane and load where the rows allow it (VEC: K3 and T2 multiples of 16 / sizeof(real)), then two
@@ -617,22 +661,20 @@ __global__ __launch_bounds__(WAVE * gather_waves<real>()) void k_gather_tiles(PM
     constexpr int GW = gather_waves<real>();
     const int bead = (blockIdx.x * GW) / t.ntiles;  // t.ntiles is a multiple of 8
     if (cg_done(conv_it, bead, iter)) return;
-    constexpr int V = VEC ? 16 / (int)sizeof(real) : 1, LPR = 16 / V, RPI = WAVE / LPR;  // reals, lanes per row, rows per load
     constexpr int MAXB = P + 7, SZ = MAXB | 1;
     __shared__ real blk_all[GW][MAXB * MAXB * SZ];
     __shared__ double lds[16];
     const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE;
     const int tile = blockIdx.x * GW + wv;
     real *blk = blk_all[wv];
-    const int BY = t.B[1], BZ = t.B[2], nrow = t.B[0] * BY;
+    const int BY = t.B[1];
     const int2 rg = range[tile];
     const int s0 = rg.x, s1 = rg.y, lt = tile - bead * t.ntiles;
     const int half = lane & 1;
     double acc[1] = {0.0};
     int u8[3];
     if (s0 < s1 && octant_tile(corg[lt >> 3], lt & 7, t, u8)) {
-        const int K1 = g.K[0], K2 = g.K[1], K3 = g.K[2];
-        phi += (size_t)bead * K1 * K2 * K3;
+        phi += (size_t)bead * g.K[0] * g.K[1] * g.K[2];
         int s = s0 + (lane >> 1);
         real4<real> st{};
         int atom = 0;
@@ -640,41 +682,7 @@ __global__ __launch_bounds__(WAVE * gather_waves<real>()) void k_gather_tiles(PM
             st = sten[s];
             atom = sidx[s];
         }
-        const int bz = V * (lane % LPR);
-        int gz = u8[2] * t.T[2] + bz;
-        gz -= gz >= K3 ? K3 : 0;
-        const int o0 = u8[0] * t.T[0], o1 = u8[1] * t.T[1];
-        const unsigned magic = 65536u / (unsigned)BY + 1u;  // row / BY for row < 256
-        constexpr int BATCH = 8;
-        for (int r0 = lane / LPR; r0 < nrow; r0 += BATCH * RPI) {
-            real v[BATCH][V];
-#pragma unroll
-            for (int u = 0; u < BATCH; ++u) {
-                const int rr = r0 + u * RPI < nrow ? r0 + u * RPI : 0;
-                const int bx = (int)(((unsigned)rr * magic) >> 16), by = rr - bx * BY;
-                int gx = o0 + bx, gy = o1 + by;
-                gx -= gx >= K1 ? K1 : 0;
-                gy -= gy >= K2 ? K2 : 0;
-                const real *src = phi + ((size_t)gx * K2 + gy) * K3 + gz;
-                if constexpr (V == 4) {
-                    const float4 q = *reinterpret_cast<const float4 *>(src);
-                    v[u][0] = q.x, v[u][1] = q.y, v[u][2] = q.z, v[u][3] = q.w;
-                } else if constexpr (V == 2) {
-                    const double2 q = *reinterpret_cast<const double2 *>(src);
-                    v[u][0] = q.x, v[u][1] = q.y;
-                } else {
-                    v[u][0] = bz < BZ ? *src : real(0);
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < BATCH; ++u)
-                if (r0 + u * RPI < nrow)
-#pragma unroll
-                    for (int k = 0; k < V; ++k)
-                        if (bz + k < BZ) blk[(r0 + u * RPI) * SZ + bz + k] = v[u][k];
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        load_tile_block<real, P, VEC>(t, g, u8, phi, blk, lane);
         constexpr int PH = (P + 1) / 2;  // x planes of the first lane of a pair
         while (__ballot(s < s1)) {
             if (s < s1) {
@@ -797,6 +805,30 @@ __global__ __launch_bounds__(256) void k_gather_combine(int n, const double *__r
     }
 }
 
+// phi-weighted sums S[wx][wy][wz] with w = 0 (theta), 1 (dtheta), 2 (d2theta):
+// gd_a = S(d along a), gw_a = q S(d along a) + sum_b e_b S(d along a, d along b / d2 if a == b).
+template <typename real>
+PGM_DEV void force_out(int i, const real4<real> &d, const PMEGeom &g, double s100, double s010, double s001, double s200, double s020,
+                       double s002, double s110, double s101, double s011, const double *__restrict__ dd,
+                       const double *__restrict__ rowf, double cself, double *__restrict__ rec_dr, double *__restrict__ gp,
+                       double *__restrict__ rec_dd) {
+    real e[3];
+    scaled_dipole<real>(d, g, e);
+    const real q = d.w;
+    const double gd[3] = {s100, s010, s001};
+    const double qq = (double)q, e0 = (double)e[0], e1 = (double)e[1], e2 = (double)e[2];
+    const double gw[3] = {qq * s100 + e0 * s200 + e1 * s110 + e2 * s101, qq * s010 + e0 * s110 + e1 * s020 + e2 * s011,
+                          qq * s001 + e0 * s101 + e1 * s011 + e2 * s002};
+    const double *es = g.escale;
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+        const double rdd = es[3 * b] * gd[0] + es[3 * b + 1] * gd[1] + es[3 * b + 2] * gd[2];
+        rec_dr[3 * i + b] = es[3 * b] * gw[0] + es[3 * b + 1] * gw[1] + es[3 * b + 2] * gw[2];
+        gp[3 * i + b] = KE * (rowf[3 * i + b] + rdd - cself * dd[3 * i + b]);
+        if (rec_dd) rec_dd[3 * i + b] = rdd;
+    }
+}
+
 // Force gather: dU_rec/dd and dU_rec/dr at fixed q, d (the autodiff of pme.py:390-411 written
 // out, with the second spline derivative), FP64 outputs; also gp = KE (rowf + dU_rec/dd - c_self d),
 // the total dE/dd of the atom for the covalent-frame pull-back.  rec_dd (optional) receives
@@ -816,13 +848,8 @@ __global__ __launch_bounds__(256) void k_gather_forces(int n, int nper, const do
 #pragma unroll
     for (int a = 0; a < 3; ++a) bspline_rounded<real, P, true>(f[a], t[a], dt[a], d2t[a]);
     const real4<real> d = dq[i];
-    real e[3];
-    scaled_dipole<real>(d, g, e);
-    const real q = d.w;
     const int K1 = g.K[0], K2 = g.K[1], K3 = g.K[2];
     phi += (size_t)(i / nper) * K1 * K2 * K3;
-    // phi-weighted sums S[wx][wy][wz] with w = 0 (theta), 1 (dtheta), 2 (d2theta), needed:
-    // gd_a = S(d along a), gw_a = q S(d along a) + sum_b e_b S(d along a, d along b / d2 if a == b)
     double s100 = 0, s010 = 0, s001 = 0, s200 = 0, s020 = 0, s002 = 0, s110 = 0, s101 = 0, s011 = 0;
 #pragma unroll
     for (int ix = 0; ix < P; ++ix) {
@@ -861,17 +888,91 @@ __global__ __launch_bounds__(256) void k_gather_forces(int n, int nper, const do
         s101 += (double)(a_z * dt[0][ix]);
         s011 += (double)(a_yz * t[0][ix]);
     }
-    const double gd[3] = {s100, s010, s001};
-    const double qq = (double)q, e0 = (double)e[0], e1 = (double)e[1], e2 = (double)e[2];
-    const double gw[3] = {qq * s100 + e0 * s200 + e1 * s110 + e2 * s101, qq * s010 + e0 * s110 + e1 * s020 + e2 * s011,
-                          qq * s001 + e0 * s101 + e1 * s011 + e2 * s002};
-    const double *es = g.escale;
+    force_out<real>(i, d, g, s100, s010, s001, s200, s020, s002, s110, s101, s011, dd, rowf, cself, rec_dr, gp, rec_dd);
+}
+
+// The force gather on tiles: the block and the two lanes per atom of k_gather_tiles, with the second
+// derivatives of the splines and k_gather_forces' sums and outputs.
+// Bound by latency and LDS reads.  Against one thread per atom on the grid in memory (k_gather_forces, which
+// untiled grids keep): forces of 9,001 waters 375 -> 345 us, strain of 2,744 waters 303 -> 270, compute of 1,331 waters
+// at order 8 1049 -> 1000.
+template <typename real, int P, bool VEC>
+__global__ __launch_bounds__(WAVE * gather_waves<real>()) void k_gather_forces_tiles(
+    PMETiles t, const int *__restrict__ corg, PMEGeom g, const int2 *__restrict__ range, const int *__restrict__ sidx,
+    const real4<real> *__restrict__ sten, const real *__restrict__ phi, const real4<real> *__restrict__ dq,
+    const double *__restrict__ dd, const double *__restrict__ rowf, double cself, double *__restrict__ rec_dr,
+    double *__restrict__ gp, double *__restrict__ rec_dd) {
+    constexpr int GW = gather_waves<real>();
+    const int bead = (blockIdx.x * GW) / t.ntiles;  // t.ntiles is a multiple of 8
+    constexpr int MAXB = P + 7, SZ = MAXB | 1;
+    __shared__ real blk_all[GW][MAXB * MAXB * SZ];
+    const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE;
+    const int tile = blockIdx.x * GW + wv;
+    real *blk = blk_all[wv];
+    const int BY = t.B[1];
+    const int2 rg = range[tile];
+    const int s1 = rg.y, lt = tile - bead * t.ntiles;
+    const int half = lane & 1;
+    int u8[3];
+    if (rg.x >= s1 || !octant_tile(corg[lt >> 3], lt & 7, t, u8)) return;
+    load_tile_block<real, P, VEC>(t, g, u8, phi + (size_t)bead * g.K[0] * g.K[1] * g.K[2], blk, lane);
+    constexpr int PH = (P + 1) / 2;  // x planes of the first lane of a pair
+    for (int s = rg.x + (lane >> 1); s < s1; s += WAVE / 2) {
+        const real4<real> st = sten[s];
+        const int i = sidx[s];
+        real tx[P], dx[P], d2x[P], ty[P], dy[P], d2y[P], tz[P], dz[P], d2z[P];
+        bspline_rounded<real, P, true>(st.x, tx, dx, d2x);
+        bspline_rounded<real, P, true>(st.y, ty, dy, d2y);
+        bspline_rounded<real, P, true>(st.z, tz, dz, d2z);
+        const int lc = unpack_loc(st.w);
+        const int lx = lc & 31, ly = (lc >> 5) & 31, lz = (lc >> 10) & 31;
+        double s100 = 0, s010 = 0, s001 = 0, s200 = 0, s020 = 0, s002 = 0, s110 = 0, s101 = 0, s011 = 0;
 #pragma unroll
-    for (int b = 0; b < 3; ++b) {
-        const double rdd = es[3 * b] * gd[0] + es[3 * b + 1] * gd[1] + es[3 * b + 2] * gd[2];
-        rec_dr[3 * i + b] = es[3 * b] * gw[0] + es[3 * b + 1] * gw[1] + es[3 * b + 2] * gw[2];
-        gp[3 * i + b] = KE * (rowf[3 * i + b] + rdd - cself * dd[3 * i + b]);
-        if (rec_dd) rec_dd[3 * i + b] = rdd;
+        for (int ixh = 0; ixh < PH; ++ixh) {
+            const int ix = half ? PH + ixh : ixh;
+            if (ix >= P) break;
+            const int ih = PH + ixh < P ? PH + ixh : P - 1;
+            const real t_x = half ? tx[ih] : tx[ixh], d_x = half ? dx[ih] : dx[ixh], d2_x = half ? d2x[ih] : d2x[ixh];
+            real a_0 = 0, a_y = 0, a_z = 0, a_yy = 0, a_zz = 0, a_yz = 0;
+#pragma unroll
+            for (int iy = 0; iy < P; ++iy) {
+                const real *line = blk + ((lx + ix) * BY + (ly + iy)) * SZ + lz;
+                real l0 = 0, l1 = 0, l2 = 0;
+#pragma unroll
+                for (int iz = 0; iz < P; ++iz) {
+                    const real v = line[iz];
+                    l0 += v * tz[iz];
+                    l1 += v * dz[iz];
+                    l2 += v * d2z[iz];
+                }
+                a_0 += l0 * ty[iy];
+                a_y += l0 * dy[iy];
+                a_z += l1 * ty[iy];
+                a_yy += l0 * d2y[iy];
+                a_zz += l2 * ty[iy];
+                a_yz += l1 * dy[iy];
+            }
+            s100 += (double)(a_0 * d_x);
+            s010 += (double)(a_y * t_x);
+            s001 += (double)(a_z * t_x);
+            s200 += (double)(a_0 * d2_x);
+            s020 += (double)(a_yy * t_x);
+            s002 += (double)(a_zz * t_x);
+            s110 += (double)(a_y * d_x);
+            s101 += (double)(a_z * d_x);
+            s011 += (double)(a_yz * t_x);
+        }
+        s100 += __shfl_xor(s100, 1, WAVE);
+        s010 += __shfl_xor(s010, 1, WAVE);
+        s001 += __shfl_xor(s001, 1, WAVE);
+        s200 += __shfl_xor(s200, 1, WAVE);
+        s020 += __shfl_xor(s020, 1, WAVE);
+        s002 += __shfl_xor(s002, 1, WAVE);
+        s110 += __shfl_xor(s110, 1, WAVE);
+        s101 += __shfl_xor(s101, 1, WAVE);
+        s011 += __shfl_xor(s011, 1, WAVE);
+        if (!half)
+            force_out<real>(i, dq[i], g, s100, s010, s001, s200, s020, s002, s110, s101, s011, dd, rowf, cself, rec_dr, gp, rec_dd);
     }
 }
 
