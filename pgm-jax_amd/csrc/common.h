@@ -284,38 +284,37 @@ template <typename real, int NMAX> PGM_DEV void pair_G(real a, real b, real r2, 
 // B_n of phi_a through the Boys functions F_n(s) = int_0^1 t^2n exp(-s t^2) dt, s = (a r)^2:
 // B_n = (2a/sqrt(pi)) (2a^2)^n F_n.  The highest one by its series of positive terms (Shavitt, Methods in
 // Computational Physics 2, 1963), F_m = exp(-s) sum_k (2s)^k / ((2m+1)(2m+3)...(2m+2k+1)), the others by
-// F_(n-1) = (2s F_n + exp(-s)) / (2n-1), which is stable downwards.  In FP64 24 terms leave 1.5e-10 of F_n
-// for s < 6 and 12 terms 1e-11 for s < 1.25; in FP32 18 and 8 terms leave less than its rounding.
-template <typename real, int NMAX, int TERMS> PGM_DEV void boys_B(real a, real s, real *B) {
-    const real x = real(2) * s, e = exp_neg(s);
-    real S = real(1);
+// F_(n-1) = (2s F_n + exp(-s)) / (2n-1), which is stable downwards.  With NMAX = 3, 24 terms leave 1.5e-10
+// of F_n for s < 6 and 12 terms 1e-11 for s < 1.25; with NMAX = 4 a quarter of that.
+template <int NMAX, int TERMS> PGM_DEV void boys_B(double a, double s, double *B) {
+    const double x = 2.0 * s, e = exp(-s);
+    double S = 1.0;
 #pragma unroll
-    for (int k = TERMS; k >= 1; --k) S = (S * x) * real(1.0 / double(2 * NMAX - 1 + 2 * k)) + real(1);
-    real F[NMAX];
-    F[NMAX - 1] = e * S * real(1.0 / double(2 * NMAX - 1));
+    for (int k = TERMS; k >= 1; --k) S = (S * x) * (1.0 / double(2 * NMAX - 1 + 2 * k)) + 1.0;
+    double F[NMAX];
+    F[NMAX - 1] = e * S * (1.0 / double(2 * NMAX - 1));
 #pragma unroll
-    for (int n = NMAX - 1; n >= 1; --n) F[n - 1] = (x * F[n] + e) * real(1.0 / double(2 * n - 1));
-    real c = real(TWO_OVER_SQRTPI) * a;
-    const real f = real(2) * a * a;
+    for (int n = NMAX - 1; n >= 1; --n) F[n - 1] = (x * F[n] + e) * (1.0 / double(2 * n - 1));
+    double c = TWO_OVER_SQRTPI * a;
+    const double f = 2.0 * a * a;
 #pragma unroll
     for (int n = 0; n < NMAX; ++n) {
         B[n] = c * F[n];
         c *= f;
     }
 }
-template <typename real, int NMAX> PGM_DEV void near_B(real a, real r2, real *B) {
-    constexpr bool wide = sizeof(real) == 8;
-    const real s = a * a * r2;
-    if (s < real(1.25)) {
-        boys_B<real, NMAX, wide ? 12 : 8>(a, s, B);
-    } else if (s < real(6)) {
-        boys_B<real, NMAX, wide ? 24 : 18>(a, s, B);
+template <int NMAX> PGM_DEV void near_B(double a, double r2, double *B) {
+    const double s = a * a * r2;
+    if (s < 1.25) {
+        boys_B<NMAX, 12>(a, s, B);
+    } else if (s < 6.0) {
+        boys_B<NMAX, 24>(a, s, B);
     } else {  // FP32: at these s neither erf nor the recursion loses accuracy (FP64 sums use pair_G)
         const float fr2 = (float)r2, ir = rsqrt_n(fr2);
         float C[NMAX];
         closed_B<float, NMAX>((float)a, fr2 * ir, ir, ir * ir, C);
 #pragma unroll
-        for (int n = 0; n < NMAX; ++n) B[n] = (real)C[n];
+        for (int n = 0; n < NMAX; ++n) B[n] = (double)C[n];
     }
 }
 
@@ -326,13 +325,50 @@ template <typename real, int NMAX> PGM_DEV void near_B(real a, real r2, real *B)
 // derivative of 2,744 waters; 3e-8 and 0.9e-6 with these).
 template <int NMAX> PGM_DEV void pair_G_near(double R2sum, double b, double r2, float *G) {
     double Ba[NMAX], Bb[NMAX];
-    near_B<double, NMAX>(1.0 / sqrt(2.0 * R2sum), r2, Ba);
-    near_B<double, NMAX>(b, r2, Bb);
+    near_B<NMAX>(1.0 / sqrt(2.0 * R2sum), r2, Ba);
+    near_B<NMAX>(b, r2, Bb);
 #pragma unroll
     for (int n = 0; n < NMAX; ++n) G[n] = (float)(Ba[n] - Bb[n]);
 }
 template <int NMAX> PGM_DEV void pair_G_near(double R2sum, double b, double r2, double *G) {
     pair_G<double, NMAX>(1.0 / sqrt(2.0 * R2sum), b, r2, G);
+}
+
+// B_1 and B_2 for the FP32 records, s = (a r)^2 < 6: F_2 = exp(-s) S / 5 with 22 terms of the series S =
+// sum_k x^k / (7 9 ... (2k+5)), x = 2s, of which the first five are added in FP64 (at s = 6 the others are a
+// fifth of S), and exp(-s) corrected for the rounding of s.  Against float64: 4e-8 rms, 1.4e-7 at most and 4e-9
+// on average at any s.  With 18 terms (8 below s = 1.25) in FP32 throughout it was 3e-7 rms with one sign just
+// below s = 6.  A function, not inlined: the record pass keeps within its 128 registers (124, none
+// spilled; inlined, 7 to 18 are).  Field of 32,768 waters 416 us, 424 with the FP32 terms, 463 inlined, 556 with
+// near_B's FP64 sums inlined; forces of 9,001 waters with split cutoffs 327 us, 346 with the FP32 terms.
+constexpr double boys2_coeff(int k, int from) {  // the coefficient of x^k over that of x^from
+    double c = 1.0;
+    for (int j = from + 1; j <= k; ++j) c /= 5 + 2 * j;
+    return c;
+}
+__device__ __attribute__((noinline)) double2 record_B(double a, double r2) {
+    const double s = a * a * r2;
+    if (s < 6.0) {
+        constexpr int TERMS = 22, WIDE = 5;
+        const float sf = (float)s, xf = 2.0f * sf;
+        float T = float(boys2_coeff(TERMS, WIDE));
+#pragma unroll
+        for (int k = TERMS - 1; k >= WIDE; --k) T = T * xf + float(boys2_coeff(k, WIDE));
+        const double x = 2.0 * s;
+        double S = (double)T * boys2_coeff(WIDE, 0);
+#pragma unroll
+        for (int k = WIDE - 1; k >= 0; --k) S = S * x + boys2_coeff(k, 0);
+        double e = (double)exp_neg(sf);
+        e += e * ((double)sf - s);
+        const double F2 = e * S * 0.2, F1 = (x * F2 + e) * (1.0 / 3.0);
+        const double f = 2.0 * a * a, c = TWO_OVER_SQRTPI * a * f;
+        return make_double2(c * F1, c * f * F2);
+    } else {  // here neither erf nor the recursion loses accuracy
+        const float fr2 = (float)r2, ir = rsqrt_n(fr2);
+        float C[3];
+        closed_B<float, 3>((float)a, fr2 * ir, ir, ir * ir, C);
+        return make_double2((double)C[1], (double)C[2]);
+    }
 }
 
 // ---------------------------------------------------------------------------- B-splines

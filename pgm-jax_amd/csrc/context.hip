@@ -809,9 +809,9 @@ static int prepare(pgm_ctx *c, const double *pos, bool defer_records = false) {
         const double beta2 = c->s.ewald_beta * c->s.ewald_beta;
         hipStream_t rs = side_records ? c->side : st;
         const bool rows_too = c->mixed && c->rc_v > c->rc_e;
-        const auto go = [&](auto k, int per_block, auto *mg, auto beta, bool rows) {
+        const auto go = [&](auto k, int per_block, auto *mg, bool rows) {
             k<<<nblk(nmol, per_block), 256, 0, rs>>>(nmol, c->mrows.as<int>(), c->mcount_full.as<int>(), c->mcap_full, c->mcap,
-                                                     c->xr.as<double4>(), c->box, rc2, rce2, beta, c->mj.as<int>(), mg,
+                                                     c->xr.as<double4>(), c->box, rc2, rce2, c->s.ewald_beta, c->mj.as<int>(), mg,
                                                      c->mcount.as<int>(), rows ? c->rows.as<int>() : nullptr, c->cap,
                                                      rows ? c->count.as<int>() : nullptr, rows ? c->count_near.as<int>() : nullptr,
                                                      beta2);
@@ -820,17 +820,16 @@ static int prepare(pgm_ctx *c, const double *pos, bool defer_records = false) {
         const bool split = nmol < MOL_SPLIT;
         float *mgf = c->mg.as<float>();
         double *mgd = c->mg.as<double>();
-        const float bf = (float)c->s.ewald_beta;
         if (rows_too)
-            go(k_mol_tensors<float, true, 1>, 4, mgf, bf, true);
+            go(k_mol_tensors<float, true, 1>, 4, mgf, true);
         else if (c->mixed && split)
-            go(k_mol_tensors<float, false, 4>, 1, mgf, bf, false);
+            go(k_mol_tensors<float, false, 4>, 1, mgf, false);
         else if (c->mixed)
-            go(k_mol_tensors<float, false, 1>, 4, mgf, bf, false);
+            go(k_mol_tensors<float, false, 1>, 4, mgf, false);
         else if (split)
-            go(k_mol_tensors<double, false, 4>, 1, mgd, c->s.ewald_beta, false);
+            go(k_mol_tensors<double, false, 4>, 1, mgd, false);
         else
-            go(k_mol_tensors<double, false, 1>, 4, mgd, c->s.ewald_beta, false);
+            go(k_mol_tensors<double, false, 1>, 4, mgd, false);
         c->atom_rows_fresh = rows_too;
         if (side_records) {
             LAUNCH_CHECK();

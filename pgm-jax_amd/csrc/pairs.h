@@ -738,7 +738,7 @@ __global__ __launch_bounds__(256) void k_mol_rows(int nmol, int nmol_bead, const
 // The closed form (both screenings with (a r)^2, (beta r)^2 >= 1) is evaluated for all nine pairs; the
 // others (the own molecule, hydrogen bonds: a few pairs per molecule) go to a queue in LDS and are
 // evaluated at the end, one per lane, so that a wave runs the series once and not once for every near
-// pair of its busiest lane.
+// pair of its busiest lane (see record_B).
 //
 // With ROWS the same pass also writes the compacted atom rows of the force pass (what
 // k_compact_rows makes from the full atom rows): for atom 3I + p every 3J + k with r^2 < rc^2,
@@ -752,7 +752,7 @@ constexpr int MOL_HELD = 64;                // near pairs a wave holds back for 
 constexpr int MOL_QUEUE = MOL_HELD + 9 * WAVE;  // and those of one round at most
 
 template <typename real>
-PGM_DEV void mol_near_pair(int I, int J, int e, int t, const double4 *__restrict__ xr, const Box &box, double rce2, real beta, int mcap,
+PGM_DEV void mol_near_pair(int I, int J, int e, int t, const double4 *__restrict__ xr, const Box &box, double rce2, double beta64, int mcap,
                            real *__restrict__ mg) {
     const int p = t / 3, k = t - 3 * p;
     const double4 a = xr[3 * I + p], b = xr[3 * J + k];
@@ -761,15 +761,14 @@ PGM_DEV void mol_near_pair(int I, int J, int e, int t, const double4 *__restrict
     const double r2d = dx * dx + dy * dy + dz * dz;
     real G[3] = {real(0), real(0), real(0)};
     if (r2d < rce2) {
-        const real x = (real)dx, y = (real)dy, z = (real)dz, r2 = x * x + y * y + z * z;
+        const double w2 = 2.0 * (a.w + b.w);
         if constexpr (sizeof(real) == 4) {
-            real A[3], B[3];
-            near_B<real, 3>((real)(1.0 / sqrt(2.0 * (a.w + b.w))), r2, A);
-            near_B<real, 3>(beta, r2, B);
-            G[1] = A[1] - B[1];
-            G[2] = A[2] - B[2];
+            const double y = (double)rsqrt_n((float)w2);  // 1/sqrt to FP32, then one Newton step
+            const double2 A = record_B(y * (1.5 - 0.5 * w2 * y * y), r2d), B = record_B(beta64, r2d);
+            G[1] = (real)(A.x - B.x);
+            G[2] = (real)(A.y - B.y);
         } else {
-            pair_G<real, 3>(rsqrt_(real(2) * (real)(a.w + b.w)), beta, r2, G);
+            pair_G<real, 3>(1.0 / sqrt(w2), beta64, r2d, G);
         }
     }
     real *g = mg + mchunk(e, I, mcap);
@@ -780,12 +779,13 @@ PGM_DEV void mol_near_pair(int I, int J, int e, int t, const double4 *__restrict
 template <typename real, bool ROWS, int WPM>
 __global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_mol_tensors(int nmol, const int *__restrict__ mrows, const int *__restrict__ mcount_full,
                                                      int mcap_full, int mcap, const double4 *__restrict__ xr, Box box,
-                                                     double rc2, double rce2, real beta, int *__restrict__ mj, real *__restrict__ mg,
+                                                     double rc2, double rce2, double beta64, int *__restrict__ mj, real *__restrict__ mg,
                                                      int *__restrict__ mcount, int *__restrict__ rows, int acap,
                                                      int *__restrict__ acount, int *__restrict__ acount_near, double beta2) {
     static_assert(!ROWS || WPM == 1, "atom rows are compacted by one wave per molecule");
     __shared__ int2 nearq[4][MOL_QUEUE];
     __shared__ int wsum[4];
+    const real beta = (real)beta64;
     const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int I = WPM == 1 ? blk * 4 + wv : blk;
@@ -939,7 +939,7 @@ __global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_mol_tensors(
             __builtin_amdgcn_wave_barrier();
             for (int u = lane; u < qlen; u += WAVE) {
                 const int2 q = queue[u];
-                mol_near_pair<real>(I, q.y, q.x >> 4, q.x & 15, xr, box, rce2, beta, mcap, mg);
+                mol_near_pair<real>(I, q.y, q.x >> 4, q.x & 15, xr, box, rce2, beta64, mcap, mg);
             }
             __builtin_amdgcn_wave_barrier();
             qlen = 0;
