@@ -107,8 +107,9 @@ int pgm_set_box(pgm_ctx *ctx, const double *H);
 int pgm_build_rows(pgm_ctx *ctx, const double *pos);
 
 /* Largest displacement [nm] of an atom of pos (all beads, device) since the rows were built (no minimum
- * image: molecules move continuously); infinity while there are no valid rows.  The caller's test for
- * pgm_build_rows, against half the skin (MDEngine's list update).  Synchronises. */
+ * image: molecules move continuously); infinity while there are no valid rows and for an atom whose
+ * position was not a number when they were built and is one now.  The caller's test for pgm_build_rows,
+ * against half the skin (MDEngine's list update).  Synchronises. */
 int pgm_rows_displacement(pgm_ctx *ctx, const double *pos, double *displacement);
 
 /* Number of stored row entries (pairs counted twice) within cutoff at the last compute. */

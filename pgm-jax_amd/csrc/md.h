@@ -313,16 +313,22 @@ __global__ __launch_bounds__(256) void k_md_second(int nmol, const double *__res
     if (threadIdx.x == 0) part[blockIdx.x] = ke[0];
 }
 
+// Squared displacement of atom i from the positions the rows were built at, for a maximum that drops what is
+// not a number: infinite for an atom that is somewhere now and was not then (no partner has it in its row).
+PGM_DEV double displacement2(const double *__restrict__ pos, const double *__restrict__ ref, int i) {
+    const double x = pos[3 * i], y = pos[3 * i + 1], z = pos[3 * i + 2];
+    const double dx = x - ref[3 * i], dy = y - ref[3 * i + 1], dz = z - ref[3 * i + 2];
+    const double d2 = dx * dx + dy * dy + dz * dz, inf = __builtin_huge_val();
+    return d2 >= 0.0 || !(fabs(x) + fabs(y) + fabs(z) < inf) ? d2 : inf;
+}
+
 // Largest displacement since the rows were built (block partials of the maximum).
 __global__ __launch_bounds__(256) void k_max_disp(int n, const double *__restrict__ pos, const double *__restrict__ ref,
                                                   double *__restrict__ part) {
     __shared__ double lds[32];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     double d = 0.0;
-    if (i < n) {
-        const double dx = pos[3 * i] - ref[3 * i], dy = pos[3 * i + 1] - ref[3 * i + 1], dz = pos[3 * i + 2] - ref[3 * i + 2];
-        d = sqrt(dx * dx + dy * dy + dz * dz);
-    }
+    if (i < n) d = sqrt(displacement2(pos, ref, i));
     d = block_max(d, lds);
     if (threadIdx.x == 0) part[blockIdx.x] = d;
 }
@@ -332,10 +338,7 @@ __global__ __launch_bounds__(1024) void k_max_disp_one(int n, const double *__re
                                                        double *__restrict__ out) {
     __shared__ double lds[32];
     double d2 = 0.0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        const double dx = pos[3 * i] - ref[3 * i], dy = pos[3 * i + 1] - ref[3 * i + 1], dz = pos[3 * i + 2] - ref[3 * i + 2];
-        d2 = fmax(d2, dx * dx + dy * dy + dz * dz);
-    }
+    for (int i = threadIdx.x; i < n; i += blockDim.x) d2 = fmax(d2, displacement2(pos, ref, i));
     d2 = block_max(d2, lds);
     if (threadIdx.x == 0) *out = sqrt(d2);
 }

@@ -38,3 +38,24 @@ def test_rows_displacement_is_the_largest_norm(nmol, edge):
         ref = torch.linalg.norm(moved - pos, dim=1).max().item()
         # three roundings of the squares and one of the root, on both sides: 4 eps
         assert abs(_ask(ff, moved) - ref) <= 4 * np.finfo(float).eps * ref
+
+
+@pytest.mark.parametrize("nmol,edge", [(343, 2.2), (5462, 5.47)])
+def test_rows_built_around_a_lost_atom_are_rebuilt(nmol, edge):
+    """Rows built while a position was not a number lack that atom: the next proper positions ask for new rows."""
+    import torch
+
+    import pgm_jax_amd as P
+
+    sys_, x, H = P.models.water_box(nmol, edge, seed=3)
+    print(f"displacement, lost atom, {nmol}", flush=True)
+    ff = P.PGMForceField(sys_, H, P.MDSettings(cutoff=0.6, skin=0.05, ewald_beta=5.0, pme_grid=(48,) * 3))
+    pos = torch.tensor(np.asarray(x), dtype=torch.float64, device="cuda").reshape(-1, 3).contiguous()
+    lost = pos.clone()
+    lost[3 * nmol - 1] = float("nan")
+    ff.build_rows(lost)
+    assert _ask(ff, lost) == 0.0
+    assert _ask(ff, pos) == np.inf
+    ff.build_rows(pos)
+    assert _ask(ff, lost) == 0.0
+    assert _ask(ff, pos) == 0.0
