@@ -450,38 +450,12 @@ static int set_box(pgm_ctx *c, const double *H) {
     return PGM_OK;
 }
 
-// Tile widths of the spread: per axis the smallest T in 8..16 (else 7..P-1) with at least two tiles
-// and a last tile at least P-1 wide; no such T: the atomic spread is used.
-// Tiles: per axis the largest T in tile_cap (8 unless tuned)..P-1 with at least three tiles and a last
-// tile at least P-1 wide, numbered in cubes of 2 x 2 x 2 tiles.  No such T: the atomic spread and the
-// per-atom gather are used.
+// The tiles (pme_tiles) and their buffers.  Without tiles the atomic spread and the per-atom gather are used.
 static int setup_tiles(pgm_ctx *c) {
     drop_graphs(c);
-    const int P = c->s.order;
     PMETiles t{};
-    bool ok = true;
-    for (int a = 0; a < 3; ++a) {
-        const int K = c->s.grid[a];
-        int best = 0;
-        for (int T = c->tile_cap; T >= P - 1 && !best; --T) {
-            const int nt = (K + T - 1) / T;
-            const int last = K - (nt - 1) * T;
-            if (nt >= 3 && last >= P - 1) best = T;
-        }
-        if (!best) {
-            ok = false;
-            break;
-        }
-        t.T[a] = best;
-        t.nt[a] = (K + best - 1) / best;
-        t.nc[a] = (t.nt[a] + 1) / 2;
-        t.B[a] = best + P - 1;
-    }
-    c->tiled = ok;
-    if (!ok) return PGM_OK;
-    t.ncubes = t.nc[0] * t.nc[1] * t.nc[2];
-    t.ntiles = 8 * t.ncubes;
-    t.bsize = t.B[0] * t.B[1] * PME_ZROW;
+    c->tiled = pme_tiles(c->s.grid, c->s.order, c->tile_cap, t);
+    if (!c->tiled) return PGM_OK;
     c->tiles = t;
     const int n = c->n;
     const size_t B = (size_t)c->nbead;
@@ -495,25 +469,9 @@ static int setup_tiles(pgm_ctx *c) {
     LAUNCH_CHECK();
     PGM_TRY(c->sten.ensure(c->rsize * 4 * (size_t)n));
     PGM_TRY(c->blocks.ensure(c->rsize * B * t.ntiles * t.bsize));
-    {  // per-axis offsets of the block merge (k_merge_table, k_pme_fwd_plane)
-        std::vector<int> tab, org;
-        for (int a = 0; a < 3; ++a) {
-            const int K = c->s.grid[a], T = t.T[a], nt = t.nt[a];
-            const int stride = a == 0 ? t.B[1] * PME_ZROW : (a == 1 ? PME_ZROW : 1);
-            const int cube = 8 * (a == 0 ? t.nc[1] * t.nc[2] : (a == 1 ? t.nc[2] : 1)), oct = 4 >> a;
-            auto A = [&](int u) { return ((u >> 1) * cube + (u & 1) * oct) * t.bsize; };
-            for (int g = 0; g < K; ++g) {
-                const int u = std::min(g / T, nt - 1), l = g - u * T;
-                tab.push_back(A(u) + l * stride);
-                if (l <= P - 2) {
-                    const int up = u > 0 ? u - 1 : nt - 1;
-                    const int width = up < nt - 1 ? T : K - (nt - 1) * T;
-                    tab.push_back(A(up) + (l + width) * stride);
-                } else {
-                    tab.push_back(-1);
-                }
-            }
-        }
+    {
+        const std::vector<unsigned> tab = pme_merge_table(c->s.grid, c->s.order, t);
+        std::vector<int> org;
         PGM_TRY(upload(c->merge_tab, tab.data(), tab.size(), c->stream));
         for (int u0 = 0; u0 < t.nc[0]; ++u0)
             for (int u1 = 0; u1 < t.nc[1]; ++u1)
@@ -988,7 +946,7 @@ static int spread_fft(pgm_ctx *c, const real4<real> *dq, bool withq, bool energy
         if (fork && (c->fork_stage == 1 || c->fork_stage == 4)) PGM_TRY((*fork)());
         const int *K = c->s.grid;
         k_merge_table<real><<<dim3(nblk(K[2], 128), K[1], K[0] * B), 128, 0, st>>>(
-            K[0], K[1], K[2], (size_t)t.ntiles * t.bsize, c->merge_tab.as<int>(), c->blocks.as<real>(), c->grid.as<real>(), conv,
+            K[0], K[1], K[2], (size_t)t.ntiles * t.bsize, c->merge_tab.as<unsigned>(), c->blocks.as<real>(), c->grid.as<real>(), conv,
             iter);
     } else {
     k_fill<real><<<nblk((long long)c->ngrid, 256), 256, 0, st>>>(c->ngrid, c->grid.as<real>(), real(0));
@@ -2398,7 +2356,7 @@ template <typename real> static int spread_api(pgm_ctx *c, const double *pos, in
         PGM_TRY(spread_tiles<real>(c, dq, withq != 0, conv, iter, st));
         const int *K = c->s.grid;
         k_merge_table<real><<<dim3(nblk(K[2], 128), K[1], K[0]), 128, 0, st>>>(
-            K[0], K[1], K[2], (size_t)t.ntiles * t.bsize, c->merge_tab.as<int>(), c->blocks.as<real>(), c->grid.as<real>(), conv,
+            K[0], K[1], K[2], (size_t)t.ntiles * t.bsize, c->merge_tab.as<unsigned>(), c->blocks.as<real>(), c->grid.as<real>(), conv,
             iter);
     } else {
         k_fill<real><<<nblk((long long)c->ngrid, 256), 256, 0, st>>>(c->ngrid, c->grid.as<real>(), real(0));
@@ -3565,7 +3523,7 @@ template <typename real> static int time_impl(pgm_ctx *c, const double *pos, int
         const int *K = c->s.grid;
         rc = timed(0, [&] {
             k_merge_table<real><<<dim3(nblk(K[2], 128), K[1], K[0] * c->nbead), 128, 0, st>>>(
-                K[0], K[1], K[2], (size_t)t.ntiles * t.bsize, c->merge_tab.as<int>(), c->blocks.as<real>(), c->grid.as<real>(),
+                K[0], K[1], K[2], (size_t)t.ntiles * t.bsize, c->merge_tab.as<unsigned>(), c->blocks.as<real>(), c->grid.as<real>(),
                 nullptr, -1);
         });
         if (rc < 0) return rc;

@@ -248,7 +248,8 @@ template <typename real> inline size_t pfft_plane_lds(const PFFTGeom &f) {
 
 // Forward plane: merge the spread blocks of plane x (bead b), r2c along z, transform along y, and
 // store the plane's K2 K3h complex values at spec[(b K1 + x) K2 K3h ...].  Launch: K1 B blocks,
-// pfft_plane_lds bytes of dynamic LDS.  The twiddle tables of lengths K3/2, K3, K2 lie one after
+// pfft_plane_lds bytes of dynamic LDS.  tab is the merge table read as int: on grids of up to 256 points per
+// axis its offsets stay below 2^31, and PME_NO_BLOCK reads as -1.  The twiddle tables of lengths K3/2, K3, K2 lie one after
 // the other from tw (offsets twM = 0, twK3 = K3/2, twK2 = K3/2 + K3).
 template <typename real, bool ODD>
 __global__ __launch_bounds__(pfft_plane_threads<real>()) void k_pme_fwd_plane(PFFTGeom f, size_t bead_blocks, const int *__restrict__ tab,

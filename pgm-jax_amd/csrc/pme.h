@@ -9,6 +9,7 @@
 #pragma once
 
 #include "common.h"
+#include "tiles.h"
 
 namespace pgm {
 
@@ -107,20 +108,6 @@ __global__ __launch_bounds__(256) void k_spread(int n, const double *__restrict_
 // wave per tile sums its atoms' stencils on the tile's block of (T+P-1)^3 points on the matrix cores
 // (k_spread_tiles), and k_merge_table (or the forward planes of the fused transform) sums, for
 // every grid point, the (up to 8) blocks that cover it in a fixed order.
-struct PMETiles {
-    int T[3];    // tile width per axis (the last tile may be narrower, >= P-1)
-    int nt[3];   // tiles per axis
-    int nc[3];   // cubes of 2 x 2 x 2 tiles per axis: (nt + 1) / 2
-    int ncubes;  // nc0 nc1 nc2
-    int ntiles;  // 8 ncubes: tiles by fine key (octants past the grid stay empty)
-    int B[3];    // extent of a tile's block per axis: T + P - 1
-    int bsize;   // values stored per block: B0 B1 PME_ZROW
-};
-
-// z rows of the stored spread blocks: padded to 16 values, so that a row is one aligned segment and one
-// column block of the matrix instructions.
-constexpr int PME_ZROW = 16;
-
 // Tiles are numbered by the fine key = cube index * 8 + octant, so that consecutive keys are near each
 // other in space.
 PGM_DEV int fine_key(const int (&u8)[3], const PMETiles &t) {
@@ -439,20 +426,20 @@ __global__ __launch_bounds__(64, sizeof(real) == 4 ? 4 : 2) void k_spread_tiles(
 // of the point in the axis part of its own tile's block -- A_a(u) bsize + l stride_a with A_0(u) =
 // ((u >> 1) nc1 nc2 8 + (u & 1) 4), A_1(u) = ((u >> 1) nc2 8 + (u & 1) 2), A_2(u) = ((u >> 1) 8 + (u & 1)),
 // strides B1 PME_ZROW, PME_ZROW, 1 -- and tab_a[2 g + 1] the same for the previous tile (local l + its
-// width) when l <= P-2, else -1.  Both the fine key and the in-block offset are sums over the axes, so a
+// width) when l <= P-2, else PME_NO_BLOCK.  Both the fine key and the in-block offset are sums over the axes, so a
 // grid point's up to 8 block values are blocks[bead base + X + Y + Z] over the axes' candidates, summed
 // in a fixed order.
 // Launch: x = z-line (blockDim.x points), y = K2 rows, z = K1 planes times beads.
 template <typename real>
-__global__ __launch_bounds__(128) void k_merge_table(int K1, int K2, int K3, size_t bead_blocks, const int *__restrict__ tab,
+__global__ __launch_bounds__(128) void k_merge_table(int K1, int K2, int K3, size_t bead_blocks, const unsigned *__restrict__ tab,
                                                      const real *__restrict__ blocks, real *__restrict__ grid,
                                                      const int *__restrict__ conv_it, int iter) {
     const int gz = blockIdx.x * blockDim.x + threadIdx.x;
     const int gy = blockIdx.y;
     const int gx = blockIdx.z % K1, bead = blockIdx.z / K1;
     if (gz >= K3 || cg_done(conv_it, bead, iter)) return;
-    const int *tx = tab, *ty = tab + 2 * K1, *tz = tab + 2 * (K1 + K2);
-    const int X[2] = {tx[2 * gx], tx[2 * gx + 1]}, Y[2] = {ty[2 * gy], ty[2 * gy + 1]}, Z[2] = {tz[2 * gz], tz[2 * gz + 1]};
+    const unsigned *tx = tab, *ty = tab + 2 * K1, *tz = tab + 2 * (K1 + K2);
+    const unsigned X[2] = {tx[2 * gx], tx[2 * gx + 1]}, Y[2] = {ty[2 * gy], ty[2 * gy + 1]}, Z[2] = {tz[2 * gz], tz[2 * gz + 1]};
     const real *b = blocks + bead_blocks * bead;
     real acc = real(0);
 #pragma unroll
@@ -461,7 +448,7 @@ __global__ __launch_bounds__(128) void k_merge_table(int K1, int K2, int K3, siz
         for (int i1 = 0; i1 < 2; ++i1)
 #pragma unroll
             for (int i2 = 0; i2 < 2; ++i2)
-                if (X[i0] >= 0 && Y[i1] >= 0 && Z[i2] >= 0) acc += b[(size_t)X[i0] + Y[i1] + Z[i2]];
+                if (X[i0] != PME_NO_BLOCK && Y[i1] != PME_NO_BLOCK && Z[i2] != PME_NO_BLOCK) acc += b[(size_t)X[i0] + Y[i1] + Z[i2]];
     grid[(((size_t)bead * K1 + gx) * K2 + gy) * K3 + gz] = acc;
 }
 
