@@ -483,6 +483,15 @@ static int setup_tiles(pgm_ctx *c) {
     return PGM_OK;
 }
 
+// Atoms that a tile holds at most: the mean, or as many as its volume holds at 128 atoms per nm^3 (liquid
+// water has 100), whichever is more, and not more than a bead has.
+static double tile_atoms(const pgm_ctx *c) {
+    double part = 1.0;
+    for (int a = 0; a < 3; ++a) part *= (double)c->tiles.T[a] / c->s.grid[a];
+    const double volume = c->box.h[0] * c->box.h[4] * c->box.h[8];
+    return std::min((double)c->nper, part * std::max((double)c->nper, 128.0 * volume));
+}
+
 // Sort the atoms by fine key and store their stencils in that order (once per geometry).
 template <typename real> static int pme_bin(pgm_ctx *c, const double *pos) {
     if (!c->tiled) return PGM_OK;
@@ -494,7 +503,7 @@ template <typename real> static int pme_bin(pgm_ctx *c, const double *pos) {
     // key and arrival number in pkey / pidx; slots (arrival order) in pskey; the sorted atoms in psidx
     k_pme_bin<<<nblk(n, 256), 256, 0, st>>>(n, c->nper, pos, c->pg, t, c->pkey.as<int>(), c->pidx.as<int>(), c->tcount.as<int>());
     LAUNCH_CHECK();
-    if (nk <= PME_SCAN_MAX) {
+    if (nk <= PME_SCAN_MAX && tile_atoms(c) <= PME_ORDER_MAX) {
         k_pme_scan<<<1, PME_SCAN_THREADS, 0, st>>>(nk, c->tcount.as<int>(), c->trange.as<int2>());
         k_pme_place<<<nblk(n, 256), 256, 0, st>>>(n, c->pkey.as<int>(), c->pidx.as<int>(), c->trange.as<int2>(), c->pskey.as<int>());
         k_pme_order<real><<<nblk(nk, 4), 256, 0, st>>>(nk, c->trange.as<int2>(), c->pskey.as<int>(), pos, c->pg, t, c->psidx.as<int>(),

@@ -149,6 +149,11 @@ __global__ void k_pme_bin(int n, int nper, const double *__restrict__ pos, PMEGe
 // One workgroup; PME_SCAN_MAX tiles at most (more are sorted by the library).  Four waves: a workgroup of
 // sixteen waited 160 us for a CU with room beside the record pass.
 constexpr int PME_SCAN_MAX = 1 << 17, PME_SCAN_THREADS = 256;
+// k_pme_order compares the m atoms of a tile with one another, m^2 / 64 steps of a wave: tiles that may hold
+// more than PME_ORDER_MAX (8^3 points 0.16 nm apart in water) leave the sort to the library too.  Spread of the
+// PME object on 48^3, 216 tiles, counts / library sort [us]: 100 atoms a tile 78 / 120, 200: 151 / 181, 400:
+// 330 / 220, 800: 931 / 369, 6,400: 36,000 / 2,310.
+constexpr int PME_ORDER_MAX = 256;
 __global__ __launch_bounds__(PME_SCAN_THREADS) void k_pme_scan(int nk, int *__restrict__ count, int2 *__restrict__ range) {
     constexpr int NW = PME_SCAN_THREADS / WAVE;
     __shared__ int wsum[NW];
