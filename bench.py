@@ -148,7 +148,7 @@ def pmc_traffic(kernel: str):
 
 
 def roofline_of(live: dict, kern: dict, entries: int, blocks: int, layout: str, n: int, K3: int, fused: bool = False,
-                lanes: int = 16, floor_us: float | None = None) -> dict:
+                floor_us: float | None = None) -> dict:
     """HBM roofline of the dominant kernel (the CG matvec's row field) with the PME spread / gather beside it.
 
     Launch durations are the averages of the HIP event pairs attached to every launch of the row
@@ -194,7 +194,7 @@ def roofline_of(live: dict, kern: dict, entries: int, blocks: int, layout: str, 
         "peak": HBM_PEAK_GBS,
         "unit": "GB/s",
         "frac": round(gbs(row_bytes, row_ms) / HBM_PEAK_GBS, 5),
-        "traffic": pmc_traffic(kname if layout != "molecule" or lanes == 16 else f"{kname}_{lanes}_lanes"),
+        "traffic": pmc_traffic(kname),
         "algorithmic_bytes": row_bytes,
         "ms_per_launch": round(row_ms, 5),
         "launches": live["row_field"]["launches"],
@@ -449,7 +449,7 @@ def main() -> int:  # noqa: C901
     log("live kernel timing over the instrumented steps:", json.dumps(live))
     kern = mdm.time_kernels(reps=50)
     entries = ffm.row_entries()
-    layout, lanes = ffm.row_layout()
+    layout = ffm.row_layout()[0]
     blocks = ffm.row_blocks()
     log("kernels (ms):", json.dumps({k: round(v, 5) for k, v in kern.items()}), "row entries", entries)
     prev = None
@@ -483,7 +483,7 @@ def main() -> int:  # noqa: C901
     log(f"launch floor: {floor_us:.2f} us per empty-kernel launch")
     n = 3 * a.waters
     K3 = a.grid**3
-    roofline = roofline_of(live, kern, entries, blocks, layout, n, K3, ffm.pme_transform()[0] == "fused", lanes, floor_us)
+    roofline = roofline_of(live, kern, entries, blocks, layout, n, K3, ffm.pme_transform()[0] == "fused", floor_us)
     roofline["events_block"] = repm["instrumented"]  # the MD steps the launch durations come from
     value = ns_per_day(ms_m, a.dt_fs)
     out = {

@@ -197,9 +197,10 @@ int pgm_set_graphs(pgm_ctx *ctx, int on);
 
 /* Layout of the CG row field (the data of PGMForceField._row_field, forcefield.py:1395-1402): 0 atom
  * rows (partner index, G1, G2 per pair in sliced ELL), 1 molecule blocks (contexts of consecutive
- * 3-atom molecules: per molecule pair the 9 atom pairs' G1, G2, `lanes` = 4, 8 or 16: at least so many
- * lanes per molecule, of which the launch takes 16 or 32 by the size of the system; the default where
- * it applies).  Same sums in another order; rows are rebuilt at the next evaluation.  pgm_row_layout reports the layout and its lanes. */
+ * 3-atom molecules: per molecule pair the 9 atom pairs' G1, G2; the default where it applies).  Same sums
+ * in another order; rows are rebuilt at the next evaluation.  `lanes` (4, 8 or 16; layout 1) is accepted and
+ * reported, and has no effect: the launch takes 16 or 32 lanes per molecule by the size of the system.
+ * pgm_row_layout reports the layout and the lanes last asked for. */
 int pgm_set_row_layout(pgm_ctx *ctx, int layout, int lanes);
 int pgm_row_layout(const pgm_ctx *ctx, int *layout, int *lanes);
 
@@ -222,16 +223,15 @@ int pgm_pme_transform(const pgm_ctx *ctx, int *fused, int *available);
 int pgm_set_row_fork(pgm_ctx *ctx, int stage);
 
 /* Autotuner (no counterpart in the reference): times, on this context's system at positions pos
- * (device), every applicable row-field layout (molecule blocks with 4, 8, 16 lanes; atom rows),
- * every valid PME tile width (8 down to order - 1 points per axis),
- * both reciprocal transforms and the point where a CG field evaluation starts the row field on its
- * side stream (before the spread, after it, after the forward planes of the fused transform) or
- * runs it on the context's stream (jointly with the row layouts within 10 % of the fastest row
- * field, by the time of a whole field evaluation),
- * `reps` launches each, and keeps the fastest.  report (host, 12 doubles): layout, lanes, spread
- * tile width per axis (3), row-field ms, spread + transform + gather ms, layouts tried, fused
- * transform chosen (1) or not (0), the other transform's ms (0 if not timed), fork point (0..4,
- * pgm_set_row_fork), whole field-evaluation ms.  Synchronises. */
+ * (device), every valid PME tile width (8 down to order - 1 points per axis), both reciprocal
+ * transforms, both row-field layouts (molecule blocks where they apply, atom rows) and, jointly with
+ * the layout by the time of a whole field evaluation, the point where a CG field evaluation starts the
+ * row field on its side stream (before the spread, after it, after the forward planes of the fused
+ * transform) or runs it on the context's stream; `reps` launches each, and keeps the fastest.  Without
+ * tiled spreading the layout goes by the row field alone.  report (host, 12 doubles): layout, lanes (as
+ * pgm_row_layout), tile width per axis (3), row-field ms, spread + transform + gather ms, settings of
+ * pgm_set_row_layout covered, fused transform chosen (1) or not (0), the other transform's ms (0 if not
+ * timed), fork point (0..4, pgm_set_row_fork), whole field-evaluation ms.  Synchronises. */
 int pgm_autotune(pgm_ctx *ctx, const double *pos, int reps, double *report);
 
 /* PGMForceField._energy_forces / energy_fixed_mu (forcefield.py:2249-2292, :2362-2430): energy

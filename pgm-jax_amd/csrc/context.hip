@@ -148,7 +148,7 @@ struct pgm_ctx {
     bool rows_valid = false;
     DevBuf rows_full, count_full, rows, count, count_near, maxcount, jell, G1, G2;
     // CG row field layout: atom rows in sliced ELL (jell, G1, G2; RL lanes per atom) or, for 3-site
-    // molecules, molecule blocks (mj, mg; rlm lanes per molecule) from the candidate molecules mrows
+    // molecules, molecule blocks (mj, mg) from the candidate molecules mrows
     bool mol3 = false;            // every bead is consecutive 3-atom molecules
     bool alpha0 = false;          // some atom has polarizability 0 (its induced dipole stays 0)
     bool atom_rows_fresh = false; // rows / count / count_near compacted for the current geometry
@@ -162,7 +162,7 @@ struct pgm_ctx {
     bool pinv_stale = true;       // its blocks are remade at the next evaluation after a row build
     DevBuf pinv;                  // its inverse 9x9 blocks, 81 reals per molecule
     int layout = 0;               // 0 atom rows, 1 molecule blocks
-    int rlm = 4;
+    int rlm = 4;  // the lanes last asked for (pgm_set_row_layout), reported and otherwise unused
     int mcap_full = 0, mcap = 0;
     DevBuf mrows, mcount_full, mcount, mj, mg;
     DevBuf key, atom, skey, satom, cell_start, cell_end, sort_tmp;
@@ -3593,10 +3593,11 @@ template <typename real> static int time_impl(pgm_ctx *c, const double *pos, int
 }
 
 // ---------------------------------------------------------------------------- autotuner
-// Time the CG matvec's pieces for every applicable shape on this context's own system and keep the
-// fastest: the row-field layout (molecule blocks with 4, 8 or 16 lanes per molecule, atom rows) by
-// the row field alone, then the spread-tile width (the largest valid width up to 8, 7, 6, ... P-1
-// per axis; the gather uses the same tiles) by spread + merge + gather.
+// Time the CG matvec's pieces for every applicable shape on this context's own system and keep the fastest:
+// the spread-tile width (the largest valid width up to 8, 7, 6, ... P-1 per axis; the gather uses the same
+// tiles) and the transform by spread + merge + gather, then the row-field layout (molecule blocks, atom
+// rows) and the fork point by a whole field evaluation.  Where there is no tiled spread the layout is chosen by
+// the row field alone.
 template <typename real> static int autotune_impl(pgm_ctx *c, const double *pos, int reps, double *out) {
     using R4 = real4<real>;
     hipStream_t st = c->stream;
@@ -3621,34 +3622,22 @@ template <typename real> static int autotune_impl(pgm_ctx *c, const double *pos,
         LAUNCH_CHECK();
         return PGM_OK;
     };
-    // row-field layouts
-    struct Lay {
-        int layout, lanes;
-    };
-    std::vector<Lay> lays;
-    if (c->mol3)
-        for (int l : {4, 8, 16}) lays.push_back({1, l});
-    lays.push_back({0, RL});
-    double best_row = 1e300;
-    Lay best_lay = lays.front();
-    std::vector<double> row_ms;
-    auto use_layout = [&](const Lay &L) -> int {
-        c->layout = L.layout;
-        if (L.layout == 1) {
-            c->rlm = L.lanes;
-            PGM_TRY(alloc_mol(c, std::max(c->mcap_full, 64)));
-        }
+    // row-field layouts: molecule blocks (one launch whatever number of lanes was asked for) and atom rows
+    const int first = c->mol3 ? 1 : 0;
+    int best_lay = first;
+    double row_ms[2] = {1e300, 1e300};
+    auto use_layout = [&](int layout) -> int {
+        c->layout = layout;
+        if (layout == 1) PGM_TRY(alloc_mol(c, std::max(c->mcap_full, 64)));
         c->rows_valid = false;
         return PGM_OK;
     };
-    for (const Lay &L : lays) {
-        PGM_TRY(use_layout(L));
+    for (int l = first; l >= 0; --l) {
+        PGM_TRY(use_layout(l));
         PGM_TRY(prepare(c, pos));
         PGM_TRY(dipoles());
-        double ms = 0;
-        PGM_TRY(time_ms([&] { (void)row_field_launch<real, false>(c, c->vp.as<R4>(), nullptr, -1, st); }, ms));
-        row_ms.push_back(ms);
-        if (ms < best_row) best_row = ms, best_lay = L;
+        PGM_TRY(time_ms([&] { (void)row_field_launch<real, false>(c, c->vp.as<R4>(), nullptr, -1, st); }, row_ms[l]));
+        if (row_ms[l] < row_ms[best_lay]) best_lay = l;
     }
     PGM_TRY(use_layout(best_lay));
     // spread-tile widths
@@ -3693,17 +3682,14 @@ template <typename real> static int autotune_impl(pgm_ctx *c, const double *pos,
         other_pme = ms[c->pme_fused ? 0 : 1];
         drop_graphs(c);
     }
-    // fork point of the row field in a whole CG field evaluation (row field beside the PME chain),
-    // jointly with the row layout among those within 10 % of the fastest row field alone: the
-    // layouts load the GPU differently beside the PME chain
+    // fork point of the row field and its layout in a whole CG field evaluation: the layouts load the GPU
+    // differently beside the PME chain, and small systems run the molecule blocks in the spread's launch
     double best_fork = 1e300;
     int fork_best = 0;
     if (c->tiled && !c->ewald) {
         const bool fz = c->pme_fused && c->fused_ok;
-        Lay fork_lay = best_lay;
-        for (size_t li = 0; li < lays.size(); ++li) {
-            if (row_ms[li] > 1.1 * best_row) continue;
-            PGM_TRY(use_layout(lays[li]));
+        for (int l = first; l >= 0; --l) {
+            PGM_TRY(use_layout(l));
             PGM_TRY(prepare(c, pos));
             PGM_TRY(dipoles());
             for (int fs = 0; fs < 5; ++fs) {
@@ -3713,13 +3699,11 @@ template <typename real> static int autotune_impl(pgm_ctx *c, const double *pos,
                 PGM_TRY(time_ms([&] {
                     (void)field_eval<real>(c, c->vp.as<R4>(), false, MODE_AV, nullptr, c->vAp.as<R4>(), c->partA.as<double>(), -1);
                 }, ms));
-                if (ms < best_fork) best_fork = ms, fork_best = fs, fork_lay = lays[li];
+                if (ms < best_fork) best_fork = ms, fork_best = fs, best_lay = l;
             }
             drop_graphs(c);
         }
-        for (size_t li = 0; li < lays.size(); ++li)
-            if (lays[li].layout == fork_lay.layout && lays[li].lanes == fork_lay.lanes) best_row = row_ms[li];
-        PGM_TRY(use_layout(fork_lay));
+        PGM_TRY(use_layout(best_lay));
         c->fork_stage = fork_best;
     }
     c->rows_valid = false;
@@ -3730,9 +3714,9 @@ template <typename real> static int autotune_impl(pgm_ctx *c, const double *pos,
     out[0] = c->layout;
     out[1] = c->layout == 1 ? c->rlm : RL;
     for (int a = 0; a < 3; ++a) out[2 + a] = c->tiled ? c->tiles.T[a] : 0;
-    out[5] = best_row;
+    out[5] = row_ms[best_lay];
     out[6] = best_pme < 1e300 ? best_pme : 0.0;
-    out[7] = (double)lays.size();
+    out[7] = first ? 4.0 : 1.0;  // settings of pgm_set_row_layout covered (three numbers of lanes are one launch)
     out[8] = c->pme_fused && c->fused_ok ? 1.0 : 0.0;
     out[9] = other_pme;
     out[10] = c->fork_stage;

@@ -510,7 +510,8 @@ class PGMForceField:
         return int(_lib.lib().pgm_row_blocks(self._ctx))
 
     def set_row_layout(self, layout: str = "molecule", lanes: int = 4) -> None:
-        """Choose the CG row-field layout: "atom" rows or "molecule" blocks (3-site molecules; 4, 8 or 16 lanes)."""
+        """Choose the CG row-field layout: "atom" rows or "molecule" blocks (3-site molecules).  lanes (4, 8 or 16)
+        is reported by row_layout and has no effect: the launch takes 16 or 32 by the size of the system."""
         code = {"atom": 0, "molecule": 1}[layout]
         _lib.check(_lib.lib().pgm_set_row_layout(self._ctx, code, int(lanes)), "pgm_set_row_layout")
         self._rows_built = False
@@ -541,7 +542,7 @@ class PGMForceField:
         _lib.check(_lib.lib().pgm_set_row_fork(self._ctx, code), "pgm_set_row_fork")
 
     def row_layout(self) -> tuple[str, int]:
-        """Return the CG row-field layout and its lanes per row."""
+        """Return the CG row-field layout and the lanes last asked for."""
         lay, lanes = C.c_int(), C.c_int()
         _lib.check(_lib.lib().pgm_row_layout(self._ctx, C.byref(lay), C.byref(lanes)), "pgm_row_layout")
         return ("atom", "molecule")[lay.value], lanes.value

@@ -1,4 +1,4 @@
-"""CG row-field layouts agree (GPU): atom rows against molecule blocks (4, 8 and 16 lanes).
+"""CG row-field layouts agree (GPU): atom rows against molecule blocks (asked for with 4, 8 and 16 lanes: one launch).
 
 The molecule blocks hold the same pair kernels G1, G2 (pair_G of the same FP64 minimum-image
 displacements rounded to the compute precision) and sum the same pair terms in molecule-pair order,
@@ -89,3 +89,17 @@ def test_autotune_keeps_the_results(precision):
     tol = 1e-11 if precision == "double" else 1e-6
     assert abs(r1.energy["total"] - r0.energy["total"]) <= tol * abs(r0.energy["total"])
     assert abs(r1.iterations - r0.iterations) <= (0 if precision == "double" else 1)
+
+
+@pytest.mark.parametrize("lanes", [4, 8, 16])
+def test_autotune_leaves_the_lanes_asked_for(lanes):
+    """The number of lanes is the caller's and no launch depends on it: the autotuner does not pick one by chance."""
+    import pgm_jax_amd as P
+
+    top, pos, H = systems.water_box(512, 2.483, seed=6)
+    print(f"autotune lanes={lanes}", flush=True)
+    ff = P.PGMForceField(_system(top), H, P.MDSettings(precision="mixed", **CFG1))
+    ff.set_row_layout("molecule", lanes)
+    rep = ff.autotune(pos, reps=5)
+    assert (rep["row_layout"], rep["row_lanes"]) == ff.row_layout()
+    assert rep["row_layout"] == "atom" or rep["row_lanes"] == lanes
