@@ -183,9 +183,10 @@ struct pgm_ctx {
     bool fused_ok = false, pme_fused = false, pfft_odd = false;  // pfft_odd: an axis has a factor 3 or 5
     // where a CG field evaluation forks the row field onto the side stream: 0 before the spread,
     // 1 after the spread, 2 after the forward planes, 3 before the spread with the forward planes
-    // waiting for it (2 and 3: fused transform only), 4 no side stream; set from the size at creation
-    // (default_fork) and by pgm_autotune
+    // waiting for it (2 and 3: fused transform only), 4 no side stream; from the size and the transform
+    // (default_fork) until pgm_set_row_fork or pgm_autotune sets it
     int fork_stage = 4;
+    bool fork_set = false;
     PFFTGeom pfg{};
     DevBuf pfft_tw;
     // tiled spread (atoms sorted by grid tile)
@@ -267,14 +268,20 @@ static double *aux_slots(const pgm_ctx *c) { return c->energy.as<double>() + 4 *
 // The largest displacement since the row build, written by the MD step's reduction into pinned host memory.
 static double *h_disp(const pgm_ctx *c) { return reinterpret_cast<double *>(c->h_mirror + 4 * (size_t)c->nbead); }
 
-// Fork point of a new context: a fork and its join cost a field evaluation 10-20 us of cross-stream
-// latency, which pays only where the row field is long enough to hide the PME chain behind it.  Whole
-// field evaluations, FP32, fork after the spread / no side stream [us]: 64 waters 57.5 / 46.7, 1,331:
-// 92.7 / 84.4, 4,096: 92.9 / 91.5, 12,167: 139 / 135, 32,768: 176 / 207.  With the library transform the
-// row field starts first: its many small kernels leave room beside it (32 beads of 1,024 waters: 4.52 ms
-// per evaluation of all beads against 4.69 with the fork after the spread).
-constexpr int FORK_ATOMS = 49152;
-static int default_fork(const pgm_ctx *c) { return c->n < FORK_ATOMS ? 4 : (c->fused_ok && c->tiled ? 1 : 0); }
+// Fork point of a context that has none set: a fork and its join cost a field evaluation 10-20 us of cross-stream
+// latency, which pays only where the row field is long enough to hide the PME chain behind it; smaller
+// systems run the two in one launch (k_spread_rows) or one after the other.  With the library transform the row
+// field starts first: its many small kernels leave room beside it.  Whole solves of 9 iterations [us], fork
+// before the spread / after it / no side stream, FP32 fused: 4,096 waters 1255 / 1270 / 1196, 8,000: 1590 / 1589 /
+// 1604, 9,261: 1577 / 1503 / 1629, 15,625: 2173 / 2025 / 2203, 32,768: 2841 / 2644 / 2885; FP32 library: 8,000:
+// 1824 / 1854 / 1802, 12,167: 1926 / 1966 / 1916, 24,389: 2594 / 2631 / 2710, 32,768: 2884 / 2974 / 3038; FP64
+// fused: 4,096: 1465 / 1474 / 1461, 6,859: 1887 / 1907 / 2047, 9,261: 2234 / 2168 / 2420, 17,576: 3788 / 3528 /
+// 3900; FP64 library: 4,096: 1412 / 1463 / 1417, 8,000: 2210 / 2219 / 2422, 17,576: 3501 / 3542 / 3546.
+constexpr int FORK_ATOMS_F32 = 24576, FORK_ATOMS_F64 = 16384;
+static int default_fork(const pgm_ctx *c) {
+    if (c->n < (c->mixed ? FORK_ATOMS_F32 : FORK_ATOMS_F64)) return 4;
+    return c->pme_fused && c->fused_ok && c->tiled ? 1 : 0;
+}
 
 static void drop_graphs(pgm_ctx *c) {
     for (hipGraphExec_t &g : c->it_graphs)
@@ -762,7 +769,7 @@ static int prepare(pgm_ctx *c, const double *pos, bool defer_records = false) {
     auto bin = [&]() -> int { return c->mixed ? pme_bin<float>(c, pos) : pme_bin<double>(c, pos); };
     // the PME binning (key, sort, tile bounds, splines) depends on the positions only: with molecule
     // blocks it runs on the side stream beside the record pass (enqueued after it, so that the record
-    // pass starts while the host still enqueues the binning's dozen launches), joined before return
+    // pass starts while the host still enqueues the binning's four launches), joined before return
     const bool fork_bin = c->layout == 1 && c->tiled && !c->ewald;
     const bool side_records = fork_bin && defer_records;
     if (fork_bin) HIP_TRY(hipEventRecord(c->ev_fork, st));
@@ -1093,8 +1100,10 @@ static int row_field_launch(pgm_ctx *c, const real4<real> *dq, const int *conv, 
             launch_timed(tp, k, dim3(nblk((long long)(c->n / 3) * lanes, 256)), dim3(256), 0, st, row_args<real>(c, ext), dq, conv, iter);
         };
         // records beyond the last-level cache are streamed past it (the allocation holds about 1.7 times the
-        // records in use): 32,768 waters (FP32) 83.9 -> 80.8 us alone and 105 -> 100 us in a step; 12,167 waters,
-        // whose records stay cached from one CG iteration to the next, would go from 24.8 to 31.7 us
+        // records in use).  Row field alone and whole solves of 9 iterations, cached / streamed [us], FP32: 12,167
+        // waters 25 / 30 and 1990 / 2031, 19,683: 44 / 50 and 2207 / 2187, 24,389 (just below the line): 53 / 59 and 2432 / 2373,
+        // 32,768: 81 / 78 and 2732 / 2698; FP64: 8,192: 31 / 36 and 3038 / 2875, 12,167 (just below the line): 42 / 50 and
+        // 3564 / 3216, 19,683: 85 / 79 and 3901 / 3705
         const bool stream = (size_t)(c->n / 3) * c->mcap * MOL_REC * sizeof(real) > ROW_STREAM_BYTES;
         if (row_field_lanes(c) == 16 && stream)
             go(k_row_field_mol<real, WITHQ, 16, true>, 16);
@@ -3705,6 +3714,7 @@ template <typename real> static int autotune_impl(pgm_ctx *c, const double *pos,
         }
         PGM_TRY(use_layout(best_lay));
         c->fork_stage = fork_best;
+        c->fork_set = true;
     }
     c->rows_valid = false;
     PGM_TRY(prepare(c, pos));
@@ -3733,6 +3743,7 @@ extern "C" int pgm_set_pme_transform(pgm_ctx *c, int fused) {
     }
     drop_graphs(c);
     c->pme_fused = fused != 0;
+    if (!c->fork_set) c->fork_stage = default_fork(c);
     if (!c->pme_fused && (c->fork_stage == 2 || c->fork_stage == 3)) c->fork_stage = c->fork_stage == 2 ? 1 : 0;
     return PGM_OK;
 }
@@ -3745,6 +3756,7 @@ extern "C" int pgm_set_row_fork(pgm_ctx *c, int stage) {
     }
     drop_graphs(c);
     c->fork_stage = stage;
+    c->fork_set = true;
     return PGM_OK;
 }
 
