@@ -171,7 +171,7 @@ PGM_DEV void fft_stage(C *buf, int N, int L, int nlines, int es, int ls, const C
             if (item < items) {
                 const int line = contiguous ? item / nb : item % nl;
                 const int j = contiguous ? item - line * nb : item / nl;
-                const int k = R == 5 ? j % L : j & (L - 1);  // L is a power of two before a radix-5 stage
+                const int k = R == 5 ? j % L : j & (L - 1);  // L is a power of two, and before a radix-5 stage may hold the 3
                 base[it] = (l0 + line) * ls;
                 jj[it] = j;
 #pragma unroll
