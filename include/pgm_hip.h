@@ -219,8 +219,9 @@ int pgm_pme_transform(const pgm_ctx *ctx, int *fused, int *available);
  * forward planes of the fused transform, 3 before the spread with the forward planes waiting for
  * the row field; 4: no side stream (the row field after the spread on the context's stream, no
  * fork or join events).  Only the overlap changes, not the results; the autotuner picks the
- * fastest.  Until one of the two sets it: 4 below 24,576 atoms (FP64 16,384), from there 1 with the fused
- * transform and 0 with the library plans, following pgm_set_pme_transform. */
+ * fastest.  Until one of the two sets it, it follows the size, the layout and the transform: molecule blocks 4
+ * below 24,576 atoms (FP64 16,384), from there 1 with the fused transform and 0 with the library plans; atom
+ * rows 1 with the fused transform from 3,072 atoms and 0 otherwise. */
 int pgm_set_row_fork(pgm_ctx *ctx, int stage);
 
 /* Autotuner (no counterpart in the reference): times, on this context's system at positions pos

@@ -276,11 +276,16 @@ static double *h_disp(const pgm_ctx *c) { return reinterpret_cast<double *>(c->h
 // 1604, 9,261: 1577 / 1503 / 1629, 15,625: 2173 / 2025 / 2203, 32,768: 2841 / 2644 / 2885; FP32 library: 8,000:
 // 1824 / 1854 / 1802, 12,167: 1926 / 1966 / 1916, 24,389: 2594 / 2631 / 2710, 32,768: 2884 / 2974 / 3038; FP64
 // fused: 4,096: 1465 / 1474 / 1461, 6,859: 1887 / 1907 / 2047, 9,261: 2234 / 2168 / 2420, 17,576: 3788 / 3528 /
-// 3900; FP64 library: 4,096: 1412 / 1463 / 1417, 8,000: 2210 / 2219 / 2422, 17,576: 3501 / 3542 / 3546.
-constexpr int FORK_ATOMS_F32 = 24576, FORK_ATOMS_F64 = 16384;
+// 3900; FP64 library: 4,096: 1412 / 1463 / 1417, 8,000: 2210 / 2219 / 2422, 17,576: 3501 / 3542 / 3546.  Atom rows
+// share no launch and gain from the side stream at every size, fused FP32 512 waters: 1014 / 1006 / 1043, 4,096:
+// 1397 / 1382 / 1474, 17,576: 2709 / 2640 / 2871; FP64 216: 1048 / 1091 / 1164, 512: 1116 / 1168 / 1230, 1,331:
+// 1410 / 1391 / 1550, 9,261: 2649 / 2249 / 2473.
+constexpr int FORK_ATOMS_F32 = 24576, FORK_ATOMS_F64 = 16384, FORK_ATOM_ROWS = 3072;
 static int default_fork(const pgm_ctx *c) {
+    const bool fused = c->pme_fused && c->fused_ok && c->tiled;
+    if (c->layout == 0) return fused && c->n >= FORK_ATOM_ROWS ? 1 : 0;
     if (c->n < (c->mixed ? FORK_ATOMS_F32 : FORK_ATOMS_F64)) return 4;
-    return c->pme_fused && c->fused_ok && c->tiled ? 1 : 0;
+    return fused ? 1 : 0;
 }
 
 static void drop_graphs(pgm_ctx *c) {
@@ -2491,6 +2496,7 @@ extern "C" int pgm_set_row_layout(pgm_ctx *c, int layout, int lanes) {
         c->rlm = lanes;
         PGM_TRY(alloc_mol(c, std::max(c->mcap_full, 64)));
     }
+    if (!c->fork_set) c->fork_stage = default_fork(c);
     c->rows_valid = false;
     return PGM_OK;
 }
