@@ -515,7 +515,7 @@ template <typename real> static int pme_bin(pgm_ctx *c, const double *pos) {
     // key and arrival number in pkey / pidx; slots (arrival order) in pskey; the sorted atoms in psidx
     k_pme_bin<<<nblk(n, 256), 256, 0, st>>>(n, c->nper, pos, c->pg, t, c->pkey.as<int>(), c->pidx.as<int>(), c->tcount.as<int>());
     LAUNCH_CHECK();
-    if (nk <= PME_SCAN_MAX && tile_atoms(c) <= PME_ORDER_MAX) {
+    if ((nk <= PME_SCAN_SMALL || (nk <= PME_SCAN_MAX && n / 4 >= nk)) && tile_atoms(c) <= PME_ORDER_MAX) {
         k_pme_scan<<<1, PME_SCAN_THREADS, 0, st>>>(nk, c->tcount.as<int>(), c->trange.as<int2>());
         k_pme_place<<<nblk(n, 256), 256, 0, st>>>(n, c->pkey.as<int>(), c->pidx.as<int>(), c->trange.as<int2>(), c->pskey.as<int>());
         k_pme_order<real><<<nblk(nk, 4), 256, 0, st>>>(nk, c->trange.as<int2>(), c->pskey.as<int>(), pos, c->pg, t, c->psidx.as<int>(),

@@ -146,9 +146,13 @@ __global__ void k_pme_bin(int n, int nper, const double *__restrict__ pos, PMEGe
     arrival[i] = atomicAdd(count + k, 1);
 }
 
-// One workgroup; PME_SCAN_MAX tiles at most (more are sorted by the library).  Four waves: a workgroup of
-// sixteen waited 160 us for a CU with room beside the record pass.
-constexpr int PME_SCAN_MAX = 1 << 17, PME_SCAN_THREADS = 256;
+// One workgroup, 2.3 us per 1,024 tiles, where the library's sort of the atoms does not depend on the tiles: beyond
+// PME_SCAN_SMALL tiles the counts are taken with four atoms a tile and more, beyond PME_SCAN_MAX never.  Spread
+// of the PME object, counts / library sort [us]: 200^3 (17,576 tiles) 300 atoms 152 / 160, 30,000: 162 / 178; 256^3
+// (32,768) 300: 355 / 386, 3,000: 356 / 337, 100,000: 389 / 394, 300,000: 429 / 503; 384^3 (110,592) 30,000:
+// 1021 / 919, 300,000: 1180 / 1145, 1,000,000: 1330 / 1338.  Four waves: a workgroup of sixteen waited 160 us for
+// a CU with room beside the record pass.
+constexpr int PME_SCAN_SMALL = 20000, PME_SCAN_MAX = 1 << 17, PME_SCAN_THREADS = 256;
 // k_pme_order compares the m atoms of a tile with one another, m^2 / 64 steps of a wave: tiles that may hold
 // more than PME_ORDER_MAX (8^3 points 0.16 nm apart in water) leave the sort to the library too.  Spread of the
 // PME object on 48^3, 216 tiles, counts / library sort [us]: 100 atoms a tile 78 / 120, 200: 151 / 181, 400:

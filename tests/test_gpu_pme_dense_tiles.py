@@ -1,8 +1,9 @@
-"""PME binning where a tile may hold more atoms than the per-tile ordering is meant for (the library's sort then).
+"""The lines between the two ways to bin the PME's atoms: counts per tile, or the library's sort.
 
-The line lies at 256 atoms in a tile: with 256 atoms in all, no tile can hold more; with 257 and wide tiles it could.  Both
-ways sort the atoms of a tile by index, so an atom more that has neither charge nor dipole changes nothing, bit for bit.
-Both are compared with the oracle's spread.  Past the line the cost per atom must not grow with the atoms per tile.
+A tile that may hold more than 256 atoms goes to the library: with 256 atoms in all, no tile can hold more; with 257 and
+wide tiles it could.  So do grids of more than 20,000 tiles (here 21,952) with fewer than four atoms a tile.  Both ways sort
+the atoms of a tile by index, so an atom more that has neither charge nor dipole changes nothing, bit for bit, though
+it takes the call across the line.  Past the first line the cost per atom must not grow with the atoms per tile.
 """
 
 import time
@@ -38,6 +39,24 @@ def test_both_sorts_give_the_same_grid(dtype, tol):
     ref = ref.spread(ref.setup(pos, H), q, d)
     got = Q[1].cpu().numpy()
     assert np.linalg.norm(got - ref) <= tol * np.linalg.norm(ref)
+
+
+def test_both_sorts_of_a_sparse_grid():
+    import torch
+
+    import pgm_jax_amd as P
+
+    rng = np.random.default_rng(6)
+    n, L = 4 * 21952, 21.6  # 28^3 tiles, in cubes of eight
+    pos, d = rng.uniform(0.0, L, (n, 3)), rng.normal(size=(n, 3)) * 0.1
+    d[-1] = 0.0
+    print("sparse grid", flush=True)
+    Q = []
+    for m in (n - 1, n):
+        pme = P.PME((224,) * 3, ORDER, 2.0)
+        Q.append(pme.spread(pme.setup(pos[:m], np.eye(3) * L), np.zeros(m), d[:m]))
+    assert torch.equal(Q[0], Q[1])
+    assert torch.count_nonzero(Q[0]).item() > n
 
 
 def test_cost_per_atom_does_not_grow_with_the_atoms_per_tile():
