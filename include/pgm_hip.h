@@ -219,9 +219,9 @@ int pgm_pme_transform(const pgm_ctx *ctx, int *fused, int *available);
  * forward planes of the fused transform, 3 before the spread with the forward planes waiting for
  * the row field; 4: no side stream (the row field after the spread on the context's stream, no
  * fork or join events).  Only the overlap changes, not the results; the autotuner picks the
- * fastest.  Until one of the two sets it, it follows the size, the layout and the transform: molecule blocks 4
- * below 24,576 atoms (FP64 16,384), from there 1 with the fused transform and 0 with the library plans; atom
- * rows 1 with the fused transform from 3,072 atoms and 0 otherwise. */
+ * fastest.  Until one of the two sets it, it follows the size, the layout and the transform: 4 below 24,576
+ * atoms (FP64 16,384), from there 1 with the fused transform and 0 with the library plans; atom rows of 150
+ * partners and more 1 with the fused transform from 3,072 atoms and 0 otherwise. */
 int pgm_set_row_fork(pgm_ctx *ctx, int stage);
 
 /* Autotuner (no counterpart in the reference): times, on this context's system at positions pos
@@ -375,7 +375,9 @@ int pgm_guess_status(pgm_ctx *ctx, double *out);
  * stream), its reciprocal spread (tiled spread + merge, or the Ewald structure factors) and its
  * gather; pgm_set_timing also clears the sums.  pgm_kernel_timing waits for the recorded events
  * and returns the average duration [ms] and the number of launches of [0] row field,
- * [1] spread, [2] gather. */
+ * [1] spread, [2] gather.  While the timing is on, contexts that run the row field in the spread's launch
+ * (molecule blocks below 8,192 molecules with no side stream) run the two as two launches, and captured
+ * iterations are not replayed: time whole calls with it off. */
 int pgm_set_timing(pgm_ctx *ctx, int on);
 int pgm_kernel_timing(pgm_ctx *ctx, double *avg_ms, long long *launches);
 

@@ -276,14 +276,18 @@ static double *h_disp(const pgm_ctx *c) { return reinterpret_cast<double *>(c->h
 // 1604, 9,261: 1577 / 1503 / 1629, 15,625: 2173 / 2025 / 2203, 32,768: 2841 / 2644 / 2885; FP32 library: 8,000:
 // 1824 / 1854 / 1802, 12,167: 1926 / 1966 / 1916, 24,389: 2594 / 2631 / 2710, 32,768: 2884 / 2974 / 3038; FP64
 // fused: 4,096: 1465 / 1474 / 1461, 6,859: 1887 / 1907 / 2047, 9,261: 2234 / 2168 / 2420, 17,576: 3788 / 3528 /
-// 3900; FP64 library: 4,096: 1412 / 1463 / 1417, 8,000: 2210 / 2219 / 2422, 17,576: 3501 / 3542 / 3546.  Atom rows
-// share no launch and gain from the side stream at every size, fused FP32 512 waters: 1014 / 1006 / 1043, 4,096:
-// 1397 / 1382 / 1474, 17,576: 2709 / 2640 / 2871; FP64 216: 1048 / 1091 / 1164, 512: 1116 / 1168 / 1230, 1,331:
-// 1410 / 1391 / 1550, 9,261: 2649 / 2249 / 2473.
-constexpr int FORK_ATOMS_F32 = 24576, FORK_ATOMS_F64 = 16384, FORK_ATOM_ROWS = 3072;
+// 3900; FP64 library: 4,096: 1412 / 1463 / 1417, 8,000: 2210 / 2219 / 2422, 17,576: 3501 / 3542 / 3546.
+// Atom rows share no launch, and the chain of an atom's row is as long as the row: with 214 partners (0.8 nm in
+// water) a side stream pays at every size, fused FP32 512 waters: 1014 / 1006 / 1043, 4,096: 1397 / 1382 / 1474,
+// 17,576: 2709 / 2640 / 2871; FP64 216: 1048 / 1091 / 1164, 1,331: 1410 / 1391 / 1550, 9,261: 2649 / 2249 / 2473;
+// with 77 (0.57 nm) it does not, FP32 216: 860 / 874 / 832 (library 1021 / 1038 / 891), 1,000: 1011 / 1002 / 1003
+// (library 1062 / 1066 / 939), FP64 216: 921 / 928 / 913, 1,000: 1084 / 1081 / 1104.
+constexpr int FORK_ATOMS_F32 = 24576, FORK_ATOMS_F64 = 16384, FORK_ATOMS_ROWS = 3072, FORK_LONG_ROW = 150;
 static int default_fork(const pgm_ctx *c) {
     const bool fused = c->pme_fused && c->fused_ok && c->tiled;
-    if (c->layout == 0) return fused && c->n >= FORK_ATOM_ROWS ? 1 : 0;
+    const double volume = c->box.h[0] * c->box.h[4] * c->box.h[8];
+    const double row = c->nper * std::min(1.0, 4.18879 * c->rc_pair * c->rc_pair * c->rc_pair / volume);
+    if (c->layout == 0 && row >= FORK_LONG_ROW) return fused && c->n >= FORK_ATOMS_ROWS ? 1 : 0;
     if (c->n < (c->mixed ? FORK_ATOMS_F32 : FORK_ATOMS_F64)) return 4;
     return fused ? 1 : 0;
 }
