@@ -747,7 +747,7 @@ __global__ __launch_bounds__(256) void k_mol_rows(int nmol, int nmol_bead, const
 // as k_compact_rows gives them.  (Used for FP32 with WPM = 1; the FP64 variant keeps its registers for
 // the tensors and leaves the atom rows to k_compact_rows.)
 //
-// VALU bound.
+// VALU bound: 186 us alone at 32,768 waters (FP32), 89 % of the instructions the SIMDs can issue in that time.
 constexpr int MOL_HELD = 64;                // near pairs a wave holds back for a later round
 constexpr int MOL_QUEUE = MOL_HELD + 9 * WAVE;  // and those of one round at most
 
@@ -956,8 +956,8 @@ __global__ __launch_bounds__(256, sizeof(real) == 4 ? 4 : 1) void k_mol_tensors(
 
 // Row field of the molecule blocks: out_i for the three atoms of I (the same sum as k_row_field over
 // the pairs within rc, in molecule-pair order).  RLM lanes per molecule take its records in turn.  Bound by the
-// record stream in large systems (32,768 waters: 338 MB in 81 us, 4.2 TB/s, where a copy reaches 4.8), by
-// the partners' gathers and latency in smaller ones.
+// record stream in large systems (32,768 waters: 338 MB, with the gathers 362 MB moved, in 78 us, 4.6 TB/s where a
+// copy reaches 4.8), by the partners' gathers and latency in smaller ones.
 template <typename real> struct RowArgs {
     int nmol, nmol_bead, mcap;
     const int *mj;
@@ -1070,7 +1070,8 @@ __global__ __launch_bounds__(256) void k_row_field_mol(RowArgs<real> A, const re
 // form read down and up (no erfc).  Pairs off it (a few per atom: its own molecule, hydrogen bonds)
 // are queued per atom in LDS and evaluated after the record loop over the molecule's lanes, in FP64 (see
 // pair_G_near).  The terms of a record are summed in `real`, then added to FP64 sums.  Grid (blocks per
-// bead, beads).  VALU bound.
+// bead, beads).  287 us alone at 32,768 waters (FP32): 62 % of the instructions the SIMDs can issue, the rest
+// waits (half of the waves' time) that three waves per SIMD do not cover.
 #define MOL_FORCE_TERMS(G0_, G1_, G2_, G3_)                                                            \
     {                                                                                                  \
         const real dix = di.x * x + di.y * y + di.z * z;                                               \

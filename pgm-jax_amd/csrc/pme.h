@@ -287,8 +287,8 @@ __global__ void k_pme_sorted(int n, const int *__restrict__ skey, int nk, const 
 // test per row, to skip those out of reach, takes the independent products out of one stream and costs
 // more than it saves (50 us).  No atomics and a fixed order: bitwise reproducible.
 //
-// Bound by the matrix instructions (8 us at 4,096 tiles of 24 atoms) and by writing the blocks (44 MB at
-// 128^3).  Measured per launch (FP32, alone) at 32,768 waters and 128^3 / 512 waters and 32^3: 24.1 / 9.8
+// Bound by the chain of one wave: at 4,096 tiles of 24 atoms four waves a SIMD are all there are, the matrix
+// cores are busy for 8.3 of 25.6 us, the VALU for a third, and 45 MB of blocks are written.  Measured per launch (FP32, alone) at 32,768 waters and 128^3 / 512 waters and 32^3: 24.1 / 9.8
 // us; the earlier form, one atom at a time with a read-add-write of its 216 points in LDS, 26.8 / 13.7 us;
 // summing the eight tiles of a cube in LDS first (22 MB written) 30.0 / 19.3 us.
 constexpr int SPREAD_CHUNK = 16;
@@ -642,7 +642,8 @@ PGM_DEV void load_tile_block(const PMETiles &t, const PMEGeom &g, const int *u8,
 // neighbouring lanes per atom (sorted order s, atom sidx[s]) sum its stencil from LDS, the first
 // (P+1)/2 x planes and the rest, and the first lane's combine_out writes the result.  Per-workgroup
 // partials of MODE_FIELD / MODE_AV go to part[blockIdx.x].  The potential of bead b is at phi + b K1 K2 K3.
-// Bound by latency and LDS reads.  Measured against one 512-thread workgroup per 16^3 points reading
+// Bound by latency and LDS reads: 16.8 us alone at 32,768 waters, the VALU issuing for 44 % of it and the waves
+// waiting for as much (51 MB read and written, a tile's block being 4 times its points).  Measured against one 512-thread workgroup per 16^3 points reading
 // stored splines (FP32, alone): 22 us at 32,768 waters and 128^3, 10.4 us at 64 waters and 32^3.
 template <typename real> constexpr int gather_waves() { return sizeof(real) == 4 ? 4 : 2; }
 template <typename real, int P, bool VEC>
@@ -889,7 +890,7 @@ __global__ __launch_bounds__(256) void k_gather_forces(int n, int nper, const do
 
 // The force gather on tiles: the block and the two lanes per atom of k_gather_tiles, with the second
 // derivatives of the splines and k_gather_forces' sums and outputs.
-// Bound by latency and LDS reads.  Against one thread per atom on the grid in memory (k_gather_forces, which
+// Bound like k_gather_tiles (19 us alone at 32,768 waters).  Against one thread per atom on the grid in memory (k_gather_forces, which
 // untiled grids keep): forces of 9,001 waters 375 -> 345 us, strain of 2,744 waters 303 -> 270, compute of 1,331 waters
 // at order 8 1049 -> 1000.
 template <typename real, int P, bool VEC>
